@@ -29,6 +29,7 @@ SOURCES = [
     "dtl_gemv.hip",
     "dtl_api.hip",
     "dtl_mfp.hip",
+    "dtl_f32.hip",
     "dtl_gguf.cpp",
     "dtl_range.cpp",
     "dtl_token.cpp",

@@ -927,6 +927,23 @@ int enqueue_forward(dtl_session* s, int T, size_t pos0, const int* pos_dev,
     for (const DevMat* mm : ms) mv[nm++] = mm;
     return fuse && gemv_fused_fits(mv, nm, pair, norm, T);
   };
+  // F32 matrices with the same input in one launch.
+  auto fits_f32 = [&](std::initializer_list<const DevMat*> ms, bool pair) {
+    return f32_mats_fit(ms.begin(), (int)ms.size(), pair);
+  };
+  auto f32_mats = [&](std::initializer_list<const DevMat*> ms, bool pair, const float* x,
+                      std::initializer_list<float*> outs, std::initializer_list<const float*> biases,
+                      std::initializer_list<int> epis, const char* cls) {
+    double bytes = (double)T * (*ms.begin())->cols * 4.0, macs = 0.0;
+    for (const DevMat* mm : ms) {
+      bytes += (double)mm->rows * mm->cols * 4.0 + (pair ? 2.0 : 4.0) * T * mm->rows;
+      macs += (double)mm->rows * mm->cols * T;
+    }
+    P.timed(st, cls, bytes, macs, [&] {
+      (void)launch_f32_mats(ms.begin(), (int)ms.size(), pair, x, T, outs.begin(), biases.begin(), epis.begin(),
+                            s->ln->err, st);
+    });
+  };
   for (size_t l = 0; l < c.block_count; l++) {
     const Layer& L = m->layers[l];
     const int e_q = L.bq ? EPI_BIAS : EPI_STORE, e_k = L.bk ? EPI_BIAS : EPI_STORE;
@@ -966,6 +983,10 @@ int enqueue_forward(dtl_session* s, int T, size_t pos0, const int* pos_dev,
                         T, s->ln->q, s->ln->k, L.bq, L.bk, e_q, e_k, s->ln->err, st);
       });
       gemm(L.wv, session_act(s, s->ln->h), s->ln->v, L.bv, e_v, nullptr);
+    } else if (fits_f32({&L.wq, &L.wk, &L.wv}, false)) {
+      a = rms(L.attn_norm, {});
+      f32_mats({&L.wq, &L.wk, &L.wv}, false, a.x, {s->ln->q, s->ln->k, s->ln->v}, {L.bq, L.bk, L.bv},
+               {e_q, e_k, e_v}, "gemm_f32_qkv");
     } else {
       a = rms(L.attn_norm, {&L.wq, &L.wk, &L.wv});
       if (L.wq.type == GGML_Q4_K && L.wk.type == GGML_Q4_K && L.wq.w32 && L.wk.w32 && T >= 16 &&
@@ -1063,6 +1084,9 @@ int enqueue_forward(dtl_session* s, int T, size_t pos0, const int* pos_dev,
         launch_gemv_q4k(L.gate, &L.up, true, Q4kIn{nullptr, s->ln->x, L.ffn_norm, c.eps}, T, s->ln->ffo,
                         nullptr, nullptr, nullptr, EPI_STORE, EPI_STORE, s->ln->err, st);
       });
+    } else if (fits_f32({&L.gate, &L.up}, true)) {
+      a = rms(L.ffn_norm, {});
+      f32_mats({&L.gate, &L.up}, true, a.x, {s->ln->ffo}, {}, {}, "gemm_f32_gate_up");
     } else {
       a = rms(L.ffn_norm, {&L.gate, &L.up});
       if (T >= 16 && L.gate.type == GGML_Q4_K && L.up.type == GGML_Q4_K &&

@@ -150,6 +150,41 @@ struct Q4kF32Args {
 void launch_q4k_mfp(const Q4kF32Args& a, int mode, hipStream_t s);
 void launch_mfp_probe(float* out, int workgroups, int iters, hipStream_t s);
 
+// F32 matrices of one launch over concatenated rows with the same input (wq,
+// wk and wv; or one matrix), or gate and up (pair) finishing as silu(gate) *
+// up into out[0].  Every dot is dot_f32_ref: eight interleaved chains.
+struct F32Mats {
+  const float* w[3];
+  float* out[3];
+  const float* bias[3];
+  int epi[3];
+  int rows[3];
+  int row_end[3];  // prefix sums of rows
+  int total_rows;
+  int cols;
+};
+// Entry m of a kernel argument's array, by selects: an index the compiler
+// does not know would put the whole argument in scratch memory.
+template <typename V>
+__host__ __device__ __forceinline__ V pick3(const V (&a)[3], int m) {
+  return m == 0 ? a[0] : (m == 1 ? a[1] : a[2]);
+}
+// Positions up to which k_gemv_f32 (dtl_f32.hip) serves a launch; more take
+// the products on the matrix cores (k_f32_mfp, dtl_mfp.hip), which cost the
+// same from 1 to 32 positions.  Microseconds per launch, GEMV at 4 / 8
+// positions against the matrix cores at 9 to 32: q/k/v of the SmolLM2-135M
+// shape 8.4 / 10.3 against 9.9, gate + up 8.5 / 11.0 against 9.8, wo and
+// down on average 14.8 / 17.2 against 14.5.
+constexpr int kF32GemvMaxT = 4;
+void launch_f32_mfp(const F32Mats& M, bool pair, const float* x, int T, int* err, hipStream_t s);
+// Whether launch_f32_mats takes these: F32, the same width, a multiple of
+// four (its 16-byte loads), and for the pair the same shape.  Other widths
+// keep k_gemm_rowlane.
+bool f32_mats_fit(const DevMat* const* mats, int nm, bool pair);
+// false (nothing launched) when they do not fit.
+bool launch_f32_mats(const DevMat* const* mats, int nm, bool pair, const float* x, int T, float* const* outs,
+                     const float* const* biases, const int* epis, int* err, hipStream_t s);
+
 // Positions up to which the decode GEMVs (one weight pass per position)
 // replace the chunked-encode GEMMs.
 constexpr int kGemvMaxT = 8;

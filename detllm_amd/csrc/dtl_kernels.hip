@@ -420,6 +420,10 @@ __global__ void __launch_bounds__(256) k_gemm_rowlane(DevMat W, DevAct A, int T,
 
 void launch_gemm(const DevMat& W, const DevAct& A, int T, float* out, const float* bias, int epi,
                  int* err, hipStream_t s) {
+  if (W.type == kGgmlF32) {
+    const DevMat* mats[1] = {&W};
+    if (launch_f32_mats(mats, 1, false, A.x, T, &out, &bias, &epi, err, s)) return;
+  }
   // Chunks of positions take the token-parallel kernels (weights decoded once
   // per wave and shared by up to 64 positions); short batches keep one lane
   // per (row, position).

@@ -208,6 +208,173 @@ void launch_mfp(const Q4kF32Args& a, hipStream_t s) {
 }
 }  // namespace
 
+// F32 weights (dot_f32_ref: chain c of eight adds the products of elements
+// c, c + 8, ... in order, then the combine tree), products on the matrix
+// cores as in k_q4k_mfp.  The eight chains are independent, so two waves
+// share each 16 x 16 tile of outputs, wave half h holding chains 4 h .. 4 h +
+// 3 (sixteen sums a lane): twice the waves for the same work, which short
+// matrices need to fill the chip.  Per 32 elements a wave issues four MFMAs,
+// MFMA m's block b taking element 8 b + 4 h + m (a lane's operands are the
+// float4 at 8 (lane / 16) + 4 h of its row and of its position), and 64 adds:
+// register 4 b + c of MFMA m is the next term of chain 4 h + m of row c, so
+// b ascending is the chain's order and sixteen adds in a row are independent.
+// A workgroup of eight waves covers 32 rows x 32 positions and stages
+// 64-element slices as k_q4k_mfp does; columns past the row are staged as
+// zeros (both operands: the products are +0.0, which changes no sum).
+//
+// Measured: 32000 x 1024 at 256 positions 307 us (27.4 T multiply-adds/s of
+// the 33.7 the pattern reaches), gate + up of that width (2 x 2816 rows) 61
+// us; short matrices are bound by the one workgroup per CU that they fill
+// (576-row q/k/v 10 us from 5 to 256 positions).  One lane per (row,
+// position), the kernel before: 607 us per launch on average over a
+// 100-position chunk of the SmolLM2-135M shape, 29 ms for six layers and the
+// output projection against 0.64.
+template <bool PAIR>
+__global__ void __launch_bounds__(512) k_f32_mfp(F32Mats M, const float* __restrict__ x, int T, int* err) {
+  constexpr int PB = 32, TR = 32, SL = 64, LD = SL + 4;
+  __shared__ __align__(16) float st[2][PB + TR][LD];
+  __shared__ __align__(16) float halves[4][64][4];
+  const int cols = M.cols;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int h = wave & 1, wp = (wave >> 1) & 1, wr = wave >> 2;
+  const int l16 = lane & 15, q = lane >> 4;
+  // The matrix and row of tile row tr (clamped to the last row).
+  auto locate = [&](int tr, int* mat, int* row) -> bool {
+    if (PAIR) {
+      const int rr = blockIdx.x * (TR / 2) + (tr >> 1);
+      *mat = tr & 1;
+      *row = rr < M.rows[0] ? rr : M.rows[0] - 1;
+      return rr < M.rows[0];
+    }
+    const int g = blockIdx.x * TR + tr;
+    const int gc = g < M.total_rows ? g : M.total_rows - 1;
+    *mat = (gc >= M.row_end[0] ? 1 : 0) + (gc >= M.row_end[1] ? 1 : 0);
+    *row = gc - (*mat == 0 ? 0 : (*mat == 1 ? M.row_end[0] : M.row_end[1]));
+    return g < M.total_rows;
+  };
+  // Staging: thread x moves column float4 x % 16 of position x / 16 and of
+  // tile row x / 16.
+  const int sr = tid >> 4, c4 = (tid & 15) * 4;
+  int sm, srow;
+  (void)locate(sr, &sm, &srow);
+  const int tt = blockIdx.y * PB + sr;
+  const float* xs = x + (size_t)(tt < T ? tt : T - 1) * cols;
+  const float* ws = pick3(M.w, sm) + (size_t)srow * cols;
+  // Two slices of loads in flight (even slices in the first pair of slots),
+  // for launches with one workgroup per CU.
+  // (named registers: as struct members or array elements they went to scratch)
+  float4 x0, w0, x1, w1;
+#define DTL_ISSUE_F(n, e0)                                 \
+  do {                                                     \
+    const int e_ = (e0) + c4 < cols ? (e0) + c4 : 0;       \
+    x##n = *reinterpret_cast<const float4*>(xs + e_);      \
+    w##n = *reinterpret_cast<const float4*>(ws + e_);      \
+  } while (0)
+#define DTL_COMMIT_F(n, b, e0)                                                                         \
+  do {                                                                                                 \
+    const bool in_ = (e0) + c4 < cols;                                                                 \
+    *reinterpret_cast<float4*>(&st[b][sr][c4]) =                                                       \
+        make_float4(in_ ? x##n.x : 0.0f, in_ ? x##n.y : 0.0f, in_ ? x##n.z : 0.0f, in_ ? x##n.w : 0.0f); \
+    *reinterpret_cast<float4*>(&st[b][PB + sr][c4]) =                                                  \
+        make_float4(in_ ? w##n.x : 0.0f, in_ ? w##n.y : 0.0f, in_ ? w##n.z : 0.0f, in_ ? w##n.w : 0.0f); \
+  } while (0)
+  DTL_ISSUE_F(0, 0);
+  DTL_ISSUE_F(1, SL);
+  DTL_COMMIT_F(0, 0, 0);
+  DTL_ISSUE_F(0, 2 * SL);
+  __syncthreads();
+  dtl_v16f zero;
+#pragma unroll
+  for (int i = 0; i < 16; i++) zero[i] = 0.0f;
+  float acc[4][4];
+#pragma unroll
+  for (int m = 0; m < 4; m++)
+#pragma unroll
+    for (int c = 0; c < 4; c++) acc[m][c] = 0.0f;
+  const int boff = (wp * 16 + l16) * LD + 8 * q + 4 * h;
+  const int aoff = (PB + wr * 16 + l16) * LD + 8 * q + 4 * h;
+  auto slice = [&](int buf) {
+    const float* sb = &st[buf][0][0];
+    dtl_v4f a4 = *(const dtl_v4f*)(sb + boff);
+    dtl_v4f w4 = *(const dtl_v4f*)(sb + aoff);
+#pragma unroll
+    for (int g = 0; g < SL; g += 32) {
+      dtl_v16f d[4];
+#pragma unroll
+      for (int m = 0; m < 4; m++) d[m] = __builtin_amdgcn_mfma_f32_16x16x1f32(w4[m], a4[m], zero, 0, 0, 0);
+      if (g + 32 < SL) {
+        a4 = *(const dtl_v4f*)(sb + boff + g + 32);
+        w4 = *(const dtl_v4f*)(sb + aoff + g + 32);
+      }
+      __builtin_amdgcn_sched_barrier(0);  // as in k_q4k_mfp
+#pragma unroll
+      for (int b = 0; b < 4; b++)
+#pragma unroll
+        for (int m = 0; m < 4; m++)
+#pragma unroll
+          for (int c = 0; c < 4; c++) acc[m][c] += d[m][4 * b + c];
+      // the next group's MFMAs after all of these adds
+      asm volatile("" : "+v"(acc[0][0]), "+v"(acc[0][1]), "+v"(acc[0][2]), "+v"(acc[0][3]), "+v"(acc[1][0]),
+                   "+v"(acc[1][1]), "+v"(acc[1][2]), "+v"(acc[1][3]), "+v"(a4));
+      asm volatile("" : "+v"(acc[2][0]), "+v"(acc[2][1]), "+v"(acc[2][2]), "+v"(acc[2][3]), "+v"(acc[3][0]),
+                   "+v"(acc[3][1]), "+v"(acc[3][2]), "+v"(acc[3][3]), "+v"(w4));
+    }
+  };
+  // Slices past the end are staged as zeros and add nothing (their adds run
+  // at most once, when the slice count is odd); refills are unconditional.
+  for (int e0 = 0; e0 < cols; e0 += 2 * SL) {
+    slice(0);
+    DTL_COMMIT_F(1, 1, e0 + SL);
+    DTL_ISSUE_F(1, e0 + 3 * SL);
+    __syncthreads();
+    slice(1);
+    DTL_COMMIT_F(0, 0, e0 + 2 * SL);
+    DTL_ISSUE_F(0, e0 + 4 * SL);
+    __syncthreads();
+  }
+#undef DTL_ISSUE_F
+#undef DTL_COMMIT_F
+  // ((a0 + a1) + (a2 + a3)) + ((a4 + a5) + (a6 + a7)): the second half's sum
+  // through LDS
+  float half[4];
+#pragma unroll
+  for (int c = 0; c < 4; c++) half[c] = (acc[0][c] + acc[1][c]) + (acc[2][c] + acc[3][c]);
+  if (h == 1) *reinterpret_cast<float4*>(halves[wave >> 1][lane]) = make_float4(half[0], half[1], half[2], half[3]);
+  __syncthreads();
+  if (h == 1) return;
+  const float4 o4 = *reinterpret_cast<const float4*>(halves[wave >> 1][lane]);
+  const float v4[4] = {half[0] + o4.x, half[1] + o4.y, half[2] + o4.z, half[3] + o4.w};
+  const int t = blockIdx.y * PB + wp * 16 + l16;
+  if (t >= T) return;
+  bool ok = true;
+  int mat, row;
+  if (PAIR) {
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      if (!locate(wr * 16 + 4 * q + 2 * i, &mat, &row)) continue;
+      const float gv = v4[2 * i], uv = v4[2 * i + 1];
+      const float v = silu_det(gv) * uv;
+      ok &= finite(gv) && finite(uv) && finite(v);
+      M.out[0][(size_t)t * M.rows[0] + row] = v;
+    }
+  } else {
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+      if (!locate(wr * 16 + 4 * q + c, &mat, &row)) continue;
+      ok &= store_epilogue(v4[c], pick3(M.out, mat), (size_t)t * pick3(M.rows, mat) + row, pick3(M.bias, mat), row, pick3(M.epi, mat));
+    }
+  }
+  if (!ok) flag(err, ERRBIT_NON_FINITE);
+}
+
+void launch_f32_mfp(const F32Mats& M, bool pair, const float* x, int T, int* err, hipStream_t s) {
+  const int rows = pair ? 2 * M.rows[0] : M.total_rows;
+  const dim3 grid((rows + 31) / 32, (T + 31) / 32);
+  if (pair) launch_kernel(k_f32_mfp<true>, grid, dim3(512), 0, s, M, x, T, err);
+  else launch_kernel(k_f32_mfp<false>, grid, dim3(512), 0, s, M, x, T, err);
+}
+
 // Measurement support: the rate of k_q4k_mfp's inner pattern on a chip
 // with nothing else to do, four 16x16x1 outer products (4096 products per
 // wave) and the 64 ordered adds per lane that take them into four chains,

@@ -75,6 +75,23 @@ def test_baseline_shapes_match_oracle(name, layers, n_tok, chunk):
     _compare_with_oracle(data, synth.tokens(w, n_tok), chunk)
 
 
+@pytest.mark.parametrize("name,heads,kv_heads", [
+    ("smollm2", 9, 3),   # 64-wide heads
+    ("qwen05", 14, 2),   # biases on the concatenated q/k/v launch
+    ("smollm2", 18, 6),  # 32-wide heads
+])
+@pytest.mark.parametrize("chunk", [1, 3, 8, 13, 34])
+def test_f32_model_matches_oracle(name, heads, kv_heads, chunk):
+    # F32 weights: q/k/v and gate/up/SwiGLU in one launch each, by GEMV up to
+    # eight positions and on the matrix cores beyond.
+    import dataclasses
+
+    from detllm_amd import synth
+
+    w = dataclasses.replace(synth.WORKLOADS[name], weight="f32", vocab=515, heads=heads, kv_heads=kv_heads)
+    _compare_with_oracle(synth.build_model(w, layers=2), synth.tokens(w, min(36, 3 * chunk)), chunk)
+
+
 @pytest.mark.parametrize("name,chunk", [("qwen05", 1), ("qwen05", 8), ("smollm2", 5)])
 @pytest.mark.parametrize("fused", [True, False])
 def test_decode_gemv_fusion_matches_oracle(monkeypatch, name, chunk, fused):

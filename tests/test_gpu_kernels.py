@@ -84,6 +84,32 @@ def test_exp_clamped_device_matches_oracle():
     assert L.lib.dtl_kernel_exp_clamped_f32(_p(y, C.c_float), _p(out, C.c_float), 2) == 42
 
 
+@pytest.mark.parametrize("rows,cols", [(1, 4), (8, 64), (33, 100), (40, 576), (65, 68), (192, 1028), (16389, 32)])
+@pytest.mark.parametrize("T", [1, 2, 3, 5, 8, 9, 15, 31, 33, 70])
+def test_f32_rows_bitexact(rows, cols, T):
+    # The F32 GEMV (up to eight positions) and the matrix-core products (more):
+    # partial row groups, position tiles and column slices, bit for bit.
+    L = _lib()
+    rng = np.random.default_rng(rows * 131 + cols + T)
+    w = rng.normal(0, 0.1, (rows, cols)).astype(np.float32)
+    x = rng.normal(0, 1.0, (T, cols)).astype(np.float32)
+    x[:, ::7] = 0.0
+    x[0, : min(cols, 5)] = -0.0
+    x[-1] *= np.float32(1e-38)  # subnormal products
+    out = np.empty((T, rows), np.float32)
+    raw = w.view(np.uint8).reshape(-1)
+    L.check(L.lib.dtl_kernel_gemv(0, _p(raw, C.c_uint8), rows, cols, _p(x, C.c_float), T, _p(out, C.c_float)), "gemv")
+    # the eight chains, each in column order, then the tree
+    pad = (-cols) % 8
+    p = np.pad((w[None] * x[:, None]).astype(np.float32), ((0, 0), (0, 0), (0, pad)))
+    acc = np.zeros((T, rows, 8), np.float32)
+    for k in range(0, cols + pad, 8):
+        acc = acc + p[:, :, k:k + 8]
+    want = (((acc[..., 0] + acc[..., 1]) + (acc[..., 2] + acc[..., 3])) +
+            ((acc[..., 4] + acc[..., 5]) + (acc[..., 6] + acc[..., 7])))
+    assert np.array_equal(out.view(np.uint32), want.view(np.uint32))
+
+
 def test_silu_bitexact():
     rng = np.random.default_rng(1)
     x = np.concatenate([rng.normal(0, 4, 100000), rng.uniform(-100, 100, 50000)]).astype(np.float32)
