@@ -1019,7 +1019,7 @@ int enqueue_forward(dtl_session* s, int T, size_t pos0, const int* pos_dev,
                      s->kc, s->vc};
       P.timed(st, "attention_dec", 2.0 * kv_rows * KV * hd * 4.0 + (double)T * (2 * H + 3 * KV) * hd * 4.0,
               2.0 * kv_rows * H * hd, [&] {
-                launch_attention_dec(s->ln->q, R, (int)l, T, (int)pos0, H, KV, (int)s->n_ctx,
+                launch_attention_dec(s->ln->q, R, (int)l, T, (int)pos0, H, KV, hd, (int)s->n_ctx,
                                      s->graph_maxlen, c.attention_scale, s->ln->scores, s->ln->attn,
                                      pos_dev, s->ln->err, st);
               });

@@ -307,8 +307,8 @@ struct RopeIn {
   float* kc;  // [layer][KV][n_ctx][hd] caches
   float* vc;
 };
-// Whether launch_attention_dec takes this shape (hd 64, at most four
-// positions, the score row within LDS).
+// Whether launch_attention_dec takes this shape (a head width it is built
+// for, at most four positions, the score row within LDS).
 bool attention_dec_applies(int hd, int T, int pos0, int n_ctx, bool pos_in_device);
 // Rows up to this many keys run the decode attention in one launch (scores
 // in LDS); longer rows run the split pair (scores through memory).
@@ -317,7 +317,7 @@ int attention_fused_max_len();
 // longest row (pos + 1) the launches may see; the caller keeps every
 // position it copies to pos_dev below it.
 void launch_attention_dec(const float* q, const RopeIn& R, int layer, int T, int pos0, int H,
-                          int KV, int n_ctx, int maxlen_dev, float scale, float* scores, float* out,
+                          int KV, int hd, int n_ctx, int maxlen_dev, float scale, float* scores, float* out,
                           const int* pos_dev, int* err, hipStream_t s);
 // Whether the decode attention (launch_attention_dec) takes the position
 // from device memory for this shape (graph replay of single-position forwards).

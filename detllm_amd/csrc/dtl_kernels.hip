@@ -9,6 +9,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "dtl_device.h"
 #include "dtl_blocks.h"
 #include "dtl_numerics.h"
@@ -1151,246 +1153,35 @@ size_t attention_hd64s_smem(int G, int scs) {
   return ((size_t)G * scs + 8 * 8 * kS64Stride) * sizeof(float);
 }
 
-// Decode shape (a few positions): one workgroup of 1024 threads per (head,
-// position), with the RoPE and cache store of the chunk folded in.  The
-// workgroup applies RoPE (lib.rs:2011-2051) to its query head and to the
-// chunk's new keys of its KV group in LDS, and the first head of each group
-// stores its position's key and value; cache rows before the chunk come from
-// memory, the chunk's own rows from LDS, so no workgroup reads a row another
-// one writes.  Then: scores (8-lane dot order), a block max, the clamped
-// exps in parallel, the 8-lane Z chains (lanes 0-7), p = e / Z in parallel.
-// P.V (lib.rs:2390-2420: out[d] = 0; out[d] += p_j * v_j[d] for j
-// ascending) splits into the products, which every thread forms for one
-// float4 of a 64-position V tile and stores dimension-major in LDS, and the
-// 64 serial sums, which wave 0 runs over the stored products (lane =
-// dimension, four products per LDS read).  V tiles stream through a ring of
-// kDecDepth registers per thread, so kDecDepth tiles of loads are in flight
-// while wave 0 sums.
-constexpr int kDecThreads = 1024, kDecTile = 64, kDecStride = 68, kDecDepth = 8, kDecMaxT = 4;
-
-__global__ void __launch_bounds__(kDecThreads) k_attention_dec(const float* q, RopeIn R, int layer,
-                                                               int pos0, int H, int KV, int n_ctx,
-                                                               float scale, float* out,
-                                                               const int* pos_dev, int* err) {
-  extern __shared__ __align__(16) float sc[];  // [len] scores -> exps -> probabilities
-  __shared__ __align__(16) float prod[2][64 * kDecStride];  // [dim][position in tile]
-  __shared__ __align__(16) float qs[64];
-  __shared__ __align__(16) float kn[kDecMaxT][64];  // the chunk's keys (after RoPE)
-  __shared__ __align__(16) float vn[kDecMaxT][64];  // the chunk's values
-  __shared__ float red[kDecThreads / 64];
-  __shared__ float zc[8];
-  constexpr int hd = 64;
-  const int h = blockIdx.x, t = blockIdx.y, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int G = H / KV, g = h / G;
-  const int pb = pos_dev ? *pos_dev : pos0;  // first position of the chunk
-  const int pos = pb + t, len = pos + 1;
-  const int half = R.rope_dim / 2;
-  const float* keys = R.kc + ((size_t)layer * KV + g) * n_ctx * hd;
-  const float* vals = R.vc + ((size_t)layer * KV + g) * n_ctx * hd;
-  float* o = out + (size_t)t * H * hd + (size_t)h * hd;
-  bool bad = false;
-  // Raw rows: the query head, then the group's keys and values of chunk
-  // positions 0..t.
-  for (int i = tid; i < (t + 2) * hd; i += kDecThreads) {
-    const int r = i >> 6, d = i & 63;
-    const float v = r == 0 ? q[((size_t)t * H + h) * hd + d] : R.k[((size_t)(r - 1) * KV + g) * hd + d];
-    bad |= !finite(v);
-    if (r == 0) qs[d] = v;
-    else kn[r - 1][d] = v;
-  }
-  for (int i = tid; i < (t + 1) * hd; i += kDecThreads)
-    vn[i >> 6][i & 63] = R.v[((size_t)(i >> 6) * KV + g) * hd + (i & 63)];
-  __syncthreads();
-  // RoPE: x0*c - x1*s, x0*s + x1*c on pairs (2j, 2j+1) or (j, j + half).
-  for (int p = tid; p < (t + 2) * half; p += kDecThreads) {
-    const int r = p / half, j = p - r * half;
-    float* base = r == 0 ? qs : kn[r - 1];
-    const int ppos = r == 0 ? pos : pb + r - 1;
-    const int ia = R.split_half ? j : 2 * j;
-    const int ib = R.split_half ? j + half : 2 * j + 1;
-    const float x0 = base[ia], x1 = base[ib];
-    const float c = R.rc[(size_t)ppos * half + j], sn = R.rs[(size_t)ppos * half + j];
-    const float y0 = x0 * c - x1 * sn;
-    const float y1 = x0 * sn + x1 * c;
-    bad |= any_nonfinite(y0, y1);
-    base[ia] = y0;
-    base[ib] = y1;
-  }
-  __syncthreads();
-  if (h % G == 0 && tid < hd) {
-    const size_t off = (((size_t)layer * KV + g) * n_ctx + pos) * hd + tid;
-    const float kv = kn[t][tid], vv = vn[t][tid];
-    bad |= any_nonfinite(kv, vv);
-    R.kc[off] = kv;
-    R.vc[off] = vv;
-  }
-  if (len == 1) {  // a single score copies V exactly (lib.rs:2319-2321)
-    if (tid < hd) o[tid] = vn[0][tid];
-    if (bad) flag(err, ERRBIT_NON_FINITE);
-    return;
-  }
-  // scores: dot_f32_ref(q, k_j) * scale.  Eight lanes per key: lane r forms
-  // the 8-lane accumulator r (dims r, r + 8, ..., r + 56 in order), three
-  // shuffle levels then give ((a0+a1)+(a2+a3))+((a4+a5)+(a6+a7)).  A round
-  // covers 128 keys; the key rows of kScoreDepth rounds are in flight.
-  {
-    constexpr int kKeysPerRound = kDecThreads / 8, kScoreDepth = 4;
-    const int r = tid & 7, kq = tid >> 3;
-    float qr[8];
-#pragma unroll
-    for (int u = 0; u < 8; u++) qr[u] = qs[r + 8 * u];
-    const int nrounds = (len + kKeysPerRound - 1) / kKeysPerRound;
-    // Key rows are loaded unconditionally (rows outside the cached part read
-    // row 0 and are replaced from LDS at use), so the loads in flight are
-    // counted rather than drained.
-    float kb[kScoreDepth][8];
-    auto load_keys = [&](float (&dst)[8], int round) {
-      const int j = kq + kKeysPerRound * round;
-      const float* kr = keys + (size_t)(j < pb ? j : 0) * hd + r;
-#pragma unroll
-      for (int u = 0; u < 8; u++) dst[u] = kr[8 * u];
-    };
-#pragma unroll
-    for (int d = 0; d < kScoreDepth; d++) load_keys(kb[d], d);
-    for (int r0 = 0; r0 < nrounds; r0 += kScoreDepth) {
-#pragma unroll
-      for (int d = 0; d < kScoreDepth; d++) {
-        const int round = r0 + d;
-        const int j = kq + kKeysPerRound * round;
-        const int jv = j - pb < 0 ? 0 : (j - pb < kDecMaxT ? j - pb : kDecMaxT - 1);
-        float acc = 0.0f;
-#pragma unroll
-        for (int u = 0; u < 8; u++) acc += qr[u] * (j < pb ? kb[d][u] : kn[jv][r + 8 * u]);
-        const float s3 = finish_8lane_dpp(acc);
-        if (r == 0 && j < len) {
-          const float sv = s3 * scale;
-          if (!finite(sv)) bad = true;
-          sc[j] = sv;
-        }
-        load_keys(kb[d], round + kScoreDepth);
-      }
-    }
-  }
-  __syncthreads();
-  // softmax_in_place (lib.rs:2361-2388)
-  float mx = -__builtin_huge_valf();
-  for (int j = tid; j < len; j += kDecThreads) mx = fmaxf(mx, sc[j]);
-  mx = wave_fmax(mx);
-  if (lane == 0) red[wave] = mx;
-  __syncthreads();
-  mx = red[0];
-#pragma unroll
-  for (int w = 1; w < kDecThreads / 64; w++) mx = fmaxf(mx, red[w]);
-  for (int j = tid; j < len; j += kDecThreads) sc[j] = exp_clamped(sc[j] - mx);
-  __syncthreads();
-  if (tid < 8) {
-    float acc = 0.0f;
-    int j = tid;
-    for (; j + 56 < len; j += 64) {
-      const float e0 = sc[j], e1 = sc[j + 8], e2 = sc[j + 16], e3 = sc[j + 24];
-      const float e4 = sc[j + 32], e5 = sc[j + 40], e6 = sc[j + 48], e7 = sc[j + 56];
-      acc += e0; acc += e1; acc += e2; acc += e3;
-      acc += e4; acc += e5; acc += e6; acc += e7;
-    }
-    for (; j < len; j += 8) acc += sc[j];
-    zc[tid] = acc;
-  }
-  __syncthreads();
-  const float z = finish_8lane(zc);
-  if (!finite(z) || z == 0.0f) bad = true;
-  for (int j = tid; j < len; j += kDecThreads) {
-    const float p = sc[j] / z;
-    if (!finite(p)) bad = true;
-    sc[j] = p;
-  }
-  __syncthreads();
-  // P.V.  Thread tid owns row jr of each tile and dimensions c4 .. c4 + 3:
-  // a wave covers 16 rows x 16 dimensions, so its product stores (dimension-
-  // major) spread over all LDS banks while each row's 64 bytes stay one
-  // coalesced global segment.
-  const int ntiles = (len + kDecTile - 1) / kDecTile;
-  const int jr = 16 * (wave & 3) + (lane & 15), c4 = 16 * (wave >> 2) + 4 * (lane >> 4);
-  // Every ring load is issued unconditionally (rows past the cached part
-  // read row 0 and are replaced at use), so the compiler can count the
-  // loads in flight instead of draining them all at each tile.
-  float4 ring[kDecDepth];
-#pragma unroll
-  for (int u = 0; u < kDecDepth; u++) {
-    const int j = u * kDecTile + jr;
-    ring[u] = *reinterpret_cast<const float4*>(vals + (size_t)(j < pb ? j : 0) * hd + c4);
-  }
-  float a = 0.0f;
-  for (int k0 = 0; k0 < ntiles; k0 += kDecDepth) {
-#pragma unroll
-    for (int u = 0; u < kDecDepth; u++) {
-      const int k = k0 + u;
-      const int j = k * kDecTile + jr;
-      // chunk rows come from LDS; rows past len contribute nothing
-      const int jv = j - pb < 0 ? 0 : (j - pb < kDecMaxT ? j - pb : kDecMaxT - 1);
-      const float4 vl = *reinterpret_cast<const float4*>(&vn[jv][c4]);
-      const float4 v = j < pb ? ring[u] : (j < len ? vl : make_float4(0.f, 0.f, 0.f, 0.f));
-      const float p = j < len ? sc[j < len ? j : 0] : 0.0f;
-      if (k < ntiles) {
-        float* pr = prod[k & 1];
-        pr[(c4 + 0) * kDecStride + jr] = p * v.x;
-        pr[(c4 + 1) * kDecStride + jr] = p * v.y;
-        pr[(c4 + 2) * kDecStride + jr] = p * v.z;
-        pr[(c4 + 3) * kDecStride + jr] = p * v.w;
-      }
-      // issued on every step (rows outside the cached part read row 0)
-      const int jn = j + kDecDepth * kDecTile;
-      ring[u] = *reinterpret_cast<const float4*>(vals + (size_t)(jn < pb ? jn : 0) * hd + c4);
-      __syncthreads();
-      if (k < ntiles && wave == 0) {
-        const float* pr = prod[k & 1] + lane * kDecStride;
-        const int n = min(kDecTile, len - k * kDecTile);
-        if (n == kDecTile) {
-          // all sixteen reads first, then the 64 adds in order
-          float4 p4[kDecTile / 4];
-#pragma unroll
-          for (int q4 = 0; q4 < kDecTile / 4; q4++)
-            p4[q4] = *reinterpret_cast<const float4*>(pr + 4 * q4);
-#pragma unroll
-          for (int q4 = 0; q4 < kDecTile / 4; q4++) {
-            a += p4[q4].x;
-            a += p4[q4].y;
-            a += p4[q4].z;
-            a += p4[q4].w;
-          }
-        } else {
-          for (int jj = 0; jj < n; jj++) a += pr[jj];
-        }
-      }
-    }
-  }
-  if (wave == 0) {
-    if (!finite(a)) bad = true;
-    o[lane] = a;
-  }
-  if (bad) flag(err, ERRBIT_NON_FINITE);
-}
-
-// Decode shape split over many workgroups.  One workgroup per (head,
-// position) streams the whole K and V prefix through a single CU, whose
-// load bandwidth then bounds the launch (about 800 KB at position 1560 for a
-// Qwen2.5-0.5B-shaped head).  Here k_attn_split_scores gives every 128-key
-// block its own workgroup, and k_attn_split_pv gives every 16 dimensions of
-// a head its own, so the K and V streams spread over the chip.  Values and
-// order are those of k_attention_dec: the same 8-lane dot per score (the
-// scores cross the launch boundary through memory as f32), the same max,
-// clamped exps, 8-lane Z chains and divisions, and per dimension the same
-// ascending chain of products p_j * v_j[d].
+// Decode attention (one to four positions), with the RoPE and cache store
+// of the chunk folded in.  A head's score row and its P.V sums are spread
+// over the chip: k_attn_split_scores gives every 128-key block of a (head,
+// position) a workgroup, which applies RoPE (lib.rs:2011-2051) to its query
+// head and to the chunk's new keys of its KV group in LDS (cache rows before
+// the chunk come from memory, the chunk's own rows from LDS, so no workgroup
+// reads a row another one writes) and stores the scores; the P.V launch
+// gives every 16 dimensions one, which forms the softmax of the row again:
+// k_attn_split_pv for 64-wide heads up to kSplitMaxRows keys, k_attn_tiles_pv
+// for longer rows and other widths.  Rows of up to kFusedMaxLen keys of
+// 64-wide heads do both in one launch (k_attn_fused).  Values and order: 8-lane dots, scale, max, clamped exps,
+// the eight Z chains, divisions, and per dimension the ascending chain of
+// products p_j * v_j[d] (lib.rs:2319-2420).
+constexpr int kDecMaxT = 4;
 constexpr int kSplitKeys = 128;   // keys per score workgroup
 constexpr int kSplitDims = 16;    // dimensions per P.V workgroup
+// Threads per score workgroup: at least one per rotated pair of the query
+// and of kDecMaxT keys.
+__host__ __device__ constexpr int split_score_threads(int hd) { return hd <= 64 ? 256 : 512; }
 
 // RoPE (lib.rs:2011-2051) of the query head and of the chunk's keys of its
 // group into LDS, from the raw projections; returns whether any input or
 // output is non-finite.  Each thread takes at most one rotated pair (the
-// launch has at least (kDecMaxT + 1) * 32 threads), whose table entries it
+// launch has at least (kDecMaxT + 1) * hd / 2 threads), whose table entries it
 // loads together with the raw rows, before the first barrier.
+template <int HD>
 __device__ bool split_rope_rows(const float* q, const RopeIn& R, int h, int g, int t, int KV, int H,
-                                int pb, float* qs, float (*kn)[64]) {
-  constexpr int hd = 64;
+                                int pb, float* qs, float (*kn)[HD]) {
+  constexpr int hd = HD;
   const int tid = threadIdx.x, nt = blockDim.x, half = R.rope_dim / 2;
   const int np = (t + 2) * half;
   const int p = tid < np ? tid : 0;
@@ -1399,7 +1190,7 @@ __device__ bool split_rope_rows(const float* q, const RopeIn& R, int h, int g, i
   const float c = R.rc[(size_t)ppos * half + pj], sn = R.rs[(size_t)ppos * half + pj];
   bool bad = false;
   for (int i = tid; i < (t + 2) * hd; i += nt) {
-    const int r = i >> 6, d = i & 63;
+    const int r = i / hd, d = i % hd;
     const float v = r == 0 ? q[((size_t)t * H + h) * hd + d] : R.k[((size_t)(r - 1) * KV + g) * hd + d];
     bad |= !finite(v);
     if (r == 0) qs[d] = v;
@@ -1424,13 +1215,14 @@ __device__ bool split_rope_rows(const float* q, const RopeIn& R, int h, int g, i
 // Scores of keys [128 b, 128 b + 128) for (head h, chunk position t); the
 // workgroup holding key `pos` of the group's first head also stores the
 // position's key and value rows into the cache.  scores: [T][H][n_ctx].
-__global__ void __launch_bounds__(256) k_attn_split_scores(const float* q, RopeIn R, int layer,
+template <int HD>
+__global__ void __launch_bounds__(split_score_threads(HD)) k_attn_split_scores(const float* q, RopeIn R, int layer,
                                                            int pos0, int H, int KV, int n_ctx,
                                                            float scale, float* scores,
                                                            const int* pos_dev, int* err) {
-  __shared__ __align__(16) float qs[64];
-  __shared__ __align__(16) float kn[kDecMaxT][64];
-  constexpr int hd = 64;
+  __shared__ __align__(16) float qs[HD];
+  __shared__ __align__(16) float kn[kDecMaxT][HD];
+  constexpr int hd = HD, DU = HD / 8;
   const int b = blockIdx.x, h = blockIdx.y, t = blockIdx.z, tid = threadIdx.x;
   const int G = H / KV, g = h / G;
   const int pb = pos_dev ? *pos_dev : pos0;
@@ -1438,23 +1230,24 @@ __global__ void __launch_bounds__(256) k_attn_split_scores(const float* q, RopeI
   const int j0 = b * kSplitKeys;
   if (j0 >= len) return;  // the grid covers the longest row the launch can see
   // Eight lanes per key: lane r forms the 8-lane accumulator r (dims r,
-  // r + 8, ..., r + 56 in order); three shuffle levels give
-  // ((a0+a1)+(a2+a3))+((a4+a5)+(a6+a7)).  All four rounds' cached key rows
+  // r + 8, ... in order); three shuffle levels give
+  // ((a0+a1)+(a2+a3))+((a4+a5)+(a6+a7)).  All rounds' cached key rows
   // are loaded before the RoPE phase, whose loads and barriers they then
   // overlap (rows outside the cached part read row 0 and are replaced from
   // LDS at use; a barrier waits for LDS only, not for these loads).
-  constexpr int kRounds = kSplitKeys / 32;
+  constexpr int kPer = split_score_threads(HD) / 8;  // keys per round
+  constexpr int kRounds = kSplitKeys / kPer;
   const float* keys = R.kc + ((size_t)layer * KV + g) * n_ctx * hd;
   const int r = tid & 7, kq = tid >> 3;
-  float kb[kRounds][8];
+  float kb[kRounds][DU];
 #pragma unroll
   for (int d = 0; d < kRounds; d++) {
-    const int j = j0 + kq + 32 * d;
+    const int j = j0 + kq + kPer * d;
     const float* kr = keys + (size_t)(j < pb ? j : 0) * hd + r;
 #pragma unroll
-    for (int u = 0; u < 8; u++) kb[d][u] = kr[8 * u];
+    for (int u = 0; u < DU; u++) kb[d][u] = kr[8 * u];
   }
-  bool bad = split_rope_rows(q, R, h, g, t, KV, H, pb, qs, kn);
+  bool bad = split_rope_rows<HD>(q, R, h, g, t, KV, H, pb, qs, kn);
   if (h % G == 0 && pos / kSplitKeys == b && tid < hd) {
     const size_t off = (((size_t)layer * KV + g) * n_ctx + pos) * hd + tid;
     const float kv = kn[t][tid], vv = R.v[((size_t)t * KV + g) * hd + tid];
@@ -1464,16 +1257,16 @@ __global__ void __launch_bounds__(256) k_attn_split_scores(const float* q, RopeI
   }
   if (len > 1) {  // a single score is never formed (the output copies V)
     float* srow = scores + ((size_t)t * H + h) * n_ctx;
-    float qr[8];
+    float qr[DU];
 #pragma unroll
-    for (int u = 0; u < 8; u++) qr[u] = qs[r + 8 * u];
+    for (int u = 0; u < DU; u++) qr[u] = qs[r + 8 * u];
 #pragma unroll
     for (int d = 0; d < kRounds; d++) {
-      const int j = j0 + kq + 32 * d;
+      const int j = j0 + kq + kPer * d;
       const int jv = j - pb < 0 ? 0 : (j - pb < kDecMaxT ? j - pb : kDecMaxT - 1);
       float acc = 0.0f;
 #pragma unroll
-      for (int u = 0; u < 8; u++) acc += qr[u] * (j < pb ? kb[d][u] : kn[jv][r + 8 * u]);
+      for (int u = 0; u < DU; u++) acc += qr[u] * (j < pb ? kb[d][u] : kn[jv][r + 8 * u]);
       const float s3 = finish_8lane_dpp(acc);
       if (r == 0 && j < len) {
         const float sv = s3 * scale;
@@ -1532,7 +1325,7 @@ constexpr int kPvThreads = 1024;
 constexpr int kSplitVBlocks = kSplitMaxRows / kPvThreads;  // 4-row blocks per thread
 static_assert(kPvThreads / 64 == 16 && 4 * (kPvThreads / 4) == kPvThreads, "one wave per dimension, 256 row quads");
 
-struct SplitLayout {  // LDS of k_attn_split_pv, in floats
+struct SplitLayout {  // LDS of k_attn_fused and k_attn_split_pv, in floats
   int len4, zs, ld, zoff, voff, total;
 };
 
@@ -1676,8 +1469,163 @@ __global__ void __launch_bounds__(kPvThreads) k_attn_split_pv(const float* score
   if (bad) flag(err, ERRBIT_NON_FINITE);
 }
 
+// softmax_in_place (lib.rs:2361-2388) of the score row, then
+// out[d] = 0; out[d] += p_j * v_j[d] (j ascending, lib.rs:2390-2420) for
+// dimensions [16 blockIdx.x, +16), rows of any length and heads of any
+// width.  The score row stays in LDS (as probabilities); V passes through it
+// dimension-major in tiles of 256 keys, double-buffered, with four tiles of
+// loads in flight per thread (one tile's sums take about 1400 cycles, less
+// than a memory round trip).  The chain-major exps of the Z chains share LDS
+// with the tiles: they end before the first tile is stored.  1024 threads,
+// so that the latency-bound phases (the clamped exps, the divisions) have
+// four waves per SIMD; the Z and P.V chains are DPP chains (chain_group_lds
+// / chain_group_dot_lds: one chain per 16-lane row, each product formed just
+// before its add).
+//
+// Bound by the serial P.V sums (about 5.5 cycles per key).  Scores and P.V
+// together, 128-wide heads, 8 query / 2 key heads: 10.5 us at 500 keys, 12.4
+// at 1000, 20.3 at 2903, 24.0 at 4000, against 165, 347, 1003 and 1377 us of
+// the one-workgroup-per-group kernel that served this width before.  64-wide
+// heads up to 2048 keys keep k_attn_split_pv, whose whole row of V is loaded
+// ahead of the softmax (token of the Qwen2.5-0.5B shape at 1501 keys 1145 us
+// against 1158, of the TinyLlama-1.1B shape at 700 keys 1539 against 1568);
+// at 2500 and 4000 keys this kernel replaces one that streamed a head's rows
+// through one workgroup.
+constexpr int kTileKeys = 256;
+constexpr int kTileLd = kTileKeys + 4;  // one dimension's keys (the transposing stores hit distinct banks)
+
+constexpr int kZSeg = 8192;            // exps per pass of the Z chains
+constexpr int kZStride = kZSeg / 8 + 4;  // chain-major row
+constexpr int kTileFloats = 2 * kSplitDims * kTileLd;
+static_assert(8 * kZStride <= kTileFloats, "the Z segment fits the V tiles' area");
+
+__host__ __device__ inline int tiles_len4(int maxlen) { return (maxlen + 3) & ~3; }
+size_t tiles_pv_smem(int maxlen) { return ((size_t)tiles_len4(maxlen) + kTileFloats) * sizeof(float); }
+
+template <int HD>
+__global__ void __launch_bounds__(kPvThreads) k_attn_tiles_pv(const float* scores, RopeIn R, int layer, int pos0,
+                                                              int H, int KV, int n_ctx, int maxlen, float* out,
+                                                              const int* pos_dev, int* err) {
+  extern __shared__ __align__(16) float pr[];
+  constexpr int NW = kPvThreads / 64;
+  __shared__ float red[NW];
+  __shared__ float zc[8];
+  constexpr int hd = HD;
+  const int dg = blockIdx.x, h = blockIdx.y, t = blockIdx.z, tid = threadIdx.x;
+  const int wave = tid >> 6, lane = tid & 63;
+  const int G = H / KV, g = h / G;
+  const int pb = pos_dev ? *pos_dev : pos0;
+  const int pos = pb + t, len = pos + 1;
+  const int d0 = dg * kSplitDims;
+  float* zcm = pr + tiles_len4(maxlen);  // [8][kZStride]
+  float* vt = zcm;                       // [2][kSplitDims][kTileLd]
+  const float* vals = R.vc + ((size_t)layer * KV + g) * n_ctx * hd;
+  float* o = out + ((size_t)t * H + h) * hd + d0;
+  bool bad = false;
+  if (len == 1) {  // a single score copies V exactly (lib.rs:2319-2321)
+    if (tid < kSplitDims) o[tid] = R.v[((size_t)t * KV + g) * hd + d0 + tid];
+    return;
+  }
+  // V rows and scores through buffer loads bounded by len: past it they
+  // return zeros without a memory request.  The scores launch has stored the
+  // current positions' rows.
+  const float* srow = scores + ((size_t)t * H + h) * n_ctx;
+  const BufRsrc srs = buf_rsrc(srow, (uint32_t)len * 4u);
+  const BufRsrc vrs = buf_rsrc(vals, (uint32_t)len * hd * 4u);
+  const int jr = tid >> 2, c = 4 * (tid & 3);  // this thread's key of a tile and its dimensions
+  auto vload = [&](int k) { return buf_load_f32x4(vrs, ((k * kTileKeys + jr) * hd + d0 + c) * 4); };
+  float mx = -__builtin_huge_valf();
+  for (int j0 = 0; j0 < len; j0 += 4 * kPvThreads) {
+    float sv[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) sv[k] = buf_load_f32(srs, 4 * (j0 + kPvThreads * k + tid));
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const int j = j0 + kPvThreads * k + tid;
+      if (j < len) {
+        pr[j] = sv[k];
+        mx = fmaxf(mx, sv[k]);
+      }
+    }
+  }
+  float4 v0 = vload(0), v1 = vload(1), v2 = vload(2), v3 = vload(3);
+  mx = wave_fmax(mx);
+  if (lane == 0) red[wave] = mx;
+  __syncthreads();
+  mx = red[0];
+#pragma unroll
+  for (int w = 1; w < NW; w++) mx = fmaxf(mx, red[w]);
+  // The exps of one segment, also stored chain-major (element j at chain
+  // j % 8) and padded to the longest chain with +0.0, which no sum of exps
+  // changes; then the eight Z chains as DPP chains, chain c on the 16-lane
+  // row c % 4 of wave c / 4.
+  float zsum = 0.0f;
+  for (int s0 = 0; s0 < len; s0 += kZSeg) {
+    const int n = len - s0 < kZSeg ? len - s0 : kZSeg, n8 = (n + 7) & ~7;
+#pragma unroll 2
+    for (int j = tid; j < n8; j += kPvThreads) {
+      const float e = j < n ? exp_clamped(pr[j < n ? s0 + j : 0] - mx) : 0.0f;
+      if (j < n) pr[s0 + j] = e;
+      zcm[(j & 7) * kZStride + (j >> 3)] = e;
+    }
+    __syncthreads();
+    if (tid < 128) zsum = chain_group_lds<16>(zsum, zcm + (tid >> 4) * kZStride, n8 / 8);
+    __syncthreads();
+  }
+  if (tid < 128 && (tid & 15) == 0) zc[tid >> 4] = zsum;
+  __syncthreads();
+  const float z = finish_8lane(zc);
+  bad |= !finite(z) || z == 0.0f;
+  for (int j = tid; j < len; j += kPvThreads) {
+    const float p = pr[j] / z;
+    bad |= !finite(p);
+    pr[j] = p;
+  }
+  auto vstore = [&](const float4& v, int b) {
+    float* d = vt + (b * kSplitDims + c) * kTileLd + jr;
+    d[0] = v.x;
+    d[kTileLd] = v.y;
+    d[2 * kTileLd] = v.z;
+    d[3 * kTileLd] = v.w;
+  };
+  const int nt = (len + kTileKeys - 1) / kTileKeys;
+  const bool adds = tid < 64 * (kSplitDims / 4);
+  float a = 0.0f;
+  vstore(v0, 0);
+  v0 = vload(4);
+  __syncthreads();
+  // Tile k is summed from buffer k % 2 while tile k + 1 is stored in the
+  // other.  Tiles past the row hold zeros and are summed over no keys; every
+  // load and store is unconditional (a refill under a branch waits for all
+  // loads in flight).
+#define DTL_PV_TILE(k, vn, kn)                                                            \
+  do {                                                                                    \
+    vstore(vn, ((k) + 1) & 1);                                                            \
+    vn = vload(kn);                                                                       \
+    if (adds) {                                                                           \
+      const int left = len - (k) * kTileKeys;                                             \
+      const int n = left < 0 ? 0 : (left < kTileKeys ? left : kTileKeys);                 \
+      a = chain_group_dot_lds<16>(a, pr + (n > 0 ? (k) : 0) * kTileKeys,                  \
+                                  vt + (((k) & 1) * kSplitDims + (tid >> 4)) * kTileLd, n); \
+    }                                                                                     \
+    __syncthreads();                                                                      \
+  } while (0)
+  for (int k = 0; k < nt; k += 4) {
+    DTL_PV_TILE(k, v1, k + 5);
+    DTL_PV_TILE(k + 1, v2, k + 6);
+    DTL_PV_TILE(k + 2, v3, k + 7);
+    DTL_PV_TILE(k + 3, v0, k + 8);
+  }
+#undef DTL_PV_TILE
+  if (adds && (tid & 15) == 0) {
+    bad |= !finite(a);
+    o[tid >> 4] = a;
+  }
+  if (bad) flag(err, ERRBIT_NON_FINITE);
+}
+
 // Decode attention in one launch for rows of at most kFusedMaxLen keys: the
-// work of k_attn_split_scores and k_attn_split_pv for (16 dimensions, head,
+// work of k_attn_split_scores and k_attn_tiles_pv for (16 dimensions, head,
 // position) in one workgroup.  Each of a head's four workgroups forms the
 // whole score row itself (the scores never leave LDS), which costs a read of
 // the head's cached keys per workgroup: cheap for short rows, where the
@@ -1746,7 +1694,7 @@ __global__ void __launch_bounds__(kPvThreads) k_attn_fused(const float* q, RopeI
 #pragma unroll
     for (int u = 0; u < 8; u++) kb[d][u] = kr[8 * u];
   }
-  bad |= split_rope_rows(q, R, h, g, t, KV, H, pb, qs, kn);
+  bad |= split_rope_rows<64>(q, R, h, g, t, KV, H, pb, qs, kn);
   if (dg == 0 && h % G == 0 && tid < hd) {
     const size_t off = (((size_t)layer * KV + g) * n_ctx + pos) * hd + tid;
     const float kv = kn[t][tid], vv = R.v[((size_t)t * KV + g) * hd + tid];
@@ -1865,62 +1813,77 @@ size_t attention_grp_smem(int H, int KV, int hd, int n_ctx) {
   return ((size_t)G * n_ctx + (size_t)(kAttnTile + 1) * hd + (size_t)G * hd) * sizeof(float);
 }
 
-// Dynamic LDS of k_attention_dec (the score row); its static LDS holds the
-// product tiles.
-constexpr size_t kDecMaxScoreBytes = 112 * 1024;
+// LDS the decode attention may use (of 160 KB).
+constexpr size_t kDecLds = 158 * 1024;
 
-bool attention_pos_dev_supported(int hd, int T, int n_ctx) {
-  return hd == 64 && T <= kDecMaxT && (size_t)n_ctx * sizeof(float) <= kDecMaxScoreBytes;
-}
+namespace {
+// The head widths k_attn_split_scores and k_attn_tiles_pv are built for.
+bool tiles_width(int hd) { return hd == 16 || hd == 32 || hd == 64 || hd == 80 || hd == 96 || hd == 128; }
+}  // namespace
+
+bool attention_pos_dev_supported(int hd, int T, int n_ctx) { return attention_dec_applies(hd, T, 0, n_ctx, true); }
 
 bool attention_dec_applies(int hd, int T, int pos0, int n_ctx, bool pos_in_device) {
-  const size_t smem = (size_t)(pos_in_device ? n_ctx : pos0 + T) * sizeof(float);
-  return hd == 64 && T <= kDecMaxT && smem <= kDecMaxScoreBytes;
+  const int maxlen = pos_in_device ? n_ctx : pos0 + T;
+  if (T > kDecMaxT) return false;
+  return tiles_width(hd) && tiles_pv_smem(maxlen) <= kDecLds;
 }
 
 int attention_fused_max_len() { return kFusedMaxLen; }
 
 void launch_attention_dec(const float* q, const RopeIn& R, int layer, int T, int pos0, int H,
-                          int KV, int n_ctx, int maxlen_dev, float scale, float* scores, float* out,
+                          int KV, int hd, int n_ctx, int maxlen_dev, float scale, float* scores, float* out,
                           const int* pos_dev, int* err, hipStream_t s) {
   // With the position in device memory the grids and LDS are sized for the
   // longest row the replays may see.
   const int maxlen = pos_dev ? maxlen_dev : pos0 + T;
-  const size_t smem = (size_t)maxlen * sizeof(float);
-  const size_t pv_smem = split_pv_smem(maxlen);
-  if (maxlen <= kFusedMaxLen) {
+  if (hd == 64 && maxlen <= kFusedMaxLen) {
     static bool attr_fused_set = false;
     if (!attr_fused_set) {
       (void)hipFuncSetAttribute((const void*)k_attn_fused, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                158 * 1024);
+                                (int)kDecLds);
       attr_fused_set = true;
     }
-    launch_kernel(k_attn_fused, dim3(64 / kSplitDims, H, T), dim3(kPvThreads), pv_smem, s, q, R, layer,
-                  pos0, H, KV, n_ctx, maxlen, scale, out, pos_dev, err);
+    launch_kernel(k_attn_fused, dim3(64 / kSplitDims, H, T), dim3(kPvThreads), split_pv_smem(maxlen), s, q, R,
+                  layer, pos0, H, KV, n_ctx, maxlen, scale, out, pos_dev, err);
     return;
   }
-  if (maxlen <= kSplitMaxRows && pv_smem <= 158 * 1024) {
+  auto scores_launch = [&](auto hdc) {
+    constexpr int HD = decltype(hdc)::value;
+    launch_kernel(k_attn_split_scores<HD>, dim3((maxlen + kSplitKeys - 1) / kSplitKeys, H, T),
+                  dim3(split_score_threads(HD)), 0, s, q, R, layer, pos0, H, KV, n_ctx, scale, scores, pos_dev, err);
+  };
+  if (hd == 64 && maxlen <= kSplitMaxRows) {
     static bool attr_pv_set = false;
     if (!attr_pv_set) {
       (void)hipFuncSetAttribute((const void*)k_attn_split_pv,
-                                hipFuncAttributeMaxDynamicSharedMemorySize, 158 * 1024);
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)kDecLds);
       attr_pv_set = true;
     }
-    launch_kernel(k_attn_split_scores, dim3((maxlen + kSplitKeys - 1) / kSplitKeys, H, T), dim3(256), 0,
-                  s, q, R, layer, pos0, H, KV, n_ctx, scale, scores, pos_dev, err);
-    launch_kernel(k_attn_split_pv, dim3(64 / kSplitDims, H, T), dim3(kPvThreads), pv_smem, s, scores, R,
-                  layer, pos0, H, KV, n_ctx, maxlen, out, pos_dev, err);
+    scores_launch(std::integral_constant<int, 64>());
+    launch_kernel(k_attn_split_pv, dim3(64 / kSplitDims, H, T), dim3(kPvThreads), split_pv_smem(maxlen), s, scores,
+                  R, layer, pos0, H, KV, n_ctx, maxlen, out, pos_dev, err);
     return;
   }
-  // Longer windows: one workgroup per (head, position).
-  static bool attr_dec_set = false;
-  if (!attr_dec_set) {
-    (void)hipFuncSetAttribute((const void*)k_attention_dec,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)kDecMaxScoreBytes);
-    attr_dec_set = true;
+  const size_t tiles_smem = tiles_pv_smem(maxlen);
+  auto go = [&](auto hdc) {
+    constexpr int HD = decltype(hdc)::value;
+    static const bool attr = hipFuncSetAttribute((const void*)k_attn_tiles_pv<HD>,
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                 (int)kDecLds) == hipSuccess;
+    (void)attr;
+    scores_launch(hdc);
+    launch_kernel(k_attn_tiles_pv<HD>, dim3(HD / kSplitDims, H, T), dim3(kPvThreads), tiles_smem, s, scores, R,
+                  layer, pos0, H, KV, n_ctx, maxlen, out, pos_dev, err);
+  };
+  switch (hd) {
+    case 16: return go(std::integral_constant<int, 16>());
+    case 32: return go(std::integral_constant<int, 32>());
+    case 64: return go(std::integral_constant<int, 64>());
+    case 80: return go(std::integral_constant<int, 80>());
+    case 96: return go(std::integral_constant<int, 96>());
+    default: return go(std::integral_constant<int, 128>());
   }
-  launch_kernel(k_attention_dec, dim3(H, T), dim3(kDecThreads), smem, s, q, R, layer, pos0, H, KV,
-                n_ctx, scale, out, pos_dev, err);
 }
 
 bool attention_quantizes_q8a(int hd, int H, int KV, int T, int pos0, int n_ctx) {

@@ -92,6 +92,66 @@ def test_f32_model_matches_oracle(name, heads, kv_heads, chunk):
     _compare_with_oracle(synth.build_model(w, layers=2), synth.tokens(w, min(36, 3 * chunk)), chunk)
 
 
+@pytest.mark.parametrize("name,d,heads,kv_heads", [
+    ("smollm2", 576, 36, 12),  # 16-wide heads
+    ("qwen05", 448, 14, 2),    # 32, split-half RoPE, biases
+    ("smollm2", 640, 8, 4),    # 80
+    ("smollm2", 576, 6, 6),    # 96, one query head per key head
+    ("qwen05", 896, 7, 1),     # 128
+    ("smollm2", 128, 2, 1),    # 64
+])
+@pytest.mark.parametrize("prefix", [0, 250, 2045])
+@pytest.mark.parametrize("graph", [True, False])
+def test_decode_attention_head_widths_match_oracle(monkeypatch, name, d, heads, kv_heads, prefix, graph):
+    # Decode attention of one to four positions at the edges of its key tiles
+    # (256 keys), of the score blocks (128) and of the 2048-key limit of the
+    # 64-wide kernels, by graph replay and by eager launches.
+    import dataclasses
+
+    from detllm_amd import synth
+
+    if not graph:
+        monkeypatch.setenv("DETLLM_NO_GRAPH", "1")
+    if prefix > 1000:  # a narrow model of the same head width keeps the oracle quick
+        hd = d // heads
+        d, heads, kv_heads = 2 * hd + (-2 * hd) % 32, 2, 1
+        if d != 2 * hd:
+            pytest.skip("no narrow model of this head width has whole 32-element blocks")
+    w = dataclasses.replace(synth.WORKLOADS[name], d=d, heads=heads, kv_heads=kv_heads, ff=64, vocab=300, ctx=2100)
+    data = synth.build_model(w, layers=1)
+    toks = [int(t) for t in synth.tokens(w, prefix + 14)]
+    ref = detref.Model(data).logits(toks)
+    m = _model(data)
+    with m.forward_workspace(2100, 64) as s:
+        for p in range(0, prefix, 64):
+            s.forward_chunk(toks[p:min(prefix, p + 64)], p)
+        p = prefix
+        for n in (1, 1, 2, 1, 4, 1, 3, 1):
+            got = s.forward_chunk(toks[p:p + n], p, want_logits=True)
+            assert np.array_equal(got.view(np.uint32), ref[p:p + n].view(np.uint32)), (p, n)
+            p += n
+
+
+def test_decode_attention_long_row_matches_oracle():
+    # The Z chains run in segments of 8192 exps: rows just below, at and past one.
+    import dataclasses
+
+    from detllm_amd import synth
+
+    w = dataclasses.replace(synth.WORKLOADS["smollm2"], d=32, heads=2, kv_heads=1, ff=32, vocab=257, ctx=8300)
+    data = synth.build_model(w, layers=1)
+    toks = [int(t) for t in synth.tokens(w, 8300)]
+    ref = detref.Model(data).logits(toks)
+    with _model(data).forward_workspace(8300, 512) as s:
+        for p in range(0, 8190, 512):
+            s.forward_chunk(toks[p:min(8190, p + 512)], p)
+        for p, n in ((8190, 1), (8191, 1), (8192, 1), (8193, 4), (8299, 1)):
+            if p == 8299:
+                s.forward_chunk(toks[8197:8299], 8197)
+            got = s.forward_chunk(toks[p:p + n], p, want_logits=True)
+            assert np.array_equal(got.view(np.uint32), ref[p:p + n].view(np.uint32)), (p, n)
+
+
 @pytest.mark.parametrize("name,chunk", [("qwen05", 1), ("qwen05", 8), ("smollm2", 5)])
 @pytest.mark.parametrize("fused", [True, False])
 def test_decode_gemv_fusion_matches_oracle(monkeypatch, name, chunk, fused):
@@ -296,11 +356,11 @@ def test_decode_attention_regimes_match_oracle(monkeypatch, graph):
 
     graph: positions below 512 replay the graph whose attention is one launch
     (k_attn_fused); from 512 on, the graph sized for the whole window, whose
-    attention runs one workgroup per (head, position) (k_attention_dec).
+    attention takes its tiled P.V launch (k_attn_tiles_pv).
     eager (DETLLM_NO_GRAPH=1, the path under profiling or after a failed
     capture): the launch is sized by the row: k_attn_fused up to 512 keys,
     the split pair (k_attn_split_scores + k_attn_split_pv) up to 2048,
-    k_attention_dec beyond; the positions between are forwarded in chunks of
+    k_attn_tiles_pv beyond; the positions between are forwarded in chunks of
     64 (chunk attention)."""
     import dataclasses
 
