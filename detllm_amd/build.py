@@ -44,9 +44,10 @@ NUMERIC_FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
 
-# Per-source additions: the MFMA-product GEMMs take their results in VGPRs
-# (the VALU adds read them; in accumulation registers each would need a copy).
+# Per-source additions: the matrix-core GEMMs take their results in VGPRs
+# (the VALU reads them; in accumulation registers each would need a copy).
 EXTRA_FLAGS = {
+    "dtl_gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "dtl_mfp.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
 }
 

@@ -944,6 +944,23 @@ int enqueue_forward(dtl_session* s, int T, size_t pos0, const int* pos_dev,
                             s->ln->err, st);
     });
   };
+  // Q8_0 / Q4_0 matrices with the same input in one launch.
+  auto fits_q8 = [&](std::initializer_list<const DevMat*> ms, bool pair) {
+    return q8_mats_fit(ms.begin(), (int)ms.size(), pair);
+  };
+  auto q8_mats = [&](std::initializer_list<const DevMat*> ms, bool pair, const DevAct& in,
+                     std::initializer_list<float*> outs, std::initializer_list<const float*> biases,
+                     std::initializer_list<int> epis, const char* cls) {
+    double bytes = (double)T * (*ms.begin())->cols * (1.0 + 4.0 / 32), macs = 0.0;
+    for (const DevMat* mm : ms) {
+      bytes += (double)mm->rows * mm->cols * weight_bytes_per_elem(mm->type) + (pair ? 2.0 : 4.0) * T * mm->rows;
+      macs += (double)mm->rows * mm->cols * T;
+    }
+    P.timed(st, cls, bytes, macs, [&] {
+      (void)launch_q8_mats(ms.begin(), (int)ms.size(), pair, in, T, outs.begin(), biases.begin(), epis.begin(),
+                           s->ln->err, st);
+    });
+  };
   for (size_t l = 0; l < c.block_count; l++) {
     const Layer& L = m->layers[l];
     const int e_q = L.bq ? EPI_BIAS : EPI_STORE, e_k = L.bk ? EPI_BIAS : EPI_STORE;
@@ -987,9 +1004,13 @@ int enqueue_forward(dtl_session* s, int T, size_t pos0, const int* pos_dev,
       a = rms(L.attn_norm, {});
       f32_mats({&L.wq, &L.wk, &L.wv}, false, a.x, {s->ln->q, s->ln->k, s->ln->v}, {L.bq, L.bk, L.bv},
                {e_q, e_k, e_v}, "gemm_f32_qkv");
+    } else if (T > kGemvMaxT && fits_q8({&L.wq, &L.wk, &L.wv}, false)) {
+      a = rms(L.attn_norm, {&L.wq});
+      q8_mats({&L.wq, &L.wk, &L.wv}, false, a, {s->ln->q, s->ln->k, s->ln->v}, {L.bq, L.bk, L.bv}, {e_q, e_k, e_v},
+              "gemm_q8_qkv");
     } else {
       a = rms(L.attn_norm, {&L.wq, &L.wk, &L.wv});
-      if (L.wq.type == GGML_Q4_K && L.wk.type == GGML_Q4_K && L.wq.w32 && L.wk.w32 && T >= 16 &&
+      if (L.wq.type == GGML_Q4_K && L.wk.type == GGML_Q4_K && L.wq.w32 && L.wk.w32 && T > kGemvMaxT &&
           (L.bq != nullptr) == (L.bk != nullptr)) {
         // wq and wk share the input: one launch over their concatenated rows.
         double bytes = (double)(L.wq.rows + L.wk.rows) * L.wq.cols * weight_bytes_per_elem(GGML_Q4_K) +
@@ -1087,9 +1108,12 @@ int enqueue_forward(dtl_session* s, int T, size_t pos0, const int* pos_dev,
     } else if (fits_f32({&L.gate, &L.up}, true)) {
       a = rms(L.ffn_norm, {});
       f32_mats({&L.gate, &L.up}, true, a.x, {s->ln->ffo}, {}, {}, "gemm_f32_gate_up");
+    } else if (T > kGemvMaxT && fits_q8({&L.gate, &L.up}, true)) {
+      a = rms(L.ffn_norm, {&L.gate});
+      q8_mats({&L.gate, &L.up}, true, a, {s->ln->ffo}, {}, {}, "gemm_q8_gate_up");
     } else {
       a = rms(L.ffn_norm, {&L.gate, &L.up});
-      if (T >= 16 && L.gate.type == GGML_Q4_K && L.up.type == GGML_Q4_K &&
+      if (T > kGemvMaxT && L.gate.type == GGML_Q4_K && L.up.type == GGML_Q4_K &&
           L.gate.rows == L.up.rows && L.gate.cols == L.up.cols) {
         // gate, up and swiglu in one pass: both chains of a row share one wave.
         double bytes = 2.0 * L.gate.rows * L.gate.cols * weight_bytes_per_elem(GGML_Q4_K) +

@@ -185,6 +185,26 @@ bool f32_mats_fit(const DevMat* const* mats, int nm, bool pair);
 bool launch_f32_mats(const DevMat* const* mats, int nm, bool pair, const float* x, int T, float* const* outs,
                      const float* const* biases, const int* epis, int* err, hipStream_t s);
 
+// The same for Q8_0 / Q4_0 matrices on the int8 matrix cores (k_q8_tile,
+// dtl_gemm.hip); w: int8 values in element order.
+struct Q8Mats {
+  const int8_t* w[3];
+  const uint16_t* d16[3];
+  float* out[3];
+  const float* bias[3];
+  int epi[3];
+  int rows[3];
+  int row_end[3];  // prefix sums of rows
+  int total_rows;
+  int nb;
+};
+// Whether launch_q8_mats takes these: Q8_0, or Q4_0 with its int8 copy, the
+// same width, and for the pair the same shape.
+bool q8_mats_fit(const DevMat* const* mats, int nm, bool pair);
+// false (nothing launched) when they do not fit.
+bool launch_q8_mats(const DevMat* const* mats, int nm, bool pair, const DevAct& A, int T, float* const* outs,
+                    const float* const* biases, const int* epis, int* err, hipStream_t s);
+
 // Positions up to which the decode GEMVs (one weight pass per position)
 // replace the chunked-encode GEMMs.
 constexpr int kGemvMaxT = 8;
@@ -281,7 +301,7 @@ void launch_q6k_planes(const DevMat& W, int8_t* planes, hipStream_t s);
 // Fills out (rows * cols bytes) with the int8 values of W's Q4_0 blocks.
 void launch_q4_0_i8(const DevMat& W, int8_t* out, hipStream_t s);
 // Two Q4_K matrices with the same input and column count (wq, wk) in one
-// launch of at least 16 positions, each with its own output, bias and
+// launch of more than kGemvMaxT positions, each with its own output, bias and
 // epilogue; false (nothing launched) when the pair does not qualify.
 bool launch_gemm_cat_q4k(const DevMat& W0, const DevMat& W1, const DevAct& A, int T, float* out0,
                          float* out1, const float* bias0, const float* bias1, int epi, int* err,

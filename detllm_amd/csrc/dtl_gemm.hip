@@ -296,56 +296,6 @@ __global__ void __launch_bounds__(256) k_q6k_tok(DevMat W, const int8_t* __restr
 }
 
 // ---------------------------------------------------------------------------
-// Q8_0: dot_q8_0_q8a (det-quant lib.rs:237-257): exact i32 block sums by
-// dot4, (dw*da)*isum, block-ordered f32 chain per lane.
-template <int R>
-__global__ void __launch_bounds__(256) k_q8_0_tok(DevMat W, const int8_t* __restrict__ qa,
-                                                  const float* __restrict__ da, int T, float* out,
-                                                  const float* bias, int epi, int* err) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int row0 = (blockIdx.x * kWaves + wave) * R;
-  const int t = blockIdx.y * 64 + lane;
-  const bool tok = t < T;
-  const int rows = W.rows, cols = W.cols, nb = W.nb;
-  const int8_t* arow = qa + (size_t)(tok ? t : 0) * cols;
-  const float* drow = da + (size_t)(tok ? t : 0) * nb;
-  float acc[R];
-#pragma unroll
-  for (int r = 0; r < R; r++) acc[r] = 0.0f;
-  for (int b = 0; b < nb; b++) {
-    int4 a0 = ((const int4*)(arow + b * 32))[0];
-    int4 a1 = ((const int4*)(arow + b * 32))[1];
-    float dab = drow[b];
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-      int row = row0 + r < rows ? row0 + r : rows - 1;
-      const int4* wp = (const int4*)((const int8_t*)W.w + (size_t)row * cols + b * 32);
-      int4 w0 = wp[0], w1 = wp[1];
-      int is = 0;
-      is = __builtin_amdgcn_sdot4(w0.x, a0.x, is, false);
-      is = __builtin_amdgcn_sdot4(w0.y, a0.y, is, false);
-      is = __builtin_amdgcn_sdot4(w0.z, a0.z, is, false);
-      is = __builtin_amdgcn_sdot4(w0.w, a0.w, is, false);
-      is = __builtin_amdgcn_sdot4(w1.x, a1.x, is, false);
-      is = __builtin_amdgcn_sdot4(w1.y, a1.y, is, false);
-      is = __builtin_amdgcn_sdot4(w1.z, a1.z, is, false);
-      is = __builtin_amdgcn_sdot4(w1.w, a1.w, is, false);
-      float scale = f16_to_f32(W.d16[(size_t)row * nb + b]) * dab;
-      acc[r] += scale * (float)is;
-    }
-  }
-  if (!tok) return;
-  bool ok = true;
-#pragma unroll
-  for (int r = 0; r < R; r++) {
-    int row = row0 + r;
-    if (row >= rows) continue;
-    ok &= store_epilogue(acc[r], out, (size_t)t * rows + row, bias, row, epi);
-  }
-  if (!ok) flag(err, ERRBIT_NON_FINITE);
-}
-
-// ---------------------------------------------------------------------------
 // Q4_K from an exact f32 copy of the weights (Q4kF32Args, the modes in
 // dtl_device.h; one matrix, or two concatenated), every output one chain of
 // products in element order.  The lanes of a wave are split over positions and rows, and each lane
@@ -576,7 +526,6 @@ void launch_q6k_planes(const DevMat& W, int8_t* planes, hipStream_t s) {
 // K steps in flight per wave in the int8 MFMA GEMMs (slots r0, r1, ...):
 // the Q6_K superblock's operands are four times a Q8_0 block pair's.
 constexpr int kQ6kRing = 2;
-constexpr int kMfmaRing = 4;
 
 template <int NT>
 __global__ void __launch_bounds__(256) k_q6k_mfma(const int8_t* __restrict__ planes,
@@ -738,169 +687,290 @@ __global__ void __launch_bounds__(256) k_q6k_mfma(const int8_t* __restrict__ pla
 // 64 covering blocks 2p and 2p+1, v_mfma_i32_16x16x64_i8 gives block 2p's
 // isum when the A operand's K quarters 2 and 3 are zero and block 2p+1's
 // when quarters 0 and 1 are: both exact in i32.  The f32 part runs on the
-// VALU in the reference's order.  Q4_0 uses the int8 copy of its weights
-// (nibble - 8, element order) built at load.
+// VALU in the reference's order: four instructions per block and output
+// (convert, dw * da, times isum, add), which bound the large launches, the
+// matrix cores taking a quarter of their time.  Q4_0 uses the int8 copy of
+// its weights (nibble - 8, element order) built at load.
 //
 // MFMA operand layout (16x16x64 i8): lane l supplies row / position l % 16
 // and K quarter l / 16 (16 bytes); result register i of lane l is row
-// 4 (l / 16) + i, position l % 16.  A wave covers 16 rows x 16 NT
-// positions; a workgroup 4 / (4 / NT) row tiles x 64 positions.
-template <int NT, bool EVEN>
-__global__ void __launch_bounds__(256) k_q8_mfma(const int8_t* __restrict__ w8,
-                                                 const uint16_t* __restrict__ d16, int rows, int nb,
-                                                 const int8_t* __restrict__ qa,
-                                                 const float* __restrict__ da, int T, float* out,
-                                                 const float* bias, int epi, int* err) {
-  constexpr int PT = 4 / NT;  // position tiles (of 16 NT) per workgroup
-  constexpr int RT = 4 / PT;  // row tiles per workgroup
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+// 4 (l / 16) + i, position l % 16.
+//
+// A wave owns RW x PW tiles of 16 rows x 16 positions (4 RW PW chains a
+// lane), a workgroup WR x WP waves.  Stages of 128 bytes of K (four blocks)
+// of the workgroup's rows and positions, with their scales as f32, pass
+// through LDS, double-buffered, with two further stages in flight in
+// registers; rows are padded to 144 bytes, so sixteen lanes' operand reads
+// fall in distinct banks.  Blocks past the row have zero scales (their terms
+// are +-0, which change no sum).  V4: a row's block count is a multiple of
+// four, so its four scales are one load.  Up to three matrices share a
+// launch over concatenated rows; PAIR alternates the rows of gate and up
+// (tile row i is matrix i % 2, row i / 2) and writes silu(gate) * up.
+//
+// Workgroups are numbered so that the position tiles of one row tile run on
+// one XCD (workgroup n runs on XCD n % 8), whose L2 then serves the weights
+// to all but the first of them.
+namespace {
+// A weight scale (a finite f16) by the hardware's conversion, exact.
+__device__ __forceinline__ float half_to_f32(uint16_t h) { return (float)__builtin_bit_cast(_Float16, h); }
+}  // namespace
+
+template <int RW, int PW, int WR, int WP, bool V4, bool PAIR>
+__global__ void __launch_bounds__(64 * WR * WP) k_q8_tile(Q8Mats M, const int8_t* __restrict__ qa,
+                                                          const float* __restrict__ da, int T, int row_tiles,
+                                                          int pos_tiles, int* err) {
+  constexpr int NT = 64 * WR * WP, TR = 16 * RW * WR, TP = 16 * PW * WP;
+  constexpr int KB = 128, LD = KB + 16;
+  constexpr int NA = (TR * 8 + NT - 1) / NT, NB = (TP * 8 + NT - 1) / NT;  // 16-byte chunks per thread
+  static_assert(TR * 8 % NT == 0 && TR + TP <= NT, "staging slots");
+  constexpr int D = 2;  // stages of loads in flight per thread (four measured no faster)
+  __shared__ __align__(16) int8_t sa[2][TR * LD];
+  __shared__ __align__(16) int8_t sb[2][TP * LD];
+  __shared__ __align__(16) float ss[2][4][TR + TP];  // the rows' scales, then the positions'
+  const int loc = blockIdx.x >> 3;
+  const int rt = loc / pos_tiles * 8 + (blockIdx.x & 7), pt = loc % pos_tiles;
+  if (rt >= row_tiles) return;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wr = wave / WP, wp = wave % WP;
   const int q = lane >> 4, li = lane & 15;
-  const int row0 = (blockIdx.x * RT + wave / PT) * 16;
-  const int p0 = blockIdx.y * 64 + (wave % PT) * 16 * NT;
-  const int cols = nb * 32;
-  const dtl_v4i zero = {0, 0, 0, 0};
-  int arow = row0 + li;
-  arow = arow < rows ? arow : rows - 1;
-  const int8_t* asrc = w8 + (size_t)arow * cols + 16 * q;
-  const int8_t* bsrc[NT];
-  const float* dsrc[NT];
-#pragma unroll
-  for (int j = 0; j < NT; j++) {
-    int pos = p0 + 16 * j + li;
-    pos = pos < T ? pos : T - 1;
-    bsrc[j] = qa + (size_t)pos * cols + 16 * q;
-    dsrc[j] = da + (size_t)pos * nb;
-  }
-  const uint16_t* dwsrc[4];
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    int row = row0 + 4 * q + i;
-    row = row < rows ? row : rows - 1;
-    dwsrc[i] = d16 + (size_t)row * nb;
-  }
-  float sums[NT][4];
-#pragma unroll
-  for (int j = 0; j < NT; j++)
-#pragma unroll
-    for (int i = 0; i < 4; i++) sums[j][i] = 0.0f;
-  // Operands of one block pair; the next pair's are in flight while the
-  // current one is multiplied.  In an odd last pair the second block's
-  // quarters re-read the first block's bytes and are zeroed.
-  // EVEN (an even block count, so every pair is whole and starts at an even
-  // block): the pair's two weight scales of a row are one 32-bit load and
-  // its two activation scales one 64-bit load (each load costs issue time;
-  // a value packed from two loads would be waited for as soon as loaded).
-  struct Ops {
-    dtl_v4i a;
-    dtl_v4i b[NT];
-    uint32_t dw[2][4];  // EVEN: dw[0][i] holds both halves
-    float dav[2][NT];
+  const int nb = M.nb, cols = nb * 32;
+  // The matrix and row of tile row tr (clamped to the last row).
+  auto locate = [&](int tr, int* mat, int* row) -> bool {
+    if (PAIR) {
+      const int r = rt * (TR / 2) + (tr >> 1);
+      *mat = tr & 1;
+      *row = r < M.rows[0] ? r : M.rows[0] - 1;
+      return r < M.rows[0];
+    }
+    const int g = rt * TR + tr;
+    const int gc = g < M.total_rows ? g : M.total_rows - 1;
+    *mat = (gc >= M.row_end[0] ? 1 : 0) + (gc >= M.row_end[1] ? 1 : 0);
+    *row = gc - (*mat == 0 ? 0 : (*mat == 1 ? M.row_end[0] : M.row_end[1]));
+    return g < M.total_rows;
   };
-  auto load = [&](Ops& o, int pr) {
-    const int b0 = 2 * pr;
-    const bool two = b0 + 1 < nb;
-    const int off = b0 * 32 + (two || q < 2 ? 0 : -32);
-    o.a = *(const dtl_v4i*)(asrc + off);
+  // Staging: chunk f = tid + k NT is byte column 16 (f % 8) of row f / 8.
+  const int cc = 16 * (tid & 7);
+  const int8_t* asrc[NA];
+  const int8_t* bsrc[NB];
 #pragma unroll
-    for (int j = 0; j < NT; j++) o.b[j] = *(const dtl_v4i*)(bsrc[j] + off);
-    const int b1 = two ? b0 + 1 : b0;
-    if constexpr (EVEN) {
+  for (int k = 0; k < NA; k++) {
+    int mat, row;
+    (void)locate((tid + k * NT) >> 3, &mat, &row);
+    asrc[k] = pick3(M.w, mat) + (size_t)row * cols;
+  }
 #pragma unroll
-      for (int i = 0; i < 4; i++) o.dw[0][i] = *(const uint32_t*)(dwsrc[i] + b0);
+  for (int k = 0; k < NB; k++) {
+    int p = pt * TP + ((tid + k * NT) >> 3);
+    p = p < T ? p : T - 1;
+    bsrc[k] = qa + (size_t)p * cols;
+  }
+  // Scales: thread t < TR moves tile row t's, TR <= t < TR + TP a position's
+  // (both loads on every thread, clamped: no load under a branch).
+  const bool is_w = tid < TR;
+  const uint16_t* wsc;
+  {
+    int mat, row;
+    (void)locate(is_w ? tid : 0, &mat, &row);
+    wsc = pick3(M.d16, mat) + (size_t)row * nb;
+  }
+  int dp = pt * TP + (is_w ? 0 : tid - TR);
+  dp = dp < T ? dp : T - 1;
+  const float* dsc = da + (size_t)dp * nb;
+  struct Regs {
+    dtl_v4i a[NA], b[NB];
+    uint16_t w[4];
+    float d[4];
+  };
+  auto issue = [&](Regs& r, int s) {
+    const int col = s * KB + cc < cols ? s * KB + cc : 0;
 #pragma unroll
-      for (int j = 0; j < NT; j++) {
-        const float2 d2 = *(const float2*)(dsrc[j] + b0);
-        o.dav[0][j] = d2.x;
-        o.dav[1][j] = d2.y;
-      }
+    for (int k = 0; k < NA; k++) r.a[k] = *(const dtl_v4i*)(asrc[k] + col);
+#pragma unroll
+    for (int k = 0; k < NB; k++) r.b[k] = *(const dtl_v4i*)(bsrc[k] + col);
+    if constexpr (V4) {
+      const int b0 = 4 * s < nb ? 4 * s : 0;
+      const uint2 u = *(const uint2*)(wsc + b0);
+      r.w[0] = (uint16_t)(u.x & 0xffffu);
+      r.w[1] = (uint16_t)(u.x >> 16);
+      r.w[2] = (uint16_t)(u.y & 0xffffu);
+      r.w[3] = (uint16_t)(u.y >> 16);
+      const float4 f = *(const float4*)(dsc + b0);
+      r.d[0] = f.x;
+      r.d[1] = f.y;
+      r.d[2] = f.z;
+      r.d[3] = f.w;
     } else {
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        o.dw[0][i] = dwsrc[i][b0];
-        o.dw[1][i] = dwsrc[i][b1];
-      }
-#pragma unroll
-      for (int j = 0; j < NT; j++) {
-        o.dav[0][j] = dsrc[j][b0];
-        o.dav[1][j] = dsrc[j][b1];
+      for (int k = 0; k < 4; k++) {
+        const int b = 4 * s + k < nb ? 4 * s + k : 0;
+        r.w[k] = wsc[b];
+        r.d[k] = dsc[b];
       }
     }
   };
-  // valid[h]: whether block 2 pr + h exists; a missing block adds +0.0f
-  // terms, which leave the sums' bits unchanged (as in k_q6k_mfma).
-  auto compute = [&](const Ops& o, bool valid0, bool valid1) {
+  auto commit = [&](const Regs& r, int buf, int s) {
 #pragma unroll
-    for (int h = 0; h < 2; h++) {
-      const bool valid = h == 0 ? valid0 : valid1;
-      const dtl_v4i a = (q >> 1) == h ? o.a : zero;
-      float dw[4];
+    for (int k = 0; k < NA; k++) *(dtl_v4i*)(sa[buf] + ((tid + k * NT) >> 3) * LD + cc) = r.a[k];
 #pragma unroll
-      for (int i = 0; i < 4; i++)
-        dw[i] = f16_to_f32((uint16_t)(EVEN ? (h == 0 ? o.dw[0][i] & 0xffffu : o.dw[0][i] >> 16) : o.dw[h][i]));
+    for (int k = 0; k < NB; k++)
+      if (NB * NT == TP * 8 || tid + k * NT < TP * 8) *(dtl_v4i*)(sb[buf] + ((tid + k * NT) >> 3) * LD + cc) = r.b[k];
+    if (TR + TP == NT || tid < TR + TP) {
 #pragma unroll
-      for (int j = 0; j < NT; j++) {
-        const dtl_v4i acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, o.b[j], zero, 0, 0, 0);
+      for (int k = 0; k < 4; k++) {
+        const float v = is_w ? half_to_f32(r.w[k]) : r.d[k];
+        ss[buf][k][tid] = 4 * s + k < nb ? v : 0.0f;
+      }
+    }
+  };
+  float sums[RW][PW][4];
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-          const float dd = dw[i] * o.dav[h][j];
-          const float term = dd * (float)acc[i];
-          sums[j][i] += valid ? term : 0.0f;
+  for (int i = 0; i < RW; i++)
+#pragma unroll
+    for (int j = 0; j < PW; j++)
+#pragma unroll
+      for (int c = 0; c < 4; c++) sums[i][j][c] = 0.0f;
+  const dtl_v4i zero = {0, 0, 0, 0};
+  auto compute = [&](int buf) {
+#pragma unroll
+    for (int pp = 0; pp < 2; pp++) {
+      dtl_v4i a[RW], b[PW];
+#pragma unroll
+      for (int i = 0; i < RW; i++) a[i] = *(const dtl_v4i*)(sa[buf] + ((wr * RW + i) * 16 + li) * LD + 64 * pp + 16 * q);
+#pragma unroll
+      for (int j = 0; j < PW; j++) b[j] = *(const dtl_v4i*)(sb[buf] + ((wp * PW + j) * 16 + li) * LD + 64 * pp + 16 * q);
+      // the blocks' K quarters of the positions, zeros in the others
+      dtl_v4i bm[2][PW];
+      float dv[2][PW];
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int j = 0; j < PW; j++) {
+          bm[h][j] = (q >> 1) == h ? b[j] : zero;
+          dv[h][j] = ss[buf][2 * pp + h][TR + (wp * PW + j) * 16 + li];
+        }
+      // Row tile n % RW of block n / RW: its MFMAs are issued ahead of the
+      // arithmetic on the one before, whose latency they cover.  The empty
+      // asms keep that order (hoisted, a stage's results needed 430
+      // registers).
+      dtl_v4i acc[2][PW];
+#pragma unroll
+      for (int j = 0; j < PW; j++) acc[0][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[0], bm[0][j], zero, 0, 0, 0);
+#pragma unroll
+      for (int n = 0; n < 2 * RW; n++) {
+        const int h = n / RW, i = n % RW;
+        if (n + 1 < 2 * RW) {
+          const int h1 = (n + 1) / RW, i1 = (n + 1) % RW;
+          asm volatile("" : "+v"(a[i1]));
+#pragma unroll
+          for (int j = 0; j < PW; j++)
+            acc[(n + 1) & 1][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[i1], bm[h1][j], zero, 0, 0, 0);
+        }
+        const float4 dw = *(const float4*)&ss[buf][2 * pp + h][(wr * RW + i) * 16 + 4 * q];
+#pragma unroll
+        for (int j = 0; j < PW; j++) {
+          const dtl_v4i r = acc[n & 1][j];
+          sums[i][j][0] += (dw.x * dv[h][j]) * (float)r[0];
+          sums[i][j][1] += (dw.y * dv[h][j]) * (float)r[1];
+          sums[i][j][2] += (dw.z * dv[h][j]) * (float)r[2];
+          sums[i][j][3] += (dw.w * dv[h][j]) * (float)r[3];
+        }
+#pragma unroll
+        for (int j = 0; j < PW; j++)
+          asm volatile("" : "+v"(sums[i][j][0]), "+v"(sums[i][j][1]), "+v"(sums[i][j][2]), "+v"(sums[i][j][3]));
+      }
+    }
+  };
+  const int ns = (nb + 3) / 4;
+  Regs r[D];
+#pragma unroll
+  for (int u = 0; u < D; u++) {
+    issue(r[u], u);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  // The epilogue's operands (the residual, the bias), in flight with the
+  // first stages where the tile leaves registers for them.
+  constexpr bool kPre = !PAIR && RW * PW <= 2;
+  float pre[kPre ? RW : 1][kPre ? PW : 1][4];
+  auto load_pre = [&](int i, int j, float (&p)[4]) {
+    int pos = pt * TP + (wp * PW + j) * 16 + li;
+    pos = pos < T ? pos : T - 1;
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+      int mat, row;
+      (void)locate((wr * RW + i) * 16 + 4 * q + c, &mat, &row);
+      p[c] = epilogue_operand(pick3(M.out, mat), (size_t)pos * pick3(M.rows, mat) + row, pick3(M.bias, mat), row,
+                              pick3(M.epi, mat));
+    }
+  };
+  if constexpr (kPre) {
+#pragma unroll
+    for (int i = 0; i < RW; i++)
+#pragma unroll
+      for (int j = 0; j < PW; j++) load_pre(i, j, pre[i][j]);
+  }
+  commit(r[0], 0, 0);
+  issue(r[0], D);
+  __syncthreads();
+  for (int s0 = 0; s0 < ns; s0 += D) {
+#pragma unroll
+    for (int u = 0; u < D; u++) {
+      if (s0 + u < ns) compute(u & 1);
+      commit(r[(u + 1) % D], (u + 1) & 1, s0 + u + 1);
+      issue(r[(u + 1) % D], s0 + u + 1 + D);
+      __syncthreads();
+    }
+  }
+  bool ok = true;
+  const bool any_operand = M.epi[0] != EPI_STORE || M.epi[1] != EPI_STORE || M.epi[2] != EPI_STORE;
+#pragma unroll
+  for (int i = 0; i < RW; i++)
+#pragma unroll
+    for (int j = 0; j < PW; j++) {
+      const int pos = pt * TP + (wp * PW + j) * 16 + li;
+      const int tr = (wr * RW + i) * 16 + 4 * q;
+      int mat, row;
+      if constexpr (PAIR) {
+#pragma unroll
+        for (int c = 0; c < 4; c += 2) {
+          if (!locate(tr + c, &mat, &row) || pos >= T) continue;
+          const float gv = sums[i][j][c], uv = sums[i][j][c + 1];
+          const float v = silu_det(gv) * uv;
+          ok &= finite(gv) && finite(uv) && finite(v);
+          M.out[0][(size_t)pos * M.rows[0] + row] = v;
+        }
+      } else {
+        float p[4];
+        if constexpr (kPre) {
+#pragma unroll
+          for (int c = 0; c < 4; c++) p[c] = pre[i][j][c];
+        } else {
+          p[0] = p[1] = p[2] = p[3] = 0.0f;
+          if (any_operand) load_pre(i, j, p);
+        }
+        const bool live = locate(tr, &mat, &row) && pos < T;
+        const int R = pick3(M.rows, mat), epi = pick3(M.epi, mat);
+        if (live && row + 3 < R && ((row | R) & 3) == 0) {
+          // four rows of one matrix at a 16-byte aligned place
+          float v[4];
+#pragma unroll
+          for (int c = 0; c < 4; c++) {
+            v[c] = sums[i][j][c];
+            ok &= finite(v[c]);
+            if (epi == EPI_BIAS) v[c] = v[c] + p[c];
+            else if (epi == EPI_RESIDUAL) v[c] = p[c] + v[c];
+            ok &= finite(v[c]);
+          }
+          *(float4*)(pick3(M.out, mat) + (size_t)pos * R + row) = make_float4(v[0], v[1], v[2], v[3]);
+        } else {
+#pragma unroll
+          for (int c = 0; c < 4; c++)
+            if (locate(tr + c, &mat, &row) && pos < T)
+              ok &= store_epilogue_pre(sums[i][j][c], p[c], pick3(M.out, mat),
+                                       (size_t)pos * pick3(M.rows, mat) + row, pick3(M.epi, mat));
         }
       }
     }
-  };
-  // Block pairs in flight, refilled unconditionally as in k_q6k_mfma
-  const int np = (nb + 1) / 2;
-  // (four slots with one position tile per wave, two with more)
-  constexpr int D = NT == 1 ? kMfmaRing : 2;
-  auto last = [&](int i) { return i < np ? i : np - 1; };
-  Ops r0, r1, r2, r3;
-  load(r0, last(0));
-  load(r1, last(1));
-  if (D == 4) {
-    load(r2, last(2));
-    load(r3, last(3));
-  }
-  // the epilogue's operands (clamped positions and rows), in flight with the
-  // first block pairs
-  float pre[NT][4];
-#pragma unroll
-  for (int j = 0; j < NT; j++) {
-    int pos = p0 + 16 * j + li;
-    pos = pos < T ? pos : T - 1;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      int row = row0 + 4 * q + i;
-      row = row < rows ? row : rows - 1;
-      pre[j][i] = epilogue_operand(out, (size_t)pos * rows + row, bias, row, epi);
-    }
-  }
-#define DTL_MFMA_STEP(r, i)                                                                \
-  compute(r, (i) < np, 2 * (i) + 1 < nb);                                                  \
-  __builtin_amdgcn_sched_barrier(0);                                                       \
-  load(r, last((i) + D));                                                                  \
-  __builtin_amdgcn_sched_barrier(0)
-  for (int p0 = 0; p0 < np; p0 += D) {
-    DTL_MFMA_STEP(r0, p0);
-    DTL_MFMA_STEP(r1, p0 + 1);
-    if (D == 4) {
-      DTL_MFMA_STEP(r2, p0 + 2);
-      DTL_MFMA_STEP(r3, p0 + 3);
-    }
-  }
-#undef DTL_MFMA_STEP
-  bool ok = true;
-#pragma unroll
-  for (int j = 0; j < NT; j++) {
-    const int pos = p0 + 16 * j + li;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int row = row0 + 4 * q + i;
-      if (row < rows && pos < T)
-        ok &= store_epilogue_pre(sums[j][i], pre[j][i], out, (size_t)pos * rows + row, epi);
-    }
-  }
   if (!ok) flag(err, ERRBIT_NON_FINITE);
 }
 
@@ -982,21 +1052,84 @@ Q4kF32Args q4k_args(const DevMat& W0, const DevMat* W1, const DevAct& A, int T, 
 }  // namespace
 
 namespace {
-template <bool EVEN>
-void launch_q8_mfma(const int8_t* w8, const DevMat& W, const DevAct& A, int T, float* out, const float* bias,
-                    int epi, int* err, hipStream_t s) {
-  const int py = (T + 63) / 64;
-  if (W.rows >= 8192)
-    launch_kernel((k_q8_mfma<4, EVEN>), dim3((W.rows + 63) / 64, py), dim3(256), 0, s, w8, W.d16, W.rows,
-                  W.nb, A.qa, A.da, T, out, bias, epi, err);
-  else if (W.rows >= 2048)
-    launch_kernel((k_q8_mfma<2, EVEN>), dim3((W.rows + 31) / 32, py), dim3(256), 0, s, w8, W.d16, W.rows,
-                  W.nb, A.qa, A.da, T, out, bias, epi, err);
-  else
-    launch_kernel((k_q8_mfma<1, EVEN>), dim3((W.rows + 15) / 16, py), dim3(256), 0, s, w8, W.d16, W.rows,
-                  W.nb, A.qa, A.da, T, out, bias, epi, err);
+template <int RW, int PW, int WR, int WP, bool V4, bool PAIR>
+void launch_q8_tile(const Q8Mats& M, const DevAct& A, int T, int* err, hipStream_t s) {
+  constexpr int TR = 16 * RW * WR, TP = 16 * PW * WP;
+  const int rows = PAIR ? 2 * M.rows[0] : M.total_rows;
+  const int rt = (rows + TR - 1) / TR, pt = (T + TP - 1) / TP;
+  launch_kernel((k_q8_tile<RW, PW, WR, WP, V4, PAIR>), dim3((rt + 7) / 8 * 8 * pt), dim3(64 * WR * WP), 0, s, M, A.qa,
+                A.da, T, rt, pt, err);
+}
+
+// The largest tile that still gives every CU two workgroups (one for 32 x
+// 64): a larger tile reads LDS less often per product, a smaller one spreads
+// a short launch.  Up to 16 positions one position tile, 64 rows where that
+// fills the chip, else 16.  us per launch, Qwen2.5-0.5B shape, against the
+// kernel without LDS staging that these replace (one to four position tiles
+// a wave, every operand straight from memory): output projection (151936 x
+// 896) 31 / 75 / 132 / 240 / 455 at 9 / 64 / 128 / 256 / 512 positions
+// against 595 (one lane per row) / 157 / 291 / 566 / 1111; gate + up with
+// SwiGLU 49 at 512 against 2 x 49 + 8; wo and down on average 14 at 9, 19 at
+// 512.  Large launches run at about 0.36 of the 424 T multiply-adds/s that
+// four VALU instructions per block and output allow.
+template <bool V4, bool PAIR>
+void launch_q8_tiles(const Q8Mats& M, const DevAct& A, int T, int* err, hipStream_t s) {
+  const int rows = PAIR ? 2 * M.rows[0] : M.total_rows;
+  auto wgs = [&](int tr, int tp) { return (long)((rows + tr - 1) / tr) * ((T + tp - 1) / tp); };
+  if (T <= 16 && wgs(64, 16) >= 256) launch_q8_tile<1, 1, 4, 1, V4, PAIR>(M, A, T, err, s);
+  else if (T <= 16) launch_q8_tile<1, 1, 1, 1, V4, PAIR>(M, A, T, err, s);
+  else if (wgs(128, 64) >= 512) launch_q8_tile<4, 2, 2, 2, V4, PAIR>(M, A, T, err, s);
+  else if (wgs(64, 64) >= 512) launch_q8_tile<2, 2, 2, 2, V4, PAIR>(M, A, T, err, s);
+  else if (T > 32 && wgs(32, 64) >= 256) launch_q8_tile<1, 2, 2, 2, V4, PAIR>(M, A, T, err, s);
+  else launch_q8_tile<1, 1, 2, 2, V4, PAIR>(M, A, T, err, s);
+}
+
+const int8_t* q8_weights(const DevMat& W) {
+  return W.type == kGgmlQ8_0 ? static_cast<const int8_t*>(W.w) : (W.type == kGgmlQ4_0 ? W.i8 : nullptr);
 }
 }  // namespace
+
+bool q8_mats_fit(const DevMat* const* mats, int nm, bool pair) {
+  if (nm < 1 || nm > 3 || (pair && nm != 2)) return false;
+  for (int i = 0; i < nm; i++) {
+    const DevMat& m = *mats[i];
+    if (!q8_weights(m) || m.cols != mats[0]->cols || m.rows <= 0) return false;
+    if (pair && m.rows != mats[0]->rows) return false;
+  }
+  return true;
+}
+
+bool launch_q8_mats(const DevMat* const* mats, int nm, bool pair, const DevAct& A, int T, float* const* outs,
+                    const float* const* biases, const int* epis, int* err, hipStream_t s) {
+  if (T < 1 || !q8_mats_fit(mats, nm, pair)) return false;
+  Q8Mats M{};
+  int acc = 0;
+  for (int i = 0; i < 3; i++) {
+    if (i < nm) {
+      M.w[i] = q8_weights(*mats[i]);
+      M.d16[i] = mats[i]->d16;
+      M.rows[i] = mats[i]->rows;
+      acc += mats[i]->rows;
+      if (!pair) {
+        M.out[i] = outs[i];
+        M.bias[i] = biases[i];
+        M.epi[i] = epis[i];
+      }
+    }
+    M.row_end[i] = acc;
+  }
+  if (pair) M.out[0] = outs[0];
+  M.total_rows = acc;
+  M.nb = mats[0]->nb;
+  if (M.nb % 4 == 0) {
+    if (pair) launch_q8_tiles<true, true>(M, A, T, err, s);
+    else launch_q8_tiles<true, false>(M, A, T, err, s);
+  } else {
+    if (pair) launch_q8_tiles<false, true>(M, A, T, err, s);
+    else launch_q8_tiles<false, false>(M, A, T, err, s);
+  }
+  return true;
+}
 
 bool gemm_tok_supported(const DevMat& W) {
   return W.type == kGgmlQ4K || W.type == kGgmlQ6K || W.type == kGgmlQ8_0 ||
@@ -1026,15 +1159,9 @@ void launch_gemm_tok(const DevMat& W, const DevAct& A, int T, float* out, const 
     }
     return;
   }
-  if ((W.type == kGgmlQ8_0 || (W.type == kGgmlQ4_0 && W.i8)) && T >= 16) {
-    // Q8_0 / Q4_0 on the int8 matrix cores: one workgroup per 64 positions
-    // and 16 (short matrices: every wave its own 16 positions), 32 or 64 rows.
-    const int8_t* w8 = W.type == kGgmlQ8_0 ? (const int8_t*)W.w : W.i8;
-    if (W.nb % 2 == 0)
-      launch_q8_mfma<true>(w8, W, A, T, out, bias, epi, err, s);
-    else
-      launch_q8_mfma<false>(w8, W, A, T, out, bias, epi, err, s);
-    return;
+  {
+    const DevMat* mats[1] = {&W};
+    if (launch_q8_mats(mats, 1, false, A, T, &out, &bias, &epi, err, s)) return;
   }
   int R = rows_per_wave(W.rows);
   dim3 grid((W.rows + kWaves * R - 1) / (kWaves * R), (T + 63) / 64);
@@ -1048,21 +1175,13 @@ void launch_gemm_tok(const DevMat& W, const DevAct& A, int T, float* out, const 
       else
         launch_kernel((k_q4k_tok<1, false>), grid, block, 0, s, W, none, A.af, T, out, nullptr, nullptr, bias, epi, err);
       break;
-    case kGgmlQ6K:
+    default:
       if (R == 4)
         launch_kernel((k_q6k_tok<4>), grid, block, 0, s, W, A.qk, A.dk, T, out, bias, epi, err);
       else if (R == 2)
         launch_kernel((k_q6k_tok<2>), grid, block, 0, s, W, A.qk, A.dk, T, out, bias, epi, err);
       else
         launch_kernel((k_q6k_tok<1>), grid, block, 0, s, W, A.qk, A.dk, T, out, bias, epi, err);
-      break;
-    default:
-      if (R == 4)
-        launch_kernel((k_q8_0_tok<4>), grid, block, 0, s, W, A.qa, A.da, T, out, bias, epi, err);
-      else if (R == 2)
-        launch_kernel((k_q8_0_tok<2>), grid, block, 0, s, W, A.qa, A.da, T, out, bias, epi, err);
-      else
-        launch_kernel((k_q8_0_tok<1>), grid, block, 0, s, W, A.qa, A.da, T, out, bias, epi, err);
       break;
   }
 }
@@ -1086,7 +1205,7 @@ void launch_gemm_pair_swiglu_q4k(const DevMat& G, const DevMat& U, const DevAct&
 bool launch_gemm_cat_q4k(const DevMat& W0, const DevMat& W1, const DevAct& A, int T, float* out0,
                          float* out1, const float* bias0, const float* bias1, int epi, int* err,
                          hipStream_t s) {
-  if (T < 16 || W0.type != kGgmlQ4K || W1.type != kGgmlQ4K || !W0.w32 || !W1.w32 ||
+  if (T <= kGemvMaxT || W0.type != kGgmlQ4K || W1.type != kGgmlQ4K || !W0.w32 || !W1.w32 ||
       W0.cols != W1.cols)
     return false;
   launch_q4k_f32w<MODE_CAT>(q4k_args(W0, &W1, A, T, out0, out1, nullptr, bias0, bias1, epi, err),

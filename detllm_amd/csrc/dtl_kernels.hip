@@ -426,14 +426,14 @@ void launch_gemm(const DevMat& W, const DevAct& A, int T, float* out, const floa
     const DevMat* mats[1] = {&W};
     if (launch_f32_mats(mats, 1, false, A.x, T, &out, &bias, &epi, err, s)) return;
   }
-  // Chunks of positions take the token-parallel kernels (weights decoded once
-  // per wave and shared by up to 64 positions); short batches keep one lane
-  // per (row, position).
-  if (gemm_tok_supported(W) && (T >= 16 || (W.type == kGgmlQ6K && T >= 2))) {
+  // Up to kGemvMaxT positions a decode GEMV per position; beyond, the
+  // kernels that decode the weights once for a tile of positions (Q6_K from
+  // two positions on).
+  if (T <= kGemvMaxT && !(W.type == kGgmlQ6K && T >= 2) && launch_gemv(W, A, T, out, bias, epi, err, s)) return;
+  if (gemm_tok_supported(W)) {
     launch_gemm_tok(W, A, T, out, bias, epi, err, s);
     return;
   }
-  if (T <= kGemvMaxT && launch_gemv(W, A, T, out, bias, epi, err, s)) return;
   dim3 grid((W.rows + 255) / 256, T);
   launch_kernel(k_gemm_rowlane, grid, dim3(256), 0, s, W, A, T, out, bias, epi, err);
 }

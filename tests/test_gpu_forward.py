@@ -92,6 +92,17 @@ def test_f32_model_matches_oracle(name, heads, kv_heads, chunk):
     _compare_with_oracle(synth.build_model(w, layers=2), synth.tokens(w, min(36, 3 * chunk)), chunk)
 
 
+@pytest.mark.parametrize("name,layers,n_tok,chunk", [
+    ("smollm2", 2, 9, 9), ("qwen05", 1, 13, 13), ("tinyllama", 2, 11, 11), ("tinyllama", 1, 15, 15),
+])
+def test_chunks_past_the_decode_gemvs_match_oracle(name, layers, n_tok, chunk):
+    # Nine to fifteen positions: one partial position tile of the chunk GEMMs.
+    from detllm_amd import synth
+
+    w = synth.WORKLOADS[name]
+    _compare_with_oracle(synth.build_model(w, layers=layers), synth.tokens(w, n_tok), chunk)
+
+
 @pytest.mark.parametrize("name,d,heads,kv_heads", [
     ("smollm2", 576, 36, 12),  # 16-wide heads
     ("qwen05", 448, 14, 2),    # 32, split-half RoPE, biases

@@ -110,6 +110,45 @@ def test_f32_rows_bitexact(rows, cols, T):
     assert np.array_equal(out.view(np.uint32), want.view(np.uint32))
 
 
+# (rows, cols, T): every tile of the int8 chunk GEMM (64 x 16, 32 x 32, 32 x
+# 64, 64 x 64 and 128 x 64 rows x positions), partial tiles of each, one block
+# per row, block counts that are and are not multiples of four, an odd and an
+# even number of four-block stages.
+@pytest.mark.parametrize("rows,cols,T", [
+    (1, 32, 9), (70, 896, 13), (64, 128, 16), (129, 576, 16), (33, 160, 17), (65, 64, 32), (37, 256, 33),
+    (40, 896, 70), (2050, 96, 129), (4099, 32, 511), (8200, 64, 512), (8195, 160, 449),
+])
+@pytest.mark.parametrize("ggml_type", [8, 2])
+def test_int8_chunk_gemm_bitexact(ggml_type, rows, cols, T):
+    L = _lib()
+    rng = np.random.default_rng(rows + cols + T)
+    nb = cols // 32
+    if ggml_type == 8:
+        q = rng.integers(-127, 128, (rows, nb, 32)).astype(np.int8)
+        body = q.view(np.uint8)
+    else:
+        body = rng.integers(0, 256, (rows, nb, 16)).astype(np.uint8)
+        q = np.concatenate([body & 15, body >> 4], 2).astype(np.int8) - 8
+    d = rng.normal(0, 0.01, (rows, nb)).astype(np.float16)
+    raw = np.concatenate([d.view(np.uint8).reshape(rows, nb, 2), body], 2)
+    raw = np.ascontiguousarray(raw).reshape(-1)
+    x = rng.normal(0, 2, (T, cols)).astype(np.float32)
+    x[T // 2, :32] = 0.0
+    out = np.empty((T, rows), np.float32)
+    L.check(L.lib.dtl_kernel_gemv(ggml_type, _p(raw, C.c_uint8), rows, cols, _p(x, C.c_float), T, _p(out, C.c_float)),
+            "gemv")
+    da = np.empty((T, nb), np.float32)
+    qa = np.empty((T, nb, 32), np.int8)
+    L.check(L.lib.dtl_kernel_quantize(_p(x, C.c_float), T, cols, _p(da, C.c_float), _p(qa, C.c_int8), None, None),
+            "quantize")
+    # (dw da) isum per block, added in block order
+    want = np.zeros((T, rows), np.float32)
+    for b in range(nb):
+        isum = qa[:, b].astype(np.float32) @ q[:, b].astype(np.float32).T  # exact: below 2^24
+        want = want + (d[None, :, b].astype(np.float32) * da[:, b, None]) * isum
+    assert np.array_equal(out.view(np.uint32), want.view(np.uint32))
+
+
 def test_silu_bitexact():
     rng = np.random.default_rng(1)
     x = np.concatenate([rng.normal(0, 4, 100000), rng.uniform(-100, 100, 50000)]).astype(np.float32)
