@@ -1008,13 +1008,15 @@ int rows_per_wave(int rows) {
 // (k_q4k_mfp) own 16 x 16 (row, position) chains per wave, so a launch of
 // wo / ffn_down or wq + wk at 64 positions has 512-576 waves: with other
 // chunks' launches in flight (the pipelined encode) they and the gate + up
-// pair (2816 waves) run there, the pipelined TinyLlama step taking 98.5 ms
-// against 118.5 with k_q4k_f32m.  A launch alone on the chip
-// (dtl_forward_chunk, the decode-size chunks) keeps one chain per lane of
-// k_q4k_f32m for wo / ffn_down and wq + wk, 8 x 8 lanes, 2 x 2 waves over
-// 16 positions x 16 rows, which fills the chip (chunk-at-a-time step: wo /
-// ffn_down 39.9 ms against 58.1 on the matrix cores, wq + wk 23.1 against
-// 24.9); gate + up takes the matrix cores there too (45.4 against 56.3 ms).
+// pair (2816 waves) run there.  Alone on the chip a launch needs about three
+// waves per CU there; below, one chain per lane of k_q4k_f32m, 8 x 8 lanes,
+// 2 x 2 waves over 16 positions x 16 rows, fills the chip better.  us per
+// launch, k_q4k_f32m against k_q4k_mfp, wo and ffn_down on average / wq + wk
+// of the TinyLlama-1.1B shape: 64 positions (512 / 576 waves) 38 against 51 /
+// 33 against 33; 96 (768 / 864) 51.7 against 51.6 / 42.2 against 41.9; 128
+// 66 against 52 / 50 against 42; 512 229 against 131 / 163 against 98.
+constexpr long kMfpWaves = 768;
+
 template <int PW, int PP, int RP, int WP, int WR, int MODE>
 void launch_q4k_f32m(const Q4kF32Args& a, int rows_total, hipStream_t s) {
   constexpr int RB = WR * RP * 64 / PW, PB = WP * PW * PP;
@@ -1024,8 +1026,9 @@ void launch_q4k_f32m(const Q4kF32Args& a, int rows_total, hipStream_t s) {
 
 template <int MODE>
 void launch_q4k_f32w(const Q4kF32Args& a, bool overlapped, hipStream_t s) {
-  if (MODE == MODE_PAIR || overlapped) return launch_q4k_mfp(a, MODE, s);
   const int rows_total = MODE == MODE_CAT ? a.rows0 + a.rows1 : a.rows0;
+  const long waves = (long)((rows_total + 15) / 16) * ((a.T + 15) / 16);
+  if (MODE == MODE_PAIR || overlapped || waves >= kMfpWaves) return launch_q4k_mfp(a, MODE, s);
   launch_q4k_f32m<8, 1, 1, 2, 2, MODE == MODE_CAT ? MODE_CAT : MODE_SINGLE>(a, rows_total, s);
 }
 
