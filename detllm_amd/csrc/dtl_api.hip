@@ -661,6 +661,15 @@ const char* lm_head_class(int type) {
 // least five queues, else three; DETLLM_LANES (1-4) overrides.
 constexpr int kMaxLanes = 4;
 
+// The pipelined encode takes at least this many positions per chunk, whatever
+// the session's max_chunk, on two lanes of its own: fewer, larger launches
+// fill the chip better than more, smaller ones side by side.  ms per window,
+// four lanes of 64 positions / two of 256 / four of 256 / two of 512: 2048
+// tokens of the TinyLlama-1.1B shape 127 / 88 / 90 / 86, 1000 tokens of the
+// Qwen2.5-0.5B shape (before the int8 GEMM's LDS tiles) 42 / 16 / 16 / 14.
+constexpr size_t kEncodeRows = 256;
+constexpr int kWideLanes = 2;
+
 static int lane_count() {
   if (const char* l = getenv("DETLLM_LANES")) {
     const int n = atoi(l);
@@ -700,6 +709,21 @@ struct Lane {
   // Pinned staging of the decoder entry points (value in, results out), so
   // that their copies are plain DMA rather than staged pageable copies.
   uint64_t* h_io = nullptr;
+
+  // Drains the stream and frees everything but the device buffers (the
+  // arena's), leaving an empty lane.
+  void release() {
+    if (stream) {
+      (void)hipStreamSynchronize(stream);
+      (void)hipStreamDestroy(stream);
+    }
+    for (hipEvent_t e : kv_ready)
+      if (e) (void)hipEventDestroy(e);
+    for (void* p : {(void*)h_tokens, (void*)h_rows, (void*)h_sym, (void*)h_freq, (void*)h_cum, (void*)h_total,
+                    (void*)h_err, (void*)h_io})
+      if (p) (void)hipHostFree(p);
+    *this = Lane();
+  }
 };
 
 // Grows a lane's pinned symbol staging to n symbols (the lane must be idle).
@@ -726,6 +750,12 @@ struct dtl_session {
   float *rope_cos = nullptr, *rope_sin = nullptr, *kc = nullptr, *vc = nullptr;
   Lane lanes[kMaxLanes];
   int nlanes = 1;        // lanes set up (the rest stay empty)
+  // Lanes of kEncodeRows positions for the pipelined encode of sessions with
+  // a smaller max_chunk, set up by its first call with more tokens than that.
+  Arena wide_arena;
+  Lane wide[kWideLanes];
+  size_t wide_rows = 0;  // positions per chunk there (0: not set up)
+  bool wide_failed = false;  // no memory for them: the session's own lanes serve
   Lane* ln = &lanes[0];  // the lane the launches below go to
   // Captured single-position forwards (see forward_device), on lane 0:
   // [0] for rows up to attention_fused_max_len() keys, [1] for the whole
@@ -738,22 +768,60 @@ struct dtl_session {
   int* pos_host = nullptr;  // pinned staging for it
   Profiler prof;
   ~dtl_session() {
-    for (Lane& L : lanes) {
-      if (L.stream) {
-        (void)hipStreamSynchronize(L.stream);
-        (void)hipStreamDestroy(L.stream);
-      }
-      for (hipEvent_t e : L.kv_ready)
-        if (e) (void)hipEventDestroy(e);
-      for (void* p : {(void*)L.h_tokens, (void*)L.h_rows, (void*)L.h_sym, (void*)L.h_freq,
-                      (void*)L.h_cum, (void*)L.h_total, (void*)L.h_err, (void*)L.h_io})
-        if (p) (void)hipHostFree(p);
-    }
+    for (Lane& L : lanes) L.release();
+    for (Lane& L : wide) L.release();
     for (hipGraphExec_t g : graph)
       if (g) (void)hipGraphExecDestroy(g);
     if (pos_host) (void)hipHostFree(pos_host);
   }
 };
+
+// Sets up a lane for chunks of up to C positions: its stream, its events, its
+// device buffers (owned by A) and its pinned staging.
+static int lane_init(dtl_session* s, Arena& A, Lane& L, size_t C) {
+  const dtl_model* m = s->m;
+  const HostConfig& c = m->c;
+  const size_t hd = m->head_dim;
+  int st;
+  HIP_TRY(hipStreamCreateWithFlags(&L.stream, hipStreamNonBlocking));
+#define ALLOC(ptr, n) \
+  if ((st = A.alloc(&L.ptr, (n)))) return st;
+  ALLOC(x, C * c.d);
+  ALLOC(h, C * c.d);
+  ALLOC(q, C * c.heads * hd);
+  ALLOC(k, C * c.kv_heads * hd);
+  ALLOC(v, C * c.kv_heads * hd);
+  ALLOC(attn, C * c.heads * hd);
+  ALLOC(g, C * c.ff);
+  ALLOC(u, C * c.ff);
+  ALLOC(ffo, C * c.ff);
+  ALLOC(logits, C * m->vocab);
+  ALLOC(scores, C * c.heads * s->n_ctx);
+  ALLOC(qa, C * s->max_in);
+  ALLOC(qk, C * s->max_in);
+  ALLOC(af, C * s->max_in);
+  ALLOC(da, C * (s->max_in / 32 + 1));
+  ALLOC(dk, C * (s->max_in / 256 + 1));
+  ALLOC(tokens, C);
+  ALLOC(err, 1);
+  ALLOC(c_sym, C);
+  ALLOC(c_freq, C);
+  ALLOC(c_cum, C);
+  ALLOC(c_total, C);
+  ALLOC(c_values, C);
+  ALLOC(c_pack, 8);
+  ALLOC(c_freq_tab, m->vocab + 256);
+  ALLOC(c_cum_tab, m->vocab + 256);
+  ALLOC(c_scratch, cdf_scratch_bytes((int)C, (int)m->vocab));
+  ALLOC(c_rows, C);
+#undef ALLOC
+  L.kv_ready.assign(c.block_count, nullptr);
+  for (hipEvent_t& e : L.kv_ready) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  HIP_TRY(hipHostMalloc((void**)&L.h_tokens, C * 4, hipHostMallocDefault));
+  HIP_TRY(hipHostMalloc((void**)&L.h_err, sizeof(int), hipHostMallocDefault));
+  HIP_TRY(hipHostMalloc((void**)&L.h_io, 8 * sizeof(uint64_t), hipHostMallocDefault));
+  return lane_reserve(L, C);
+}
 
 namespace {
 
@@ -762,6 +830,23 @@ size_t max_input_width(const dtl_model* m) {
   if (m->c.ff > w) w = m->c.ff;
   if (m->c.heads * m->head_dim > w) w = m->c.heads * m->head_dim;
   return w;
+}
+
+// Sets up the wide lanes; false when there is no memory for them.
+bool ensure_wide(dtl_session* s) {
+  if (s->wide_rows) return true;
+  if (s->wide_failed) return false;
+  const size_t rows = kEncodeRows < s->n_ctx ? kEncodeRows : s->n_ctx;
+  for (Lane& L : s->wide)
+    if (lane_init(s, s->wide_arena, L, rows) != DTL_OK) {
+      (void)hipGetLastError();
+      for (Lane& W : s->wide) W.release();
+      s->wide_arena.release();
+      s->wide_failed = true;
+      return false;
+    }
+  s->wide_rows = rows;
+  return true;
 }
 
 int read_err(dtl_session* s, int* bits) {
@@ -1434,44 +1519,7 @@ int dtl_session_new(const dtl_model* m, size_t n_ctx, size_t max_chunk, dtl_sess
   s->nlanes = lane_count();
   for (int li = 0; li < s->nlanes; li++) {
     Lane& L = s->lanes[li];
-    HIP_TRY(hipStreamCreateWithFlags(&L.stream, hipStreamNonBlocking));
-#define ALLOC(ptr, n) \
-  if ((st = A.alloc(&L.ptr, (n)))) return st;
-    ALLOC(x, C * c.d);
-    ALLOC(h, C * c.d);
-    ALLOC(q, C * c.heads * hd);
-    ALLOC(k, C * c.kv_heads * hd);
-    ALLOC(v, C * c.kv_heads * hd);
-    ALLOC(attn, C * c.heads * hd);
-    ALLOC(g, C * c.ff);
-    ALLOC(u, C * c.ff);
-    ALLOC(ffo, C * c.ff);
-    ALLOC(logits, C * m->vocab);
-    ALLOC(scores, C * c.heads * n_ctx);
-    ALLOC(qa, C * s->max_in);
-    ALLOC(qk, C * s->max_in);
-    ALLOC(af, C * s->max_in);
-    ALLOC(da, C * (s->max_in / 32 + 1));
-    ALLOC(dk, C * (s->max_in / 256 + 1));
-    ALLOC(tokens, C);
-    ALLOC(err, 1);
-    ALLOC(c_sym, C);
-    ALLOC(c_freq, C);
-    ALLOC(c_cum, C);
-    ALLOC(c_total, C);
-    ALLOC(c_values, C);
-    ALLOC(c_pack, 8);
-    ALLOC(c_freq_tab, m->vocab + 256);
-    ALLOC(c_cum_tab, m->vocab + 256);
-    ALLOC(c_scratch, cdf_scratch_bytes((int)C, (int)m->vocab));
-    ALLOC(c_rows, C);
-#undef ALLOC
-    L.kv_ready.assign(c.block_count, nullptr);
-    for (hipEvent_t& e : L.kv_ready) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    HIP_TRY(hipHostMalloc((void**)&L.h_tokens, C * 4, hipHostMallocDefault));
-    HIP_TRY(hipHostMalloc((void**)&L.h_err, sizeof(int), hipHostMallocDefault));
-    HIP_TRY(hipHostMalloc((void**)&L.h_io, 8 * sizeof(uint64_t), hipHostMallocDefault));
-    if ((st = lane_reserve(L, C))) return st;
+    if ((st = lane_init(s.get(), A, L, C))) return st;
   }
   HIP_TRY(hipHostMalloc((void**)&s->pos_host, sizeof(int), hipHostMallocDefault));
   HIP_TRY(hipMemsetAsync(s->kc, 0, kv * 4, s->ln->stream));
@@ -1634,7 +1682,7 @@ int dtl_forward_ranges(dtl_session* s, const uint32_t* tokens, size_t n, size_t 
   if (!s || !tokens || (n_sym && (!rows || !symbols || !cum || !freq || !total)))
     return DTL_ERR_INVALID_ARGUMENT;
   const dtl_model* m = s->m;
-  const size_t V = m->vocab, C = s->max_chunk;
+  const size_t V = m->vocab;
   if (n == 0 || pos0 + n > s->n_ctx) return DTL_ERR_SHAPE;
   if (V + tail > kMaxSymbols) return DTL_ERR_CDF_TOO_MANY_SYMBOLS;
   for (size_t i = 0; i < n; i++)
@@ -1644,24 +1692,31 @@ int dtl_forward_ranges(dtl_session* s, const uint32_t* tokens, size_t n, size_t 
     if (symbols[i] >= V + tail) return DTL_ERR_CDF_SYMBOL_OUT_OF_RANGE;
   }
   HIP_TRY(hipSetDevice(m->device));
-  // Back on lane 0 with both lanes drained however this returns.
+  const bool wide = n > s->max_chunk && s->max_chunk < kEncodeRows && ensure_wide(s);
+  Lane* const lanes = wide ? s->wide : s->lanes;
+  const int nl = wide ? std::min(kWideLanes, s->nlanes) : s->nlanes;
+  const size_t C = wide ? s->wide_rows : s->max_chunk;  // positions (and symbols per CDF launch) of a lane
+  // Back on lane 0 with every lane drained however this returns.
   struct Restore {
     dtl_session* s;
+    Lane* lanes;
+    int nl;
     ~Restore() {
-      for (int li = 0; li < s->nlanes; li++) (void)hipStreamSynchronize(s->lanes[li].stream);
+      for (int li = 0; li < nl; li++) (void)hipStreamSynchronize(lanes[li].stream);
       s->ln = &s->lanes[0];
       s->overlapped = false;
     }
-  } restore{s};
-  s->overlapped = s->nlanes > 1;
+  } restore{s, lanes, nl};
+  // (one chunk has the chip to itself)
+  s->overlapped = nl > 1 && n > C;
   for (Lane& L : s->lanes) {
     L.rows_valid = 0;
     L.cdf_ready_row = SIZE_MAX;
   }
-  const int nl = s->nlanes;
   size_t first[kMaxLanes] = {}, count[kMaxLanes] = {};  // symbols of each lane's chunk
+  static_assert(kWideLanes <= kMaxLanes, "lane counters");
   auto collect = [&](int li) -> int {
-    Lane& L = s->lanes[li];
+    Lane& L = lanes[li];
     HIP_TRY(hipStreamSynchronize(L.stream));
     if (*L.h_err & ERRBIT_NON_FINITE) return DTL_ERR_NON_FINITE;
     if (int st = cdf_status(*L.h_err)) return st;
@@ -1679,19 +1734,19 @@ int dtl_forward_ranges(dtl_session* s, const uint32_t* tokens, size_t n, size_t 
     const int li = (int)(c % nl);
     if (c >= (size_t)nl)
       if (int st = collect(li)) return st;
-    Lane& L = s->lanes[li];
+    Lane& L = lanes[li];
     s->ln = &L;
     const size_t p0 = c * C, T = std::min(C, n - p0);
     std::memcpy(L.h_tokens, tokens + p0, T * sizeof(uint32_t));
     HIP_TRY(hipMemcpyAsync(L.tokens, L.h_tokens, T * 4, hipMemcpyHostToDevice, L.stream));
-    const Lane* prev = c ? &s->lanes[(c - 1) % nl] : nullptr;
+    const Lane* prev = c ? &lanes[(c - 1) % nl] : nullptr;
     int rc = enqueue_forward(s, (int)T, pos0 + p0, nullptr, prev, true);
     if (rc) return rc;
     const size_t k0 = k;
     while (k < n_sym && rows[k] < p0 + T) k++;
     // Several symbols may share a row (byte escapes), so a chunk can code
     // more symbols than it has rows: the host staging grows to fit, the
-    // device staging and CDF scratch take max_chunk symbols per launch.
+    // device staging and CDF scratch take C symbols per launch.
     const size_t ms = k - k0;
     if (int st = lane_reserve(L, ms)) return st;
     for (size_t i = 0; i < ms; i++) {

@@ -96,6 +96,43 @@ def test_forward_ranges_equals_chunk_at_a_time(monkeypatch, name, layers, n, chu
         assert [(int(cum[i]), int(freq[i]), int(total[i])) for i in pick] == ref
 
 
+@pytest.mark.parametrize("name,n,chunk", [
+    ("tinyllama", 515, 64),   # two lanes of 256 positions, a last chunk of three
+    ("smollm2", 1030, 1),     # reused lanes, from a single-position session
+    ("smollm2", 700, 300),    # the session's own lanes (max_chunk past 256)
+    ("smollm2", 257, 255),
+])
+def test_forward_ranges_over_several_wide_chunks(name, n, chunk):
+    from detllm_amd import synth
+    from detllm_amd.model import F32Llama
+
+    w = dataclasses.replace(synth.WORKLOADS[name], vocab=1001)
+    m = F32Llama.from_gguf(synth.build_model(w, layers=2))
+    toks = synth.tokens(w, n)
+    rows, syms = _rows_symbols(n, m.vocab, 256, seed=n)
+    with m.forward_workspace(n, 128) as s:
+        want = [], [], []
+        for p in range(0, n, 128):
+            T = min(128, n - p)
+            s.forward_chunk(toks[p:p + T], p)
+            sel = (rows >= p) & (rows < p + T)
+            if sel.any():
+                for dst, src in zip(want, s.symbol_ranges_rows(rows[sel] - p, syms[sel], 256)):
+                    dst.append(src)
+    with m.forward_workspace(n, chunk) as s:
+        for _ in range(3):
+            for got, ref in zip(s.forward_ranges(toks, 0, rows, syms, 256), want):
+                assert np.array_equal(got, np.concatenate(ref))
+            # the session's own lanes afterwards, on the cache the wide lanes wrote
+            s.forward_chunk(toks[n - 1:], n - 1)
+            cum, freq, total = s.symbol_ranges([7], 0, 256)
+            with m.forward_workspace(n, 64) as t:
+                for p in range(0, n, 64):
+                    t.forward_chunk(toks[p:min(n, p + 64)], p)
+                last = t.symbol_ranges([7], (n - 1) % 64, 256)
+            assert (cum[0], freq[0], total[0]) == (last[0][0], last[1][0], last[2][0])
+
+
 def test_forward_ranges_errors():
     from detllm_amd import synth
     from detllm_amd._lib import DetllmError
