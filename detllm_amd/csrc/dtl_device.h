@@ -349,6 +349,11 @@ void launch_attention(const float* q, const float* kc, const float* vc, int laye
                       int H, int KV, int hd, int n_ctx, float scale, float* scores, float* out,
                       int* err, hipStream_t s, int8_t* qa = nullptr, float* da = nullptr,
                       float* af = nullptr);
+// Chunk attention in three launches (scores, softmax, P.V; dtl_mfp.hip) for
+// the head widths it is built for; false (nothing launched) for others and
+// for rows past its softmax's LDS.
+bool launch_attention_mfp(const float* q, const float* kc, const float* vc, int layer, int T, int pos0, int H, int KV,
+                          int hd, int n_ctx, float scale, float* scores, float* out, int* err, hipStream_t s);
 void launch_swiglu(const float* g, const float* u, int count, float* out, int* err, hipStream_t s);
 void launch_rope_table(float base, int rope_dim, int positions, float* cos_out, float* sin_out,
                        int* err, hipStream_t s);

@@ -1936,6 +1936,7 @@ void launch_attention(const float* q, const float* kc, const float* vc, int laye
       return;
     }
   }
+  if (launch_attention_mfp(q, kc, vc, layer, T, pos0, H, KV, hd, n_ctx, scale, scores, out, err, s)) return;
   size_t smem = attention_grp_smem(H, KV, hd, n_ctx);
   if (G <= 16 && hd <= 256 && smem <= 150 * 1024) {
     static bool attr_set = false;

@@ -375,6 +375,310 @@ void launch_f32_mfp(const F32Mats& M, bool pair, const float* x, int T, int* err
   else launch_kernel(k_f32_mfp<false>, grid, dim3(512), 0, s, M, x, T, err);
 }
 
+// ---------------------------------------------------------------------------
+// Chunk attention in three launches: the scores and the P.V sums as products
+// on the matrix cores, the softmax between them through the score rows in
+// memory.  A KV group's query rows (position t, head h) are numbered r = t G +
+// h % G, so a tile of rows shares the group's keys and has rows of nearly the
+// same length.  Every value is formed as in k_attention (dtl_kernels.hip):
+// scores in dot_f32_ref's order, then * scale; max, clamped exps, the eight Z
+// chains, divisions; out[d] += p_j * v_j[d] with j ascending (lib.rs:2319-2420).
+//
+// Bound by P.V's serial sums when the rows are few (a wave adds 16 keys in
+// about 400 cycles), by the adds of both products when they are many.  128-wide
+// heads, 8 query / 2 key heads, us per layer at 1000 keys and 5 / 16 / 64 /
+// 128 / 512 positions: 37 / 37 / 44 / 51 / 106, against 344 to 350 up to 64
+// positions of the kernel these widths ran before (one workgroup per KV group
+// and position, K and V through one LDS tile).
+
+// Scores of 32 query rows x 32 keys, HD contracted: the wave pair and chain
+// split of k_f32_mfp, all of HD staged at once.
+template <int HD>
+__global__ void __launch_bounds__(512) k_attn_qk_mfp(const float* __restrict__ q, const float* __restrict__ kc,
+                                                     int layer, int T, int pos0, int H, int KV, int n_ctx,
+                                                     float scale, float* __restrict__ scores, int* err) {
+  constexpr int KP = (HD + 31) / 32 * 32, LD = KP + 4, F4 = KP / 4;
+  __shared__ __align__(16) float sq[32][LD];
+  __shared__ __align__(16) float sk[32][LD];
+  __shared__ __align__(16) float halves[4][64][4];
+  const int G = H / KV, rows = T * G;
+  const int g = blockIdx.z, r0 = blockIdx.x * 32, j0 = blockIdx.y * 32;
+  const int rlast = (r0 + 31 < rows ? r0 + 31 : rows - 1);
+  if (j0 > pos0 + rlast / G) return;  // no row of the tile sees these keys
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int h = wave & 1, wp = (wave >> 1) & 1, wr = wave >> 2;
+  const int l16 = lane & 15, qd = lane >> 4;
+  const float* keys = kc + ((size_t)layer * KV + g) * n_ctx * HD;
+  const int jmax = pos0 + T - 1;
+  for (int f = tid; f < 32 * F4; f += 512) {
+    const int i = f / F4, c = 4 * (f % F4);
+    const int r = r0 + i < rows ? r0 + i : rows - 1, j = j0 + i < jmax ? j0 + i : jmax;
+    float4 a = make_float4(0.0f, 0.0f, 0.0f, 0.0f), b = a;
+    if (HD == KP || c < HD) {
+      a = *reinterpret_cast<const float4*>(q + ((size_t)(r / G) * H + g * G + r % G) * HD + c);
+      b = *reinterpret_cast<const float4*>(keys + (size_t)j * HD + c);
+    }
+    *reinterpret_cast<float4*>(&sq[i][c]) = a;
+    *reinterpret_cast<float4*>(&sk[i][c]) = b;
+  }
+  __syncthreads();
+  dtl_v16f zero;
+#pragma unroll
+  for (int i = 0; i < 16; i++) zero[i] = 0.0f;
+  float acc[4][4];
+#pragma unroll
+  for (int m = 0; m < 4; m++)
+#pragma unroll
+    for (int c = 0; c < 4; c++) acc[m][c] = 0.0f;
+  // MFMA rows are keys (a lane's four results are consecutive keys of one
+  // query row), columns query rows
+  const float* ap = &sk[wr * 16 + l16][8 * qd + 4 * h];
+  const float* bp = &sq[wp * 16 + l16][8 * qd + 4 * h];
+#pragma unroll
+  for (int k0 = 0; k0 < KP; k0 += 32) {
+    dtl_v4f a4 = *(const dtl_v4f*)(ap + k0);
+    dtl_v4f b4 = *(const dtl_v4f*)(bp + k0);
+    asm volatile("" : "+v"(a4), "+v"(b4));
+    dtl_v16f d[4];
+#pragma unroll
+    for (int m = 0; m < 4; m++) d[m] = __builtin_amdgcn_mfma_f32_16x16x1f32(a4[m], b4[m], zero, 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int b = 0; b < 4; b++)
+#pragma unroll
+      for (int m = 0; m < 4; m++)
+#pragma unroll
+        for (int c = 0; c < 4; c++) acc[m][c] += d[m][4 * b + c];
+    asm volatile("" : "+v"(acc[0][0]), "+v"(acc[0][1]), "+v"(acc[0][2]), "+v"(acc[0][3]), "+v"(acc[1][0]),
+                 "+v"(acc[1][1]), "+v"(acc[1][2]), "+v"(acc[1][3]));
+    asm volatile("" : "+v"(acc[2][0]), "+v"(acc[2][1]), "+v"(acc[2][2]), "+v"(acc[2][3]), "+v"(acc[3][0]),
+                 "+v"(acc[3][1]), "+v"(acc[3][2]), "+v"(acc[3][3]));
+  }
+  float half[4];
+#pragma unroll
+  for (int c = 0; c < 4; c++) half[c] = (acc[0][c] + acc[1][c]) + (acc[2][c] + acc[3][c]);
+  if (h == 1) *reinterpret_cast<float4*>(halves[wave >> 1][lane]) = make_float4(half[0], half[1], half[2], half[3]);
+  __syncthreads();
+  if (h == 1) return;
+  const float4 o4 = *reinterpret_cast<const float4*>(halves[wave >> 1][lane]);
+  const int r = r0 + wp * 16 + l16, j = j0 + wr * 16 + 4 * qd;
+  if (r >= rows) return;
+  const int pos = pos0 + r / G;
+  float* srow = scores + ((size_t)(r / G) * H + g * G + r % G) * n_ctx;
+  const float s4[4] = {(half[0] + o4.x) * scale, (half[1] + o4.y) * scale, (half[2] + o4.z) * scale,
+                       (half[3] + o4.w) * scale};
+  bool ok = true;
+#pragma unroll
+  for (int c = 0; c < 4; c++)
+    if (j + c <= pos) {
+      ok &= finite(s4[c]);
+      srow[j + c] = s4[c];
+    }
+  if (!ok && pos > 0) flag(err, ERRBIT_NON_FINITE);  // a single score is never formed
+}
+
+// softmax_in_place (lib.rs:2361-2388) of one score row, in place; the row's
+// places up to the chunk's last position are set to zero, so that a tile of
+// rows can be summed over one range.  LDS: the row, and its exps chain-major
+// (element j at chain j % 8, slot j / 8).
+__host__ __device__ inline int softmax_zs(int maxlen) { return (((maxlen + 7) / 8 + 3) & ~3) + 4; }
+
+__global__ void __launch_bounds__(256) k_attn_softmax(float* scores, int T, int pos0, int H, int n_ctx, int* err) {
+  extern __shared__ __align__(16) float lds[];
+  __shared__ float red[4];
+  __shared__ float zc[8];
+  const int h = blockIdx.x, t = blockIdx.y, tid = threadIdx.x;
+  const int len = pos0 + t + 1, end = pos0 + T;
+  const int zs = softmax_zs(end);
+  float* zcm = lds;             // [8][zs]
+  float* row = lds + 8 * zs;    // [len]
+  float* srow = scores + ((size_t)t * H + h) * n_ctx;
+  for (int j = len + tid; j < end; j += 256) srow[j] = 0.0f;
+  if (len == 1) {
+    if (tid == 0) srow[0] = 1.0f;
+    return;
+  }
+  float mx = -__builtin_huge_valf();
+  for (int j0 = tid; j0 < len; j0 += 1024) {
+    float v[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) v[k] = srow[j0 + 256 * k < len ? j0 + 256 * k : len - 1];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      if (j0 + 256 * k < len) row[j0 + 256 * k] = v[k];
+      mx = fmaxf(mx, v[k]);
+    }
+  }
+  mx = wave_fmax(mx);
+  if ((tid & 63) == 0) red[tid >> 6] = mx;
+  __syncthreads();
+  mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  const int n8 = (len + 7) & ~7;
+#pragma unroll 4
+  for (int j = tid; j < n8; j += 256) {
+    // padded to the longest chain with +0.0, which no sum of exps changes
+    const float e = j < len ? exp_clamped(row[j < len ? j : 0] - mx) : 0.0f;
+    if (j < len) row[j] = e;
+    zcm[(j & 7) * zs + (j >> 3)] = e;
+  }
+  __syncthreads();
+  if (tid < 128) {
+    const float z = chain_group_lds<16>(0.0f, zcm + (tid >> 4) * zs, n8 / 8);
+    if ((tid & 15) == 0) zc[tid >> 4] = z;
+  }
+  __syncthreads();
+  const float z = finish_8lane(zc);
+  bool ok = finite(z) && z != 0.0f;
+#pragma unroll 4
+  for (int j = tid; j < len; j += 256) {
+    const float p = row[j] / z;
+    ok &= finite(p);
+    srow[j] = p;
+  }
+  if (!ok) flag(err, ERRBIT_NON_FINITE);
+}
+
+// out[r][d] = sum over j of p_r[j] v_j[d], one chain per output, j ascending
+// (the pattern of k_q4k_mfp): MFMA rows are sixteen dimensions, columns
+// sixteen query rows, the wave's 16 keys per group the four MFMAs' K.  A
+// workgroup has a wave per (sixteen dimensions, row tile) of RT row tiles and
+// stages 64 keys of its rows' probabilities and of V, double-buffered.
+// Keys past a row's own position have probability +0.0 (products +-0, which
+// change no sum).
+template <int HD>
+constexpr int pv_row_tiles() { return HD <= 64 ? 2 : 1; }
+
+template <int HD>
+__global__ void __launch_bounds__(HD / 16 * pv_row_tiles<HD>() * 64) k_attn_pv_mfp(
+    const float* __restrict__ scores, const float* __restrict__ vc, int layer, int T, int pos0, int H, int KV,
+    int n_ctx, float* __restrict__ out, int* err) {
+  constexpr int DT = HD / 16, RT = pv_row_tiles<HD>(), NT = 64 * DT * RT, SL = 64;
+  constexpr int LDV = HD + 4, LDP = SL + 4;
+  constexpr int NV = SL * HD / 4 / NT, NP = (16 * RT * SL + NT - 1) / NT;  // staging slots per thread
+  static_assert(SL * HD / 4 % NT == 0, "whole staging rounds");
+  __shared__ __align__(16) float sv[2][SL][LDV];
+  __shared__ __align__(16) float sp[2][16 * RT][LDP];
+  const int G = H / KV, rows = T * G;
+  const int g = blockIdx.y, r0 = blockIdx.x * 16 * RT;
+  const int rlast = r0 + 16 * RT - 1 < rows ? r0 + 16 * RT - 1 : rows - 1;
+  const int end = pos0 + rlast / G + 1;  // keys the tile's longest row sees
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int dt = wave % DT, rt = wave / DT;
+  const int l16 = lane & 15, qd = lane >> 4;
+  const float* vals = vc + ((size_t)layer * KV + g) * n_ctx * HD;
+  const float* prow[NP];
+#pragma unroll
+  for (int k = 0; k < NP; k++) {
+    const int r = r0 + (tid + k * NT) / SL, rc = r < rows ? r : rows - 1;
+    prow[k] = scores + ((size_t)(rc / G) * H + g * G + rc % G) * n_ctx;
+  }
+  dtl_v4f v[NV];
+  float p[NP];
+  auto issue = [&](int k0) {
+#pragma unroll
+    for (int k = 0; k < NV; k++) {
+      const int f = tid + k * NT, j = k0 + f / (HD / 4);
+      v[k] = *reinterpret_cast<const dtl_v4f*>(vals + (size_t)(j < end ? j : 0) * HD + 4 * (f % (HD / 4)));
+    }
+#pragma unroll
+    for (int k = 0; k < NP; k++) {
+      const int j = k0 + (tid + k * NT) % SL;
+      p[k] = prow[k][j < end ? j : 0];
+    }
+  };
+  auto commit = [&](int b, int k0) {
+#pragma unroll
+    for (int k = 0; k < NV; k++) {
+      const int f = tid + k * NT;
+      *reinterpret_cast<dtl_v4f*>(&sv[b][f / (HD / 4)][4 * (f % (HD / 4))]) = v[k];
+    }
+#pragma unroll
+    for (int k = 0; k < NP; k++) {
+      const int f = tid + k * NT;
+      if (16 * RT * SL % NT == 0 || f < 16 * RT * SL) sp[b][f / SL][f % SL] = k0 + f % SL < end ? p[k] : 0.0f;
+    }
+  };
+  dtl_v16f zero;
+#pragma unroll
+  for (int i = 0; i < 16; i++) zero[i] = 0.0f;
+  float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  issue(0);
+  commit(0, 0);
+  __syncthreads();
+  int buf = 0;
+  for (int k0 = 0; k0 < end; k0 += SL) {
+    issue(k0 + SL);  // unconditional: past the end row 0, not summed
+    const float* ap = &sv[buf][4 * qd][dt * 16 + l16];
+    const float* bp = &sp[buf][rt * 16 + l16][4 * qd];
+#pragma unroll
+    for (int e = 0; e < SL; e += 16) {
+      dtl_v4f a4 = {ap[e * LDV], ap[(e + 1) * LDV], ap[(e + 2) * LDV], ap[(e + 3) * LDV]};
+      dtl_v4f b4 = *(const dtl_v4f*)(bp + e);
+      asm volatile("" : "+v"(a4), "+v"(b4));
+      dtl_v16f d[4];
+#pragma unroll
+      for (int m = 0; m < 4; m++) d[m] = __builtin_amdgcn_mfma_f32_16x16x1f32(a4[m], b4[m], zero, 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int b = 0; b < 4; b++)
+#pragma unroll
+        for (int m = 0; m < 4; m++)
+#pragma unroll
+          for (int c = 0; c < 4; c++) acc[c] += d[m][4 * b + c];
+      asm volatile("" : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]));
+    }
+    commit(buf ^ 1, k0 + SL);
+    __syncthreads();
+    buf ^= 1;
+  }
+  const int r = r0 + rt * 16 + l16, d0 = dt * 16 + 4 * qd;
+  if (r >= rows) return;
+  float4 o = make_float4(acc[0], acc[1], acc[2], acc[3]);
+  if (pos0 + r / G == 0) o = *reinterpret_cast<const float4*>(vals + d0);  // a single score copies V exactly
+  else if (!(finite(o.x) && finite(o.y) && finite(o.z) && finite(o.w))) flag(err, ERRBIT_NON_FINITE);
+  *reinterpret_cast<float4*>(out + ((size_t)(r / G) * H + g * G + r % G) * HD + d0) = o;
+}
+
+namespace {
+constexpr size_t kSoftmaxLds = 150 * 1024;
+size_t softmax_smem(int maxlen) { return ((size_t)8 * softmax_zs(maxlen) + ((maxlen + 3) & ~3)) * sizeof(float); }
+
+template <int HD>
+void launch_attention_hd(const float* q, const float* kc, const float* vc, int layer, int T, int pos0, int H, int KV,
+                         int n_ctx, float scale, float* scores, float* out, int* err, hipStream_t s) {
+  const int rows = T * (H / KV), end = pos0 + T;
+  constexpr int RT = 16 * pv_row_tiles<HD>();
+  launch_kernel(k_attn_qk_mfp<HD>, dim3((rows + 31) / 32, (end + 31) / 32, KV), dim3(512), 0, s, q, kc, layer, T,
+                pos0, H, KV, n_ctx, scale, scores, err);
+  static const bool attr = hipFuncSetAttribute((const void*)k_attn_softmax,
+                                               hipFuncAttributeMaxDynamicSharedMemorySize,
+                                               (int)kSoftmaxLds) == hipSuccess;
+  (void)attr;
+  launch_kernel(k_attn_softmax, dim3(H, T), dim3(256), softmax_smem(end), s, scores, T, pos0, H, n_ctx, err);
+  launch_kernel(k_attn_pv_mfp<HD>, dim3((rows + RT - 1) / RT, KV), dim3(HD / 16 * pv_row_tiles<HD>() * 64), 0, s,
+                scores, vc, layer, T, pos0, H, KV, n_ctx, out, err);
+}
+}  // namespace
+
+bool launch_attention_mfp(const float* q, const float* kc, const float* vc, int layer, int T, int pos0, int H, int KV,
+                          int hd, int n_ctx, float scale, float* scores, float* out, int* err, hipStream_t s) {
+  if (softmax_smem(pos0 + T) > kSoftmaxLds) return false;
+#define DTL_ATTN_HD(w) \
+  case w: launch_attention_hd<w>(q, kc, vc, layer, T, pos0, H, KV, n_ctx, scale, scores, out, err, s); return true
+  switch (hd) {
+    DTL_ATTN_HD(16);
+    DTL_ATTN_HD(32);
+    DTL_ATTN_HD(64);
+    DTL_ATTN_HD(80);
+    DTL_ATTN_HD(96);
+    DTL_ATTN_HD(128);
+  }
+#undef DTL_ATTN_HD
+  return false;
+}
+
 // Measurement support: the rate of k_q4k_mfp's inner pattern on a chip
 // with nothing else to do, four 16x16x1 outer products (4096 products per
 // wave) and the 64 ordered adds per lane that take them into four chains,

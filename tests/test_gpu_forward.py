@@ -143,6 +143,35 @@ def test_decode_attention_head_widths_match_oracle(monkeypatch, name, d, heads, 
             p += n
 
 
+@pytest.mark.parametrize("name,d,heads,kv_heads", [
+    ("smollm2", 576, 36, 12),  # 16-wide heads, three query heads per key head
+    ("qwen05", 448, 14, 2),    # 32, seven
+    ("smollm2", 640, 8, 4),    # 80
+    ("smollm2", 576, 6, 6),    # 96, one
+    ("qwen05", 896, 7, 1),     # 128, seven
+])
+@pytest.mark.parametrize("chunks", [(5, 11), (33, 64, 31), (130, 7)])
+def test_chunk_attention_head_widths_match_oracle(name, d, heads, kv_heads, chunks):
+    # Chunk attention on the matrix cores: tiles of 16 or 32 query rows that
+    # start and end inside a position, partial key tiles, position 0 (which
+    # copies its value row), rows past one 64-key slice.
+    import dataclasses
+
+    from detllm_amd import synth
+
+    w = dataclasses.replace(synth.WORKLOADS[name], d=d, heads=heads, kv_heads=kv_heads, ff=64, vocab=300, ctx=301)
+    data = synth.build_model(w, layers=2)
+    toks = [int(t) for t in synth.tokens(w, sum(chunks))]
+    ref = detref.Model(data).logits(toks)
+    with _model(data).forward_workspace(301, 130) as s:
+        p = 0
+        for n in chunks:
+            got = s.forward_chunk(toks[p:p + n], p, want_logits=True)
+            bad = np.nonzero(got.view(np.uint32) != ref[p:p + n].view(np.uint32))
+            assert bad[0].size == 0, (p, bad[0][:1], bad[1][:1])
+            p += n
+
+
 def test_decode_attention_long_row_matches_oracle():
     # The Z chains run in segments of 8192 exps: rows just below, at and past one.
     import dataclasses
