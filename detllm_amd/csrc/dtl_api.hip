@@ -1816,8 +1816,9 @@ int dtl_cdf(dtl_session* s, size_t row, size_t tail, uint32_t* freq, uint64_t* c
   if (tail > 256) return DTL_ERR_INVALID_ARGUMENT;  // table staging holds vocab + 256 entries
   HIP_TRY(hipSetDevice(s->m->device));
   clear_err(s);
-  launch_cdf(s->ln->logits + row * V, 1, (int)V, (int)tail, 1, nullptr, nullptr, nullptr, nullptr,
-             s->ln->c_total, nullptr, s->ln->c_freq_tab, s->ln->c_cum_tab, s->ln->err, s->ln->stream);
+  s->ln->cdf_ready_row = SIZE_MAX;  // the scratch changes hands
+  launch_cdf_table(s->ln->logits + row * V, (int)V, (int)tail, s->ln->c_scratch, s->ln->c_freq_tab, s->ln->c_cum_tab,
+                   s->ln->c_total, s->ln->err, s->ln->stream);
   HIP_TRY(hipMemcpyAsync(freq, s->ln->c_freq_tab, (V + tail) * 4, hipMemcpyDeviceToHost, s->ln->stream));
   HIP_TRY(hipMemcpyAsync(cum, s->ln->c_cum_tab, (V + tail) * 8, hipMemcpyDeviceToHost, s->ln->stream));
   HIP_TRY(hipMemcpyAsync(total, s->ln->c_total, 8, hipMemcpyDeviceToHost, s->ln->stream));
@@ -1947,15 +1948,13 @@ int run_cdf_host(const float* logits, size_t n, size_t tail, int mode, uint32_t 
     if ((st = sc.arena.alloc(&dft, n + tail))) return st;
     if ((st = sc.arena.alloc(&dct, n + tail))) return st;
   }
-  if (mode == 1) {
-    launch_cdf(dl, 1, (int)n, (int)tail, mode, dsym, nullptr, dcum, dfreq, dtot, nullptr, dft, dct,
-               sc.err, sc.stream);
-  } else {
-    uint8_t* scratch;
-    if ((st = sc.arena.alloc(&scratch, cdf_scratch_bytes(1, (int)n)))) return st;
+  uint8_t* scratch;
+  if ((st = sc.arena.alloc(&scratch, cdf_scratch_bytes(1, (int)n)))) return st;
+  if (mode == 1)
+    launch_cdf_table(dl, (int)n, (int)tail, scratch, dft, dct, dtot, sc.err, sc.stream);
+  else
     launch_cdf_blocks(dl, nullptr, 1, (int)n, (int)tail, mode, dsym, nullptr, dcum, dfreq, dtot,
                       nullptr, scratch, false, sc.err, sc.stream);
-  }
   if (mode == 1) {
     HIP_TRY(hipMemcpyAsync(freq_tab, dft, (n + tail) * 4, hipMemcpyDeviceToHost, sc.stream));
     HIP_TRY(hipMemcpyAsync(cum_tab, dct, (n + tail) * 8, hipMemcpyDeviceToHost, sc.stream));

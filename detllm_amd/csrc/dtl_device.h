@@ -358,16 +358,10 @@ void launch_swiglu(const float* g, const float* u, int count, float* out, int* e
 void launch_rope_table(float base, int rope_dim, int positions, float* cos_out, float* sin_out,
                        int* err, hipStream_t s);
 
-// CDF over rows of logits [R][V].
+// CDF over rows of logits [R][V], spread over many workgroups per row.
 //   mode 0: symbol range for symbols[r]        -> cum[r], freq[r], total[r]
-//   mode 1: full table for one row             -> freq_tab[V+tail], cum_tab[V+tail], total[0]
 //   mode 2: decoder lookup of values[r]        -> sym[r], cum[r], freq[r], total[r]
 //   mode 3: decoder total only                 -> total[r]
-void launch_cdf(const float* logits, int R, int V, int tail, int mode, const uint32_t* symbols,
-                const uint64_t* values, uint64_t* cum, uint32_t* freq, uint64_t* total,
-                uint32_t* sym, uint32_t* freq_tab, uint64_t* cum_tab, int* err, hipStream_t s);
-
-// Modes 0, 2 and 3 of launch_cdf spread over many workgroups per row;
 // scratch holds cdf_scratch_bytes(R, V) bytes of device memory.  rows
 // (device, optional): row r of the launch is logits row rows[r].
 // finish_only: the scratch already holds this row's block results (a
@@ -386,6 +380,10 @@ void launch_cdf_blocks(const float* logits, const uint32_t* rows, int R, int V, 
                        const uint32_t* symbols, const uint64_t* values, uint64_t* cum,
                        uint32_t* freq, uint64_t* total, uint32_t* sym, void* scratch,
                        bool finish_only, int* err, hipStream_t s);
+// The full table of one row: freq_tab[V + tail], cum_tab[V + tail] (both
+// 16-byte aligned), total[0]; scratch as for one row above.
+void launch_cdf_table(const float* logits, int V, int tail, void* scratch, uint32_t* freq_tab, uint64_t* cum_tab,
+                      uint64_t* total, int* err, hipStream_t s);
 // One row's decoder step: the block pass, then the lookup of the value
 // RangeDecoder::decode_freq forms from the decoder's window (cml = code -
 // low, rng = range) against the row's total.  pack[0..6]: symbol, cum, freq,

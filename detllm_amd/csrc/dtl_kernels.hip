@@ -1995,13 +1995,11 @@ void launch_rope_table(float base, int rope_dim, int positions, float* cos_out, 
 }
 
 // ---------------------------------------------------------------------------
-// logits -> integer CDF (det-coder cdf.rs).  One workgroup of 256 threads
-// per row.  max -> e_i = exp_f32(max(l_i - m, -88)) -> Z by the 8-lane sum
-// (8 chains over LDS tiles) -> f_i = (u32)(e_i/Z * 2^24) + 1 -> exact
+// logits -> integer CDF (det-coder cdf.rs): max -> e_i = exp_f32(max(l_i - m,
+// -88)) -> Z by the 8-lane sum -> f_i = (u32)(e_i/Z * 2^24) + 1 -> exact
 // integer sums / scans.
 namespace {
 constexpr int kCdfThreads = 256;
-constexpr int kCdfTile = kCdfThreads * 8;
 
 __device__ __forceinline__ uint32_t cdf_freq(float e, float z) {
   float p = e / z;
@@ -2028,220 +2026,10 @@ __device__ uint64_t block_scan_u64(uint64_t v, uint64_t* sh, uint64_t* total) {
 }
 }  // namespace
 
-__global__ void __launch_bounds__(256) k_cdf(const float* logits, int V, int tail, int mode,
-                                             const uint32_t* symbols, const uint64_t* values,
-                                             uint64_t* cum, uint32_t* freq, uint64_t* total,
-                                             uint32_t* sym, uint32_t* freq_tab, uint64_t* cum_tab,
-                                             int* err) {
-  // Z tiles, chain-major: element idx of a tile sits at [idx % 8][idx / 8],
-  // double-buffered (wave 0 sums one while waves 1-3 fill the other).
-  constexpr int kChainLen = kCdfTile / 8;
-  constexpr int kChainStride = kChainLen + 4;
-  __shared__ __align__(16) float ztile[2][8][kChainStride];
-  __shared__ float chain[8];
-  __shared__ float red[kCdfThreads / 64];
-  __shared__ uint64_t scan[kCdfThreads];
-  int r = blockIdx.x, tid = threadIdx.x;
-  const float* l = logits + (size_t)r * V;
-  // max (order independent) + finiteness
-  // Strided passes over the row load 8 values ahead of their use.
-  constexpr int kBatch = 8;
-  float mx = -__builtin_huge_valf();
-  bool bad = false;
-  for (int i0 = tid; i0 < V; i0 += kBatch * kCdfThreads) {
-    float v[kBatch];
-#pragma unroll
-    for (int k = 0; k < kBatch; k++) {
-      int i = i0 + k * kCdfThreads;
-      v[k] = i < V ? l[i] : -__builtin_huge_valf();
-    }
-#pragma unroll
-    for (int k = 0; k < kBatch; k++) {
-      if (i0 + k * kCdfThreads < V && !finite(v[k])) bad = true;
-      mx = fmaxf(mx, v[k]);
-    }
-  }
-  mx = wave_fmax(mx);
-  if ((tid & 63) == 0) red[tid / 64] = mx;
-  __syncthreads();
-  mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-  if (bad) flag(err, ERRBIT_CDF_NON_FINITE);
-  // Z: chain c adds e_i for i = c mod 8 ascending (tiles start at multiples
-  // of 8, so tile index idx keeps i's class).  Waves 1-3 produce tile k+1
-  // while lanes 0-7 of wave 0 consume tile k.
-  const int ntiles = (V + kCdfTile - 1) / kCdfTile;
-  constexpr int kProducers = kCdfThreads - 64;
-  constexpr int kPerProducer = (kCdfTile + kProducers - 1) / kProducers;
-  auto produce = [&](int k) {
-    const int base = k * kCdfTile;
-    float(*dst)[kChainStride] = ztile[k & 1];
-    float v[kPerProducer];
-#pragma unroll
-    for (int j = 0; j < kPerProducer; j++) {
-      int idx = tid - 64 + j * kProducers;
-      int i = base + idx;
-      v[j] = idx < kCdfTile && i < V ? l[i] : 0.0f;
-    }
-#pragma unroll
-    for (int j = 0; j < kPerProducer; j++) {
-      int idx = tid - 64 + j * kProducers;
-      int i = base + idx;
-      if (idx < kCdfTile) dst[idx & 7][idx >> 3] = i < V ? exp_clamped(v[j] - mx) : 0.0f;
-    }
-  };
-  float acc = 0.0f;
-  if (tid >= 64) produce(0);
-  __syncthreads();
-  for (int k = 0; k < ntiles; k++) {
-    if (tid >= 64) {
-      if (k + 1 < ntiles) produce(k + 1);
-    } else if (tid < 8) {
-      const int base = k * kCdfTile;
-      const int lim = V - base < kCdfTile ? V - base : kCdfTile;
-      const int cnt = (lim - tid + 7) / 8;  // elements tid, tid+8, ... below lim
-      const float* my = ztile[k & 1][tid];
-      int j = 0;
-      for (; j + 16 <= cnt; j += 16) {
-        float4 f0 = *reinterpret_cast<const float4*>(my + j);
-        float4 f1 = *reinterpret_cast<const float4*>(my + j + 4);
-        float4 f2 = *reinterpret_cast<const float4*>(my + j + 8);
-        float4 f3 = *reinterpret_cast<const float4*>(my + j + 12);
-        acc += f0.x; acc += f0.y; acc += f0.z; acc += f0.w;
-        acc += f1.x; acc += f1.y; acc += f1.z; acc += f1.w;
-        acc += f2.x; acc += f2.y; acc += f2.z; acc += f2.w;
-        acc += f3.x; acc += f3.y; acc += f3.z; acc += f3.w;
-      }
-      for (; j < cnt; j++) acc += my[j];
-    }
-    __syncthreads();
-  }
-  if (tid < 8) chain[tid] = acc;
-  __syncthreads();
-  float z = finish_8lane(chain);
-  if (mode == 0) {
-    // Symbol range: three plain sums (every f_i, the f_i below the symbol)
-    // and the symbol's own f; integer sums are exact in any order.
-    const uint32_t want_sym = symbols[r];
-    uint64_t run_part = 0, below_part = 0;
-    uint32_t found_freq = 0;
-    bool found = false;
-    for (int i0 = tid; i0 < V; i0 += kBatch * kCdfThreads) {
-      float v[kBatch];
-#pragma unroll
-      for (int k = 0; k < kBatch; k++) {
-        int i = i0 + k * kCdfThreads;
-        v[k] = i < V ? l[i] : 0.0f;
-      }
-#pragma unroll
-      for (int k = 0; k < kBatch; k++) {
-        int i = i0 + k * kCdfThreads;
-        if (i < V) {
-          uint32_t f = cdf_freq(exp_clamped(v[k] - mx), z);
-          run_part += f;
-          if ((uint32_t)i < want_sym) below_part += f;
-          if ((uint32_t)i == want_sym) {
-            found = true;
-            found_freq = f;
-          }
-        }
-      }
-    }
-    uint64_t run, below;
-    block_scan_u64(run_part, scan, &run);
-    block_scan_u64(below_part, scan, &below);
-    uint64_t tot_all = run + (uint64_t)tail;
-    if (tid == 0 && (run >= (1ull << 31) || tot_all >= (1ull << 31))) flag(err, ERRBIT_CDF_TOTAL);
-    if (found) {
-      cum[r] = below;
-      freq[r] = found_freq;
-    }
-    if (tid == 0) {
-      if (want_sym >= (uint32_t)V) {
-        cum[r] = run + (want_sym - (uint32_t)V);
-        freq[r] = 1;
-      }
-      total[r] = tot_all;
-    }
-    return;
-  }
-  // Table / lookup / total: each thread owns 8 consecutive entries of a
-  // tile; an exact block scan gives each entry's cumulative frequency.
-  uint64_t target = 0, run = 0;
-  if (mode == 2) target = values[r];
-  uint64_t found_cum = 0;
-  uint32_t found_freq = 0, found_sym = 0;
-  bool found = false;
-  for (int base = 0; base < V; base += kCdfTile) {
-    uint32_t f[8];
-    uint64_t local = 0;
-    int i0 = base + tid * 8;
-#pragma unroll
-    for (int k = 0; k < 8; k++) {
-      int i = i0 + k;
-      f[k] = i < V ? cdf_freq(exp_clamped(l[i] - mx), z) : 0u;
-      local += f[k];
-    }
-    uint64_t tot;
-    uint64_t incl = block_scan_u64(local, scan, &tot);
-    uint64_t c = run + incl - local;
-#pragma unroll
-    for (int k = 0; k < 8; k++) {
-      int i = i0 + k;
-      if (i < V) {
-        if (mode == 1) {
-          freq_tab[i] = f[k];
-          cum_tab[i] = c;
-        } else if (mode == 2 && !found && target >= c && target < c + f[k]) {
-          found = true;
-          found_sym = (uint32_t)i;
-          found_cum = c;
-          found_freq = f[k];
-        }
-        c += f[k];
-      }
-    }
-    run += tot;
-  }
-  // run = sum of all f_i over the vocabulary
-  uint64_t tot_all = run + (uint64_t)tail;
-  if (run >= (1ull << 31) || tot_all >= (1ull << 31)) {
-    if (tid == 0) flag(err, ERRBIT_CDF_TOTAL);
-  }
-  if (mode == 1) {
-    for (int k = tid; k < tail; k += kCdfThreads) {
-      freq_tab[V + k] = 1;
-      cum_tab[V + k] = run + (uint64_t)k;
-    }
-    if (tid == 0) total[0] = tot_all;
-  } else if (mode == 2) {
-    if (found) {
-      sym[r] = found_sym;
-      cum[r] = found_cum;
-      freq[r] = found_freq;
-    }
-    if (tid == 0) {
-      total[r] = tot_all;
-      if (target >= run) {
-        uint64_t off = target - run;
-        if (off < (uint64_t)tail) {
-          sym[r] = (uint32_t)(V + off);
-          cum[r] = target;
-          freq[r] = 1;
-        } else {
-          flag(err, ERRBIT_CDF_LOOKUP);
-        }
-      }
-    }
-  } else {
-    if (tid == 0) total[r] = tot_all;
-  }
-}
-
-// ---------------------------------------------------------------------------
-// The same CDF split over many workgroups per row (modes 0, 2, 3): block
-// maxima, block exps written chain-major, one wave per row for the eight
-// serial Z chains, block frequency sums, and a per-row finish with the exact
-// integer sums / search.  Every f32 operation is the one k_cdf performs.
+// Split over many workgroups per row: block maxima, block exps written
+// chain-major, the eight Z chains, block frequency sums, and a finish with
+// the exact integer sums: per row a symbol's range, a total or a lookup
+// (k_cdf_finish), or per block its part of the table (k_cdf_table).
 namespace {
 constexpr int kCdfBlk = (int)kCdfBlockElems;  // elements per workgroup (256 threads x 16)
 
@@ -2600,6 +2388,64 @@ __global__ void __launch_bounds__(256) k_cdf_finish(int V, int nb, int tail, int
   }
 }
 
+// The full table of one row: block b's frequencies and their exclusive sums,
+// from the block sums before it; the last block also writes the escape
+// symbols and the total.  A thread owns 16 consecutive symbols, written as
+// 16-byte stores.  One workgroup for the whole row took 561 us for 151936
+// logits.
+__global__ void __launch_bounds__(256) k_cdf_table(int V, int tail, CdfScratch cs, uint32_t* freq_tab,
+                                                   uint64_t* cum_tab, uint64_t* total, int* err) {
+  __shared__ uint64_t scan[256];
+  const int b = blockIdx.x, nb = gridDim.x, tid = threadIdx.x;
+  const int v8 = cdf_v8(V);
+  uint64_t base = 0;
+  for (int k = 0; k < b; k++) base += cs.bsum[k];
+  const float z = cs.z[0];
+  const int i0 = b * kCdfBlk + 16 * tid;
+  __align__(16) uint32_t f[16];
+  __align__(16) uint64_t c[16];
+  uint64_t local = 0;
+#pragma unroll
+  for (int k = 0; k < 16; k++) {
+    const int i = i0 + k;
+    f[k] = i < V ? cdf_freq(cs.ebuf[(size_t)(i & 7) * v8 + (i >> 3)], z) : 0u;
+    local += f[k];
+  }
+  uint64_t all;
+  uint64_t run = base + block_scan_u64(local, scan, &all) - local;
+#pragma unroll
+  for (int k = 0; k < 16; k++) {
+    c[k] = run;
+    run += f[k];
+  }
+  if (i0 + 15 < V) {
+#pragma unroll
+    for (int k = 0; k < 16; k += 4)
+      *reinterpret_cast<uint4*>(freq_tab + i0 + k) = make_uint4(f[k], f[k + 1], f[k + 2], f[k + 3]);
+#pragma unroll
+    for (int k = 0; k < 16; k += 2)
+      *reinterpret_cast<ulonglong2*>(cum_tab + i0 + k) = make_ulonglong2(c[k], c[k + 1]);
+  } else {
+#pragma unroll
+    for (int k = 0; k < 16; k++)
+      if (i0 + k < V) {
+        freq_tab[i0 + k] = f[k];
+        cum_tab[i0 + k] = c[k];
+      }
+  }
+  if (b != nb - 1) return;
+  const uint64_t sum = base + all;
+  for (int k = tid; k < tail; k += 256) {
+    freq_tab[V + k] = 1;
+    cum_tab[V + k] = sum + (uint64_t)k;
+  }
+  if (tid == 0) {
+    const uint64_t tot = sum + (uint64_t)tail;
+    if (sum >= (1ull << 31) || tot >= (1ull << 31)) flag(err, ERRBIT_CDF_TOTAL);
+    total[0] = tot;
+  }
+}
+
 // The block kernels of launch_cdf_blocks: block maxima, exps, Z and block
 // sums (mode 0: also the sums below symbols[r]).
 void launch_cdf_block_pass(const float* logits, const uint32_t* rows, int R, int V, int mode,
@@ -2639,11 +2485,11 @@ void launch_cdf_decode(const float* logits, int V, int tail, uint64_t cml, uint6
                 (uint32_t*)nullptr, cs, err, cml, rng, pack);
 }
 
-void launch_cdf(const float* logits, int R, int V, int tail, int mode, const uint32_t* symbols,
-                const uint64_t* values, uint64_t* cum, uint32_t* freq, uint64_t* total,
-                uint32_t* sym, uint32_t* freq_tab, uint64_t* cum_tab, int* err, hipStream_t s) {
-  launch_kernel(k_cdf, dim3(R), dim3(kCdfThreads), 0, s, logits, V, tail, mode, symbols,
-                     values, cum, freq, total, sym, freq_tab, cum_tab, err);
+void launch_cdf_table(const float* logits, int V, int tail, void* scratch, uint32_t* freq_tab, uint64_t* cum_tab,
+                      uint64_t* total, int* err, hipStream_t s) {
+  CdfScratch cs = cdf_scratch(scratch, 1, V);
+  launch_cdf_block_pass(logits, nullptr, 1, V, 3, nullptr, cs, err, s);
+  launch_kernel(k_cdf_table, dim3(cdf_nblk(V)), dim3(256), 0, s, V, tail, cs, freq_tab, cum_tab, total, err);
 }
 
 // ---------------------------------------------------------------------------
