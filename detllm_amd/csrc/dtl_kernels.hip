@@ -2208,15 +2208,197 @@ __global__ void __launch_bounds__(256) k_cdf_z(int V, CdfScratch cs) {
   if (tid == 0) cs.z[r] = finish_8lane(zc);
 }
 
+// One chain of Z by many threads, with the same bits as its serial sum.  The
+// terms are positive, so the running sum s only grows, and while it stays in
+// one binade [2^k, 2^(k+1)) every addition rounds to the same grid u =
+// 2^(k-23): in units of u, s is an integer S in [2^23, 2^24), and fl(s + e)
+// is S + n with n = e / u rounded to the nearest integer, a tie going to the n
+// that makes S + n even.  n depends on S only through its parity, and only
+// for ties, so a run of terms is a map from the parity of S to an integer
+// increment; maps compose associatively.  Each thread forms the map of a
+// block of terms, a scan composes them, and the first block at whose end S
+// would reach 2^24 is added serially (as f32 adds, from the exact sum before
+// it); the next terms go on in the next binade.  The first kZHead terms are
+// added serially (the sum doubles often there); after them a chain of n
+// terms crosses about log2(n / kZHead) binades.  Increments saturate at 2^25,
+// past any crossing.
+//
+// One workgroup per (chain, row); the chain in LDS.  Sums go to the row's
+// block maxima (8 of its floats, no longer needed).  Bound by the passes'
+// latencies (scan, barriers) and by the workgroup's instruction issue.
+//
+// Chosen up to V / 2048 rows: with more, the serial chains of k_cdf_z run
+// side by side on more CUs and take fewer instructions in all.  us per
+// symbol-range call, k_cdf_z against this: V = 151936 with 1 / 16 / 64 / 512
+// rows 83 / 90 / 114 / 417 against 50 / 60 / 98 / 547; 49152 with 4 / 16 / 32
+// rows 46.6 / 46.3 / 47.1 against 42.5 / 44.3 / 48.1; 32768 with 1 row 39.7
+// against 37.3.
+constexpr int kZParThreads = 1024;
+constexpr int kZHead = 512;
+constexpr int kZParMinV = 32768;  // from here a row has at least eight block maxima
+constexpr int kZParRowDiv = 2048;
+constexpr size_t kZParLds = 140 * 1024;  // a chain of 2^18 / 8 terms takes 128 KB
+
+__global__ void __launch_bounds__(kZParThreads) k_cdf_zpar(int V, int nb, CdfScratch cs) {
+  extern __shared__ __align__(16) float e[];
+  constexpr int NW = kZParThreads / 64;
+  constexpr int kSat = 1 << 25, kTop = 1 << 24;
+  __shared__ __align__(16) int w0[NW], w1[NW];
+  __shared__ int cross, s_at;
+  __shared__ float s_sh;
+  const int c = blockIdx.x, r = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int cnt = (V - c + 7) / 8, v8 = cdf_v8(V);
+  const float* src = cs.ebuf + ((size_t)r * 8 + c) * v8;
+  for (int j = 4 * tid; j < v8; j += 4 * kZParThreads) {
+    const float4 f = *reinterpret_cast<const float4*>(src + j);
+    e[j] = j < cnt ? f.x : 0.0f;
+    e[j + 1] = j + 1 < cnt ? f.y : 0.0f;
+    e[j + 2] = j + 2 < cnt ? f.z : 0.0f;
+    e[j + 3] = j + 3 < cnt ? f.w : 0.0f;
+  }
+  __syncthreads();
+  int p = cnt < kZHead ? cnt : kZHead;  // terms added so far (a multiple of four, or all)
+  if (wave == 0) {
+    const float s0 = chain_group_lds<16>(0.0f, e, p);
+    if (lane == 0) s_sh = s0;
+  }
+  __syncthreads();
+  float s = s_sh;
+  while (p < cnt) {  // the same on every thread
+    const int ex = (int)((f2u(s) >> 23) & 0xffu);
+    if (ex == 0 || ex == 255) {  // no such grid (a subnormal or non-finite sum): serially
+      __syncthreads();
+      if (wave == 0) {
+        const float t = chain_group_lds<16>(s, e + p, cnt - p);
+        if (lane == 0) s_sh = t;
+      }
+      __syncthreads();
+      s = s_sh;
+      break;
+    }
+    const int sh = 23 - (ex - 127);  // e / u = e 2^sh
+    const int S = (int)((f2u(s) & 0x7fffffu) | 0x800000u);
+    // As many terms as the sum has had at most doubles again: the pass takes
+    // twice that, and at least four per thread.
+    const int W = 2 * p > 4 * kZParThreads ? 2 * p : 4 * kZParThreads;
+    const int lim = cnt - p < W ? cnt : p + W;
+    const int B = ((lim - p + kZParThreads - 1) / kZParThreads + 3) & ~3;
+    const int j0 = p + tid * B, j1 = j0 + B < lim ? j0 + B : lim;
+    // d0 / d1: the block's increment of an even / odd S
+    int d0 = 0, d1 = 0;
+    bool big = false;
+#pragma unroll 2
+    for (int j = j0; j < j1; j += 4) {  // terms past the chain are +0.0
+      const float4 e4 = *reinterpret_cast<const float4*>(e + j);
+      const float ev[4] = {e4.x, e4.y, e4.z, e4.w};
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const float x = __builtin_ldexpf(ev[k], sh);  // exact, or past any crossing
+        big |= !(x < 16777216.0f);
+        const float rn = __builtin_rintf(x), t = x - rn;
+        const int n = (int)rn;
+        if (t == 0.5f || t == -0.5f) {
+          // the neighbour that leaves S even: n, or the integer on the other side
+          const int o = n + (t > 0.0f ? 1 : -1);
+          d0 += ((d0 + n) & 1) ? o : n;
+          d1 += ((1 + d1 + n) & 1) ? o : n;
+        } else {
+          d0 += n;
+          d1 += n;
+        }
+      }
+      d0 = d0 < kSat ? d0 : kSat;
+      d1 = d1 < kSat ? d1 : kSat;
+    }
+    if (big) d0 = d1 = kSat;
+    // Inclusive scan over the wave's blocks, earlier block first, by DPP (lanes
+    // without a source get the identity, 0 / 0): within rows, then row 0 into
+    // row 1 and row 2 into row 3, then rows 0-1 into rows 2 and 3.
+    int i0 = d0, i1 = d1;
+    auto after_map = [&](int o0, int o1) {
+      const int n0 = o0 + ((o0 & 1) ? i1 : i0), n1 = o1 + (((1 + o1) & 1) ? i1 : i0);
+      i0 = n0 < kSat ? n0 : kSat;
+      i1 = n1 < kSat ? n1 : kSat;
+    };
+#define DTL_Z_STEP(ctrl, rows)                                                 \
+  after_map(__builtin_amdgcn_update_dpp(0, i0, ctrl, rows, 0xf, false),        \
+            __builtin_amdgcn_update_dpp(0, i1, ctrl, rows, 0xf, false))
+    DTL_Z_STEP(0x111, 0xf);  // row_shr:1
+    DTL_Z_STEP(0x112, 0xf);
+    DTL_Z_STEP(0x114, 0xf);
+    DTL_Z_STEP(0x118, 0xf);
+    DTL_Z_STEP(kDppRowBcast15, 0xa);
+    DTL_Z_STEP(kDppRowBcast31, 0xc);
+#undef DTL_Z_STEP
+    const int p0 = __shfl_up(i0, 1), p1 = __shfl_up(i1, 1);
+    if (lane == 63) {
+      w0[wave] = i0;
+      w1[wave] = i1;
+    }
+    if (tid == 0) cross = -1;
+    __syncthreads();
+    int sw = S;  // S before this wave's blocks
+    int m0[NW], m1[NW];
+#pragma unroll
+    for (int w = 0; w < NW; w += 4) {
+      const int4 a0 = *reinterpret_cast<const int4*>(w0 + w), a1 = *reinterpret_cast<const int4*>(w1 + w);
+      m0[w] = a0.x, m0[w + 1] = a0.y, m0[w + 2] = a0.z, m0[w + 3] = a0.w;
+      m1[w] = a1.x, m1[w + 1] = a1.y, m1[w + 2] = a1.z, m1[w + 3] = a1.w;
+    }
+#pragma unroll
+    for (int w = 0; w < NW - 1; w++) {
+      const int n = sw + ((sw & 1) ? m1[w] : m0[w]);
+      sw = w < wave ? (n < kSat ? n : kSat) : sw;
+    }
+    const int before = lane == 0 ? sw : sw + ((sw & 1) ? p1 : p0);
+    const int after = sw + ((sw & 1) ? i1 : i0);
+    if (before < kTop && after >= kTop) {  // one thread at most: S never falls
+      cross = tid;
+      s_at = before;
+    } else if (tid == kZParThreads - 1 && after < kTop) {
+      s_at = after;
+    }
+    __syncthreads();
+    const int ct = cross;
+    s = __builtin_ldexpf((float)s_at, -sh);
+    if (ct < 0) {
+      p = lim;
+      __syncthreads();  // s_at, cross and the waves' totals are read
+      continue;
+    }
+    const int q = p + ct * B, n = lim - q < B ? lim - q : B;
+    if (wave == 0) {
+      const float t = chain_group_lds<16>(s, e + q, n);
+      if (lane == 0) s_sh = t;
+    }
+    __syncthreads();
+    s = s_sh;
+    p = q + n;
+    __syncthreads();
+  }
+  if (tid == 0) cs.pmax[(size_t)r * nb + c] = s;
+}
+
 // Block sums of f_i = (u32)(e_i / Z * 2^24) + 1 (exact integers): all, and
 // (mode 0) those below the symbol, plus the symbol's own f.
-__global__ void __launch_bounds__(256) k_cdf_bfreq(int V, int mode, const uint32_t* symbols,
+// zsums: the row's eight Z chain sums are in its block maxima (k_cdf_zpar);
+// every block joins them, the first also stores Z.
+__global__ void __launch_bounds__(256) k_cdf_bfreq(int V, int mode, const uint32_t* symbols, bool zsums,
                                                    CdfScratch cs) {
   __shared__ uint64_t red[4];
   const int r = blockIdx.y, b = blockIdx.x, nb = gridDim.x;
   const int v8 = cdf_v8(V);
   const float* e = cs.ebuf + (size_t)r * 8 * v8;
-  const float z = cs.z[r];
+  float z;
+  if (zsums) {
+    float part[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) part[k] = cs.pmax[(size_t)r * nb + k];
+    z = finish_8lane(part);
+    if (b == 0 && threadIdx.x == 0) cs.z[r] = z;
+  } else {
+    z = cs.z[r];
+  }
   const uint32_t want = mode == 0 ? symbols[r] : 0xffffffffu;
   // This block's elements b*4096 .. +4096 sit at chain positions
   // [c][512 b .. 512 b + 511]; thread x takes c = x / 32 and 16 consecutive j.
@@ -2453,15 +2635,23 @@ void launch_cdf_block_pass(const float* logits, const uint32_t* rows, int R, int
   const int nb = cdf_nblk(V);
   launch_kernel(k_cdf_bmax, dim3(nb, R), dim3(256), 0, s, logits, rows, V, cs, err);
   launch_kernel(k_cdf_bexp, dim3(nb, R), dim3(256), 0, s, logits, rows, V, cs);
-  constexpr size_t kZRing = 3 * 8 * 1024 * sizeof(float);  // k_cdf_z's segment ring
-  static bool z_attr_set = false;
-  if (!z_attr_set) {
-    (void)hipFuncSetAttribute((const void*)k_cdf_z, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)kZRing);
-    z_attr_set = true;
+  const bool zpar = V >= kZParMinV && R <= V / kZParRowDiv && (size_t)cdf_v8(V) * sizeof(float) <= kZParLds;
+  if (zpar) {
+    static const bool attr = hipFuncSetAttribute((const void*)k_cdf_zpar, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                 (int)kZParLds) == hipSuccess;
+    (void)attr;
+    launch_kernel(k_cdf_zpar, dim3(8, R), dim3(kZParThreads), (size_t)cdf_v8(V) * sizeof(float), s, V, nb, cs);
+  } else {
+    constexpr size_t kZRing = 3 * 8 * 1024 * sizeof(float);  // k_cdf_z's segment ring
+    static bool z_attr_set = false;
+    if (!z_attr_set) {
+      (void)hipFuncSetAttribute((const void*)k_cdf_z, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)kZRing);
+      z_attr_set = true;
+    }
+    launch_kernel(k_cdf_z, dim3(R), dim3(256), kZRing, s, V, cs);
   }
-  launch_kernel(k_cdf_z, dim3(R), dim3(256), kZRing, s, V, cs);
-  launch_kernel(k_cdf_bfreq, dim3(nb, R), dim3(256), 0, s, V, mode, symbols, cs);
+  launch_kernel(k_cdf_bfreq, dim3(nb, R), dim3(256), 0, s, V, mode, symbols, zpar, cs);
 }
 
 void launch_cdf_blocks(const float* logits, const uint32_t* rows, int R, int V, int tail, int mode,

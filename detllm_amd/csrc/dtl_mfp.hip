@@ -720,14 +720,18 @@ void launch_mfp_probe(float* out, int workgroups, int iters, hipStream_t s) {
   launch_kernel(k_mfp_probe, dim3(workgroups), dim3(256), 0, s, out, 1.0001f, 0.5f, iters);
 }
 
-// Tiles (waves over positions x rows), chosen on the pipelined TinyLlama
-// encode (64 positions, four chunks in flight; ms per step): gate + up
-// 2 x 2 (98.5; 4 x 1 100.5, 2 x 1 105.8, 1 x 2 106.0), the other matrices
-// 4 x 1 (98.5; 2 x 2 100.5, 2 x 1 106.4, 1 x 2 106.4, 1 x 1 109.2).
+// Tiles (waves over positions x rows): 2 x 2.  For the short matrices 4 x 1
+// (one row tile, four position tiles) was the faster with 64-position launches
+// side by side; from 96 positions on 2 x 2 is: us per launch alone, wo and
+// ffn_down on average / wq + wk of the TinyLlama-1.1B shape, 4 x 1 against 2 x
+// 2: 96 positions 51.4 against 48.5 / 42.1 against 31.7, 256 66.3 against 64.2
+// / 61.7 against 59.1, 512 130.6 against 115.4 / 97.9 against 93.0; the
+// pipelined 2048-token window 88.5 against 88.3 ms (86.8 against 88.3 in
+// chunks of 512).
 void launch_q4k_mfp(const Q4kF32Args& a, int mode, hipStream_t s) {
   if (mode == MODE_PAIR) return launch_mfp<2, 2, MODE_PAIR>(a, s);
-  if (mode == MODE_CAT) return launch_mfp<4, 1, MODE_CAT>(a, s);
-  launch_mfp<4, 1, MODE_SINGLE>(a, s);
+  if (mode == MODE_CAT) return launch_mfp<2, 2, MODE_CAT>(a, s);
+  launch_mfp<2, 2, MODE_SINGLE>(a, s);
 }
 
 }  // namespace dtl

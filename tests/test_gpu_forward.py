@@ -388,6 +388,47 @@ def test_standalone_cdf_kernel_matches_oracle(V):
             assert (r.cum, r.freq, r.total) == detref.symbol_range(lg, s, tail)
 
 
+@pytest.mark.parametrize("V", [32767, 32768, 40003, 151936, 261888])
+@pytest.mark.parametrize("pattern", ["equal", "halves", "spread", "peaked", "growing", "tiny chains", "ulps", "random"])
+def test_cdf_normaliser_by_many_threads_matches_oracle(V, pattern):
+    # From 32768 logits a few rows' Z chains are summed by many threads (maps
+    # of rounded increments, composed): terms that are ties of the running
+    # sum's grid in both directions, sums that cross many binades, late or in
+    # one block, one dominant term, terms far below the grid, chains whose
+    # sums stay subnormal, and (f sensitive to Z's last bits) large
+    # probabilities in each.
+    from detllm_amd import coder
+
+    rng = np.random.default_rng(V)
+    ln2 = np.log(2.0)
+    if pattern == "equal":
+        lg = np.zeros(V)
+    elif pattern == "halves":  # e near powers of two: bits just below the grid
+        lg = -ln2 * rng.integers(0, 24, V)
+    elif pattern == "spread":
+        lg = np.linspace(-80, 0, V)[rng.permutation(V)]
+    elif pattern == "peaked":
+        lg = rng.normal(-20, 3, V)
+        lg[V // 3], lg[V // 2], lg[7] = 0.0, -0.7, -3.0
+    elif pattern == "growing":  # the largest terms last
+        lg = np.linspace(-60, 0, V)
+    elif pattern == "tiny chains":  # only chain 3 holds terms that are not subnormal
+        lg = np.full(V, -200.0)
+        lg[3::8] = rng.normal(-1, 1, lg[3::8].size)
+    elif pattern == "ulps":
+        lg = rng.normal(0, 1e-6, V)
+        lg[: V // 2] -= 9.0
+    else:
+        lg = rng.normal(0, 3, V)
+    lg = lg.astype(np.float32)
+    rf, rc, rt = detref.logits_to_cdf(lg, 256)
+    got = coder.logits_to_cdf_with_byte_escapes(lg)
+    assert np.array_equal(got.freq, rf) and np.array_equal(got.cum, rc) and got.total == rt
+    for sym in (0, V // 3, V - 1):
+        r = coder.logits_to_symbol_range_with_byte_escapes(lg, sym)
+        assert (r.cum, r.freq, r.total) == (int(rc[sym]), int(rf[sym]), rt)
+
+
 @pytest.mark.parametrize("graph", [True, False])
 def test_decode_attention_regimes_match_oracle(monkeypatch, graph):
     """Single-position forwards in a 4096-position window (1-layer SmolLM2
