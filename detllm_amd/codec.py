@@ -62,6 +62,9 @@ class CodecError(enum.IntEnum):
     VocabMismatch = 93
 
 
+_BUFFER_TOO_SMALL = 44  # DTL_ERR_BUFFER_TOO_SMALL
+
+
 def _u8(data: bytes):
     buf = bytes(data)
     return (C.c_uint8 * max(len(buf), 1)).from_buffer_copy(buf or b"\0"), len(buf)
@@ -147,13 +150,18 @@ def encode_symbols_with_model(session: Session, symbols: Sequence[int], overlap:
     """encode_symbols_with_model with window n_ctx = session.n_ctx."""
     sym = np.ascontiguousarray(np.asarray(symbols, dtype=np.uint32))
     n = C.c_size_t()
-    st = lib.dtl_codec_encode(session._h, ptr(sym, C.c_uint32), sym.size, overlap, int(use_byte_escapes),
-                              None, 0, C.byref(n))
+    # one pass: room for eight bytes per symbol (a symbol codes to four or
+    # fewer, the range's underflow aside); a larger payload's size comes back
+    cap = 8 * sym.size + 64
+    while True:
+        buf = np.empty(cap, np.uint8)
+        st = lib.dtl_codec_encode(session._h, ptr(sym, C.c_uint32), sym.size, overlap, int(use_byte_escapes),
+                                  ptr(buf, C.c_uint8), buf.size, C.byref(n))
+        if st != _BUFFER_TOO_SMALL:
+            break
+        cap = n.value
     check(st, "encode_symbols_with_model")
-    buf = (C.c_uint8 * max(n.value, 1))()
-    check(lib.dtl_codec_encode(session._h, ptr(sym, C.c_uint32), sym.size, overlap, int(use_byte_escapes),
-                               buf, n.value, C.byref(n)), "encode_symbols_with_model")
-    return bytes(buf[: n.value])
+    return buf[: n.value].tobytes()
 
 
 def encode_tokens_with_model(session: Session, tokens: Sequence[int], overlap: int) -> bytes:

@@ -10,6 +10,7 @@
 #include <cstring>
 #include <memory>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../include/detllm.h"
@@ -670,6 +671,12 @@ constexpr int kMaxLanes = 4;
 constexpr size_t kEncodeRows = 256;
 constexpr int kWideLanes = 2;
 
+// Results of this size and more reach the caller's memory through pinned
+// slices on several host threads (see copy_out).
+constexpr size_t kCopyParallelBytes = 2u << 20;
+constexpr size_t kCopySlice = 1u << 20;
+constexpr int kCopyThreads = 8;
+
 static int lane_count() {
   if (const char* l = getenv("DETLLM_LANES")) {
     const int n = atoi(l);
@@ -719,26 +726,25 @@ struct Lane {
     }
     for (hipEvent_t e : kv_ready)
       if (e) (void)hipEventDestroy(e);
-    for (void* p : {(void*)h_tokens, (void*)h_rows, (void*)h_sym, (void*)h_freq, (void*)h_cum, (void*)h_total,
-                    (void*)h_err, (void*)h_io})
+    for (void* p : {(void*)h_cum, (void*)h_io})
       if (p) (void)hipHostFree(p);
     *this = Lane();
   }
 };
 
-// Grows a lane's pinned symbol staging to n symbols (the lane must be idle).
+// Grows a lane's pinned symbol staging to n symbols (the lane must be idle):
+// one block that starts at h_cum.
 static int lane_reserve(Lane& L, size_t n) {
   if (n <= L.h_cap) return DTL_OK;
-  for (void* p : {(void*)L.h_rows, (void*)L.h_sym, (void*)L.h_freq, (void*)L.h_cum, (void*)L.h_total})
-    if (p) (void)hipHostFree(p);
+  if (L.h_cum) (void)hipHostFree(L.h_cum);
   L.h_rows = L.h_sym = L.h_freq = nullptr;
   L.h_cum = L.h_total = nullptr;
   L.h_cap = 0;
-  HIP_TRY(hipHostMalloc((void**)&L.h_rows, n * 4, hipHostMallocDefault));
-  HIP_TRY(hipHostMalloc((void**)&L.h_sym, n * 4, hipHostMallocDefault));
-  HIP_TRY(hipHostMalloc((void**)&L.h_freq, n * 4, hipHostMallocDefault));
-  HIP_TRY(hipHostMalloc((void**)&L.h_cum, n * 8, hipHostMallocDefault));
-  HIP_TRY(hipHostMalloc((void**)&L.h_total, n * 8, hipHostMallocDefault));
+  HIP_TRY(hipHostMalloc((void**)&L.h_cum, n * 28, hipHostMallocDefault));
+  L.h_total = L.h_cum + n;
+  L.h_rows = reinterpret_cast<uint32_t*>(L.h_total + n);
+  L.h_sym = L.h_rows + n;
+  L.h_freq = L.h_sym + n;
   L.h_cap = n;
   return DTL_OK;
 }
@@ -749,13 +755,21 @@ struct dtl_session {
   Arena arena;
   float *rope_cos = nullptr, *rope_sin = nullptr, *kc = nullptr, *vc = nullptr;
   Lane lanes[kMaxLanes];
-  int nlanes = 1;        // lanes set up (the rest stay empty)
+  int nlanes = 1;        // lanes the pipelined encode may use; lane 0 is set up
+                         // with the session, the others by the first call that
+                         // needs them (ensure_lanes)
+  Arena lane_arena[kMaxLanes];
   // Lanes of kEncodeRows positions for the pipelined encode of sessions with
   // a smaller max_chunk, set up by its first call with more tokens than that.
   Arena wide_arena;
   Lane wide[kWideLanes];
   size_t wide_rows = 0;  // positions per chunk there (0: not set up)
   bool wide_failed = false;  // no memory for them: the session's own lanes serve
+  // Pinned slices and their events for large results (copy_out), set up by
+  // the first such copy.
+  uint8_t* out_pin = nullptr;
+  hipEvent_t out_ev[kCopyThreads] = {};
+  bool out_failed = false;
   Lane* ln = &lanes[0];  // the lane the launches below go to
   // Captured single-position forwards (see forward_device), on lane 0:
   // [0] for rows up to attention_fused_max_len() keys, [1] for the whole
@@ -773,6 +787,9 @@ struct dtl_session {
     for (hipGraphExec_t g : graph)
       if (g) (void)hipGraphExecDestroy(g);
     if (pos_host) (void)hipHostFree(pos_host);
+    if (out_pin) (void)hipHostFree(out_pin);
+    for (hipEvent_t e : out_ev)
+      if (e) (void)hipEventDestroy(e);
   }
 };
 
@@ -784,42 +801,54 @@ static int lane_init(dtl_session* s, Arena& A, Lane& L, size_t C) {
   const size_t hd = m->head_dim;
   int st;
   HIP_TRY(hipStreamCreateWithFlags(&L.stream, hipStreamNonBlocking));
-#define ALLOC(ptr, n) \
-  if ((st = A.alloc(&L.ptr, (n)))) return st;
-  ALLOC(x, C * c.d);
-  ALLOC(h, C * c.d);
-  ALLOC(q, C * c.heads * hd);
-  ALLOC(k, C * c.kv_heads * hd);
-  ALLOC(v, C * c.kv_heads * hd);
-  ALLOC(attn, C * c.heads * hd);
-  ALLOC(g, C * c.ff);
-  ALLOC(u, C * c.ff);
-  ALLOC(ffo, C * c.ff);
-  ALLOC(logits, C * m->vocab);
-  ALLOC(scores, C * c.heads * s->n_ctx);
-  ALLOC(qa, C * s->max_in);
-  ALLOC(qk, C * s->max_in);
-  ALLOC(af, C * s->max_in);
-  ALLOC(da, C * (s->max_in / 32 + 1));
-  ALLOC(dk, C * (s->max_in / 256 + 1));
-  ALLOC(tokens, C);
-  ALLOC(err, 1);
-  ALLOC(c_sym, C);
-  ALLOC(c_freq, C);
-  ALLOC(c_cum, C);
-  ALLOC(c_total, C);
-  ALLOC(c_values, C);
-  ALLOC(c_pack, 8);
-  ALLOC(c_freq_tab, m->vocab + 256);
-  ALLOC(c_cum_tab, m->vocab + 256);
-  ALLOC(c_scratch, cdf_scratch_bytes((int)C, (int)m->vocab));
-  ALLOC(c_rows, C);
+  // One device allocation, each buffer at a 256-byte boundary: first the
+  // sizes, then the places.
+  uint8_t* base = nullptr;
+  for (int pass = 0; pass < 2; pass++) {
+    size_t at = 0;
+#define ALLOC(ptr, n)                                              \
+  do {                                                             \
+    if (base) L.ptr = reinterpret_cast<decltype(L.ptr)>(base + at); \
+    at += ((size_t)(n) * sizeof(*L.ptr) + 255) & ~(size_t)255;     \
+  } while (0)
+    ALLOC(x, C * c.d);
+    ALLOC(h, C * c.d);
+    ALLOC(q, C * c.heads * hd);
+    ALLOC(k, C * c.kv_heads * hd);
+    ALLOC(v, C * c.kv_heads * hd);
+    ALLOC(attn, C * c.heads * hd);
+    ALLOC(g, C * c.ff);
+    ALLOC(u, C * c.ff);
+    ALLOC(ffo, C * c.ff);
+    ALLOC(logits, C * m->vocab);
+    ALLOC(scores, C * c.heads * s->n_ctx);
+    ALLOC(qa, C * s->max_in);
+    ALLOC(qk, C * s->max_in);
+    ALLOC(af, C * s->max_in);
+    ALLOC(da, C * (s->max_in / 32 + 1));
+    ALLOC(dk, C * (s->max_in / 256 + 1));
+    ALLOC(tokens, C);
+    ALLOC(err, 1);
+    ALLOC(c_sym, C);
+    ALLOC(c_freq, C);
+    ALLOC(c_cum, C);
+    ALLOC(c_total, C);
+    ALLOC(c_values, C);
+    ALLOC(c_pack, 8);
+    ALLOC(c_freq_tab, m->vocab + 256);
+    ALLOC(c_cum_tab, m->vocab + 256);
+    ALLOC(c_scratch, cdf_scratch_bytes((int)C, (int)m->vocab));
+    ALLOC(c_rows, C);
 #undef ALLOC
+    if (!base && (st = A.alloc(&base, at))) return st;
+  }
   L.kv_ready.assign(c.block_count, nullptr);
   for (hipEvent_t& e : L.kv_ready) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-  HIP_TRY(hipHostMalloc((void**)&L.h_tokens, C * 4, hipHostMallocDefault));
-  HIP_TRY(hipHostMalloc((void**)&L.h_err, sizeof(int), hipHostMallocDefault));
-  HIP_TRY(hipHostMalloc((void**)&L.h_io, 8 * sizeof(uint64_t), hipHostMallocDefault));
+  // one pinned block: the decoder entry points' staging, the error flag (a
+  // cache line each), the token ids
+  HIP_TRY(hipHostMalloc((void**)&L.h_io, 128 + C * 4, hipHostMallocDefault));
+  L.h_err = reinterpret_cast<int*>(L.h_io + 8);
+  L.h_tokens = reinterpret_cast<uint32_t*>(L.h_io + 16);
   return lane_reserve(L, C);
 }
 
@@ -830,6 +859,19 @@ size_t max_input_width(const dtl_model* m) {
   if (m->c.ff > w) w = m->c.ff;
   if (m->c.heads * m->head_dim > w) w = m->c.heads * m->head_dim;
   return w;
+}
+
+// Sets up lanes 1 .. n - 1; how many of lanes 0 .. n - 1 there are (fewer
+// when memory is short).
+int ensure_lanes(dtl_session* s, int n) {
+  for (int li = 1; li < n; li++)
+    if (!s->lanes[li].stream && lane_init(s, s->lane_arena[li], s->lanes[li], s->max_chunk) != DTL_OK) {
+      (void)hipGetLastError();
+      s->lanes[li].release();
+      s->lane_arena[li].release();
+      return li;
+    }
+  return n;
 }
 
 // Sets up the wide lanes; false when there is no memory for them.
@@ -847,6 +889,67 @@ bool ensure_wide(dtl_session* s) {
     }
   s->wide_rows = rows;
   return true;
+}
+
+bool ensure_copy_out(dtl_session* s) {
+  if (s->out_pin) return true;
+  if (s->out_failed) return false;
+  bool ok = hipHostMalloc((void**)&s->out_pin, kCopyThreads * kCopySlice, hipHostMallocDefault) == hipSuccess;
+  for (hipEvent_t& e : s->out_ev) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+  if (ok) return true;
+  (void)hipGetLastError();
+  if (s->out_pin) (void)hipHostFree(s->out_pin);
+  s->out_pin = nullptr;
+  for (hipEvent_t& e : s->out_ev) {
+    if (e) (void)hipEventDestroy(e);
+    e = nullptr;
+  }
+  s->out_failed = true;
+  return false;
+}
+
+// Device results to the caller's (pageable) memory, on the lane's stream;
+// returns when they are there.  One copy of a large result runs at 8 GB/s
+// here: the runtime stages it and one thread touches every fresh page of the
+// destination (65 MB of logits, 512 positions of a 32000-token vocabulary:
+// about 8 ms).  From kCopyParallelBytes the slices are spread over up to
+// kCopyThreads host threads, thread t taking every t-th slice through its own
+// pinned buffer, so page faults and copies run side by side with the DMA of
+// other slices.  The threads end with the call.
+int copy_out(dtl_session* s, void* dst, const void* src, size_t bytes) {
+  hipStream_t st = s->ln->stream;
+  if (bytes < kCopyParallelBytes || !ensure_copy_out(s)) {
+    HIP_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipStreamSynchronize(st));
+    return DTL_OK;
+  }
+  const size_t slices = (bytes + kCopySlice - 1) / kCopySlice;
+  const int nt = slices < (size_t)kCopyThreads ? (int)slices : kCopyThreads;
+  const int device = s->m->device;
+  std::atomic<int> status{DTL_OK};
+  auto work = [&](int t) {
+    hipError_t e = hipSetDevice(device);
+    uint8_t* pin = s->out_pin + (size_t)t * kCopySlice;
+    for (size_t i = t; e == hipSuccess && i < slices; i += nt) {
+      const size_t off = i * kCopySlice, n = std::min(kCopySlice, bytes - off);
+      e = hipMemcpyAsync(pin, (const uint8_t*)src + off, n, hipMemcpyDeviceToHost, st);
+      if (e == hipSuccess) e = hipEventRecord(s->out_ev[t], st);
+      if (e == hipSuccess) e = hipEventSynchronize(s->out_ev[t]);
+      if (e == hipSuccess) std::memcpy((uint8_t*)dst + off, pin, n);
+    }
+    if (e != hipSuccess) status = hip_status(e);
+  };
+  std::vector<std::thread> threads;
+  int started = 1;  // slices of threads that could not be started are copied here
+  try {
+    threads.reserve(nt - 1);
+    for (; started < nt; started++) threads.emplace_back(work, started);
+  } catch (const std::exception&) {
+  }
+  work(0);
+  for (int t = started; t < nt; t++) work(t);
+  for (std::thread& t : threads) t.join();
+  return status;
 }
 
 int read_err(dtl_session* s, int* bits) {
@@ -1517,10 +1620,7 @@ int dtl_session_new(const dtl_model* m, size_t n_ctx, size_t max_chunk, dtl_sess
   ALLOC(pos_dev, 1);
 #undef ALLOC
   s->nlanes = lane_count();
-  for (int li = 0; li < s->nlanes; li++) {
-    Lane& L = s->lanes[li];
-    if ((st = lane_init(s.get(), A, L, C))) return st;
-  }
+  if ((st = lane_init(s.get(), s->lane_arena[0], s->lanes[0], C))) return st;  // the others: ensure_lanes
   HIP_TRY(hipHostMalloc((void**)&s->pos_host, sizeof(int), hipHostMallocDefault));
   HIP_TRY(hipMemsetAsync(s->kc, 0, kv * 4, s->ln->stream));
   HIP_TRY(hipMemsetAsync(s->vc, 0, kv * 4, s->ln->stream));
@@ -1556,12 +1656,7 @@ int dtl_forward_chunk(dtl_session* s, const uint32_t* tokens, size_t n, size_t p
   if (n == 0 || n > s->max_chunk) return DTL_ERR_SHAPE;
   int st = forward_device(s, tokens, (int)n, pos0);
   if (st) return st;
-  if (logits) {
-    HIP_TRY(hipMemcpyAsync(logits, s->ln->logits, n * s->m->vocab * sizeof(float),
-                           hipMemcpyDeviceToHost, s->ln->stream));
-    HIP_TRY(hipStreamSynchronize(s->ln->stream));
-  }
-  return DTL_OK;
+  return logits ? copy_out(s, logits, s->ln->logits, n * s->m->vocab * sizeof(float)) : DTL_OK;
 }
 
 int dtl_forward_one(dtl_session* s, uint32_t token, size_t pos, float* logits) {
@@ -1572,10 +1667,7 @@ int dtl_session_logits(dtl_session* s, size_t first, size_t n, float* out) {
   if (!s || !out) return DTL_ERR_INVALID_ARGUMENT;
   if (first + n > s->ln->rows_valid) return DTL_ERR_SHAPE;
   HIP_TRY(hipSetDevice(s->m->device));
-  HIP_TRY(hipMemcpyAsync(out, s->ln->logits + first * s->m->vocab, n * s->m->vocab * sizeof(float),
-                         hipMemcpyDeviceToHost, s->ln->stream));
-  HIP_TRY(hipStreamSynchronize(s->ln->stream));
-  return DTL_OK;
+  return copy_out(s, out, s->ln->logits + first * s->m->vocab, n * s->m->vocab * sizeof(float));
 }
 
 int dtl_logits_hash(const dtl_model* m, const uint32_t* tokens, size_t n, size_t chunk,
@@ -1694,8 +1786,10 @@ int dtl_forward_ranges(dtl_session* s, const uint32_t* tokens, size_t n, size_t 
   HIP_TRY(hipSetDevice(m->device));
   const bool wide = n > s->max_chunk && s->max_chunk < kEncodeRows && ensure_wide(s);
   Lane* const lanes = wide ? s->wide : s->lanes;
-  const int nl = wide ? std::min(kWideLanes, s->nlanes) : s->nlanes;
   const size_t C = wide ? s->wide_rows : s->max_chunk;  // positions (and symbols per CDF launch) of a lane
+  const size_t nchunks = (n + C - 1) / C;
+  int nl = (int)std::min((size_t)(wide ? std::min(kWideLanes, s->nlanes) : s->nlanes), nchunks);
+  if (!wide) nl = ensure_lanes(s, nl);
   // Back on lane 0 with every lane drained however this returns.
   struct Restore {
     dtl_session* s;
@@ -1728,7 +1822,6 @@ int dtl_forward_ranges(dtl_session* s, const uint32_t* tokens, size_t n, size_t 
     count[li] = 0;
     return DTL_OK;
   };
-  const size_t nchunks = (n + C - 1) / C;
   size_t k = 0;
   for (size_t c = 0; c < nchunks; c++) {
     const int li = (int)(c % nl);
@@ -1936,20 +2029,25 @@ int run_cdf_host(const float* logits, size_t n, size_t tail, int mode, uint32_t 
   Scratch sc;
   int st = sc.init();
   if (st) return st;
-  float* dl;
-  uint32_t *dsym, *dfreq, *dft = nullptr;
-  uint64_t *dcum, *dtot, *dct = nullptr;
-  if ((st = sc.arena.upload(&dl, logits, n))) return st;
-  if ((st = sc.arena.upload(&dsym, &symbol, 1))) return st;
-  if ((st = sc.arena.alloc(&dfreq, 1))) return st;
-  if ((st = sc.arena.alloc(&dcum, 1))) return st;
-  if ((st = sc.arena.alloc(&dtot, 1))) return st;
-  if (mode == 1) {
-    if ((st = sc.arena.alloc(&dft, n + tail))) return st;
-    if ((st = sc.arena.alloc(&dct, n + tail))) return st;
-  }
-  uint8_t* scratch;
-  if ((st = sc.arena.alloc(&scratch, cdf_scratch_bytes(1, (int)n)))) return st;
+  // one allocation for everything (each costs a call into the driver, and so
+  // does its release)
+  size_t at = 0;
+  auto take = [&](size_t bytes) {
+    const size_t o = at;
+    at += (bytes + 255) & ~(size_t)255;
+    return o;
+  };
+  const size_t o_l = take(n * 4), o_cum = take(8), o_tot = take(8), o_freq = take(4), o_sym = take(4);
+  const size_t o_ft = take(mode == 1 ? (n + tail) * 4 : 0), o_ct = take(mode == 1 ? (n + tail) * 8 : 0);
+  const size_t o_scr = take(cdf_scratch_bytes(1, (int)n));
+  uint8_t* base;
+  if ((st = sc.arena.alloc(&base, at))) return st;
+  float* dl = (float*)(base + o_l);
+  uint32_t *dsym = (uint32_t*)(base + o_sym), *dfreq = (uint32_t*)(base + o_freq), *dft = (uint32_t*)(base + o_ft);
+  uint64_t *dcum = (uint64_t*)(base + o_cum), *dtot = (uint64_t*)(base + o_tot), *dct = (uint64_t*)(base + o_ct);
+  uint8_t* scratch = base + o_scr;
+  HIP_TRY(hipMemcpyAsync(dl, logits, n * 4, hipMemcpyHostToDevice, sc.stream));
+  HIP_TRY(hipMemcpyAsync(dsym, &symbol, 4, hipMemcpyHostToDevice, sc.stream));
   if (mode == 1)
     launch_cdf_table(dl, (int)n, (int)tail, scratch, dft, dct, dtot, sc.err, sc.stream);
   else
