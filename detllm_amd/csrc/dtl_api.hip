@@ -1198,7 +1198,7 @@ int enqueue_forward(dtl_session* s, int T, size_t pos0, const int* pos_dev,
               "gemm_q8_qkv");
     } else {
       a = rms(L.attn_norm, {&L.wq, &L.wk, &L.wv});
-      if (L.wq.type == GGML_Q4_K && L.wk.type == GGML_Q4_K && L.wq.w32 && L.wk.w32 && T > kGemvMaxT &&
+      if (L.wq.type == GGML_Q4_K && L.wk.type == GGML_Q4_K && L.wq.w32 && L.wk.w32 && T > kQ4kGemvMaxT &&
           (L.bq != nullptr) == (L.bk != nullptr)) {
         // wq and wk share the input: one launch over their concatenated rows.
         double bytes = (double)(L.wq.rows + L.wk.rows) * L.wq.cols * weight_bytes_per_elem(GGML_Q4_K) +
@@ -1301,7 +1301,7 @@ int enqueue_forward(dtl_session* s, int T, size_t pos0, const int* pos_dev,
       q8_mats({&L.gate, &L.up}, true, a, {s->ln->ffo}, {}, {}, "gemm_q8_gate_up");
     } else {
       a = rms(L.ffn_norm, {&L.gate, &L.up});
-      if (T > kGemvMaxT && L.gate.type == GGML_Q4_K && L.up.type == GGML_Q4_K &&
+      if (T > (L.gate.w32 && L.up.w32 ? kQ4kGemvMaxT : kGemvMaxT) && L.gate.type == GGML_Q4_K && L.up.type == GGML_Q4_K &&
           L.gate.rows == L.up.rows && L.gate.cols == L.up.cols) {
         // gate, up and swiglu in one pass: both chains of a row share one wave.
         double bytes = 2.0 * L.gate.rows * L.gate.cols * weight_bytes_per_elem(GGML_Q4_K) +

@@ -208,6 +208,25 @@ bool launch_q8_mats(const DevMat* const* mats, int nm, bool pair, const DevAct& 
 // Positions up to which the decode GEMVs (one weight pass per position)
 // replace the chunked-encode GEMMs.
 constexpr int kGemvMaxT = 8;
+// Q4_K, where the chunk GEMMs have their f32 copy: the GEMV's chains of all
+// positions share three waves per workgroup, so its time grows with them (us
+// per forward of four TinyLlama-1.1B-shaped layers at 2 / 3 / 4 / 5 / 8
+// positions 471 / 705 / 945 / 1786 / 3070), the chunk GEMMs' does not (756 /
+// 774 / 783 / 783 / 784).  Up to 1024 rows the chunk GEMM has too few waves
+// and the GEMV stays for a fourth position (1024 x 2816 at 4 positions 22.8
+// against 33.2 us; four layers of that width 397 with this rule, 428 with
+// GEMVs alone, 446 with chunk GEMMs alone; at 5 / 8 positions GEMVs 579 / 824,
+// chunk GEMMs 468 / 475).
+constexpr int kQ4kGemvMaxT = 3;
+inline int q4k_gemv_max_t(const DevMat& W) {
+  return !W.w32 ? kGemvMaxT : kQ4kGemvMaxT + (W.rows <= 1024);
+}
+// Tall Q8_0 / Q4_0 matrices on their own (the output projection): from this
+// many outputs the chunk GEMM, which reads the weights once for all
+// positions (us, GEMV against chunk GEMM: 151936 x 896 at 2 / 4 / 8 positions
+// 45 / 86 / 169 against 30 / 30 / 31; 49152 x 576 15 / 27 / 50 against 12;
+// 32000 x 1024 Q4_0 10.1 / 16.1 / 28 against 12.0 / 10.9 / 10.9).
+constexpr long kQ8TileOutputs = 90000;
 
 // Matrices of one fused decode GEMV launch (same type, cols and input).
 struct FusedMats {
@@ -301,7 +320,7 @@ void launch_q6k_planes(const DevMat& W, int8_t* planes, hipStream_t s);
 // Fills out (rows * cols bytes) with the int8 values of W's Q4_0 blocks.
 void launch_q4_0_i8(const DevMat& W, int8_t* out, hipStream_t s);
 // Two Q4_K matrices with the same input and column count (wq, wk) in one
-// launch of more than kGemvMaxT positions, each with its own output, bias and
+// launch of more than kQ4kGemvMaxT positions, each with its own output, bias and
 // epilogue; false (nothing launched) when the pair does not qualify.
 bool launch_gemm_cat_q4k(const DevMat& W0, const DevMat& W1, const DevAct& A, int T, float* out0,
                          float* out1, const float* bias0, const float* bias1, int epi, int* err,

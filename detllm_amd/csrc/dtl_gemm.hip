@@ -707,9 +707,9 @@ __global__ void __launch_bounds__(256) k_q6k_mfma(const int8_t* __restrict__ pla
 // launch over concatenated rows; PAIR alternates the rows of gate and up
 // (tile row i is matrix i % 2, row i / 2) and writes silu(gate) * up.
 //
-// Workgroups are numbered so that the position tiles of one row tile run on
-// one XCD (workgroup n runs on XCD n % 8), whose L2 then serves the weights
-// to all but the first of them.
+// Workgroups are numbered row tile first.  Numbered so that the position
+// tiles of a row tile run on one XCD, for its L2, the launches took 1 to 2%
+// longer (output projection at 512 positions 452 against 442 us).
 namespace {
 // A weight scale (a finite f16) by the hardware's conversion, exact.
 __device__ __forceinline__ float half_to_f32(uint16_t h) { return (float)__builtin_bit_cast(_Float16, h); }
@@ -717,8 +717,7 @@ __device__ __forceinline__ float half_to_f32(uint16_t h) { return (float)__built
 
 template <int RW, int PW, int WR, int WP, bool V4, bool PAIR>
 __global__ void __launch_bounds__(64 * WR * WP) k_q8_tile(Q8Mats M, const int8_t* __restrict__ qa,
-                                                          const float* __restrict__ da, int T, int row_tiles,
-                                                          int pos_tiles, int* err) {
+                                                          const float* __restrict__ da, int T, int* err) {
   constexpr int NT = 64 * WR * WP, TR = 16 * RW * WR, TP = 16 * PW * WP;
   constexpr int KB = 128, LD = KB + 16;
   constexpr int NA = (TR * 8 + NT - 1) / NT, NB = (TP * 8 + NT - 1) / NT;  // 16-byte chunks per thread
@@ -727,9 +726,7 @@ __global__ void __launch_bounds__(64 * WR * WP) k_q8_tile(Q8Mats M, const int8_t
   __shared__ __align__(16) int8_t sa[2][TR * LD];
   __shared__ __align__(16) int8_t sb[2][TP * LD];
   __shared__ __align__(16) float ss[2][4][TR + TP];  // the rows' scales, then the positions'
-  const int loc = blockIdx.x >> 3;
-  const int rt = loc / pos_tiles * 8 + (blockIdx.x & 7), pt = loc % pos_tiles;
-  if (rt >= row_tiles) return;
+  const int rt = blockIdx.x, pt = blockIdx.y;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wr = wave / WP, wp = wave % WP;
@@ -976,7 +973,7 @@ __global__ void __launch_bounds__(64 * WR * WP) k_q8_tile(Q8Mats M, const int8_t
 
 // int8 copy of a Q4_0 matrix in element order (nibble - 8; det-quant
 // lib.rs:259-279: element i < 16 is the low nibble of byte i, element
-// i + 16 its high nibble), the A operand of k_q8_mfma.
+// i + 16 its high nibble), the A operand of k_q8_tile.
 __global__ void k_q4_0_i8(DevMat W, int8_t* out) {
   const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   const size_t total = (size_t)W.rows * W.cols;
@@ -1060,8 +1057,7 @@ void launch_q8_tile(const Q8Mats& M, const DevAct& A, int T, int* err, hipStream
   constexpr int TR = 16 * RW * WR, TP = 16 * PW * WP;
   const int rows = PAIR ? 2 * M.rows[0] : M.total_rows;
   const int rt = (rows + TR - 1) / TR, pt = (T + TP - 1) / TP;
-  launch_kernel((k_q8_tile<RW, PW, WR, WP, V4, PAIR>), dim3((rt + 7) / 8 * 8 * pt), dim3(64 * WR * WP), 0, s, M, A.qa,
-                A.da, T, rt, pt, err);
+  launch_kernel((k_q8_tile<RW, PW, WR, WP, V4, PAIR>), dim3(rt, pt), dim3(64 * WR * WP), 0, s, M, A.qa, A.da, T, err);
 }
 
 // The largest tile that still gives every CU two workgroups (one for 32 x
@@ -1070,7 +1066,7 @@ void launch_q8_tile(const Q8Mats& M, const DevAct& A, int T, int* err, hipStream
 // fills the chip, else 16.  us per launch, Qwen2.5-0.5B shape, against the
 // kernel without LDS staging that these replace (one to four position tiles
 // a wave, every operand straight from memory): output projection (151936 x
-// 896) 31 / 75 / 132 / 240 / 455 at 9 / 64 / 128 / 256 / 512 positions
+// 896) 31 / 73 / 129 / 234 / 442 at 9 / 64 / 128 / 256 / 512 positions
 // against 595 (one lane per row) / 157 / 291 / 566 / 1111; gate + up with
 // SwiGLU 49 at 512 against 2 x 49 + 8; wo and down on average 14 at 9, 19 at
 // 512.  Large launches run at about 0.36 of the 424 T multiply-adds/s that
@@ -1208,7 +1204,7 @@ void launch_gemm_pair_swiglu_q4k(const DevMat& G, const DevMat& U, const DevAct&
 bool launch_gemm_cat_q4k(const DevMat& W0, const DevMat& W1, const DevAct& A, int T, float* out0,
                          float* out1, const float* bias0, const float* bias1, int epi, int* err,
                          hipStream_t s) {
-  if (T <= kGemvMaxT || W0.type != kGgmlQ4K || W1.type != kGgmlQ4K || !W0.w32 || !W1.w32 ||
+  if (T <= kQ4kGemvMaxT || W0.type != kGgmlQ4K || W1.type != kGgmlQ4K || !W0.w32 || !W1.w32 ||
       W0.cols != W1.cols)
     return false;
   launch_q4k_f32w<MODE_CAT>(q4k_args(W0, &W1, A, T, out0, out1, nullptr, bias0, bias1, epi, err),

@@ -1947,7 +1947,7 @@ bool gemv_q4k_fit(const DevMat& W0, const DevMat* W1, bool pair, bool prologue, 
                   const DevMat* v6) {
   int RB, SL;
   size_t smem;
-  if (T > kGemvMaxT || W0.type != kGgmlQ4K) return false;
+  if (T > q4k_gemv_max_t(W0) || W0.type != kGgmlQ4K) return false;
   if (W1 && (W1->type != kGgmlQ4K || W1->cols != W0.cols || (pair && W1->rows != W0.rows)))
     return false;
   if (v6 && (!prologue || v6->type != kGgmlQ6K || v6->cols != W0.cols || v6->nb > 8)) return false;

@@ -103,6 +103,19 @@ def test_chunks_past_the_decode_gemvs_match_oracle(name, layers, n_tok, chunk):
     _compare_with_oracle(synth.build_model(w, layers=layers), synth.tokens(w, n_tok), chunk)
 
 
+@pytest.mark.parametrize("mirror", [True, False])
+@pytest.mark.parametrize("chunk", [3, 4, 8])
+def test_q4k_few_positions_match_oracle(monkeypatch, mirror, chunk):
+    # Q4_K chunks at the edge between the GEMV and the chunk GEMMs, and past
+    # it without the f32 copies (the GEMV then serves up to eight positions).
+    from detllm_amd import synth
+
+    if not mirror:
+        monkeypatch.setenv("DETLLM_NO_F32_MIRROR", "1")
+    w = synth.WORKLOADS["tinyllama"]
+    _compare_with_oracle(synth.build_model(w, layers=2), synth.tokens(w, chunk), chunk)
+
+
 @pytest.mark.parametrize("name,d,heads,kv_heads", [
     ("smollm2", 576, 36, 12),  # 16-wide heads
     ("qwen05", 448, 14, 2),    # 32, split-half RoPE, biases

@@ -117,6 +117,7 @@ def test_f32_rows_bitexact(rows, cols, T):
 @pytest.mark.parametrize("rows,cols,T", [
     (1, 32, 9), (70, 896, 13), (64, 128, 16), (129, 576, 16), (33, 160, 17), (65, 64, 32), (37, 256, 33),
     (40, 896, 70), (2050, 96, 129), (4099, 32, 511), (8200, 64, 512), (8195, 160, 449),
+    (45003, 64, 2), (11250, 160, 8), (11249, 96, 8),  # tall matrices of a few positions, and just too short
 ])
 @pytest.mark.parametrize("ggml_type", [8, 2])
 def test_int8_chunk_gemm_bitexact(ggml_type, rows, cols, T):
