@@ -1192,7 +1192,7 @@ int enqueue_forward(dtl_session* s, int T, size_t pos0, const int* pos_dev,
       a = rms(L.attn_norm, {});
       f32_mats({&L.wq, &L.wk, &L.wv}, false, a.x, {s->ln->q, s->ln->k, s->ln->v}, {L.bq, L.bk, L.bv},
                {e_q, e_k, e_v}, "gemm_f32_qkv");
-    } else if (T > kGemvMaxT && fits_q8({&L.wq, &L.wk, &L.wv}, false)) {
+    } else if (T > q8_gemv_max_t(L.wq) && fits_q8({&L.wq, &L.wk, &L.wv}, false)) {
       a = rms(L.attn_norm, {&L.wq});
       q8_mats({&L.wq, &L.wk, &L.wv}, false, a, {s->ln->q, s->ln->k, s->ln->v}, {L.bq, L.bk, L.bv}, {e_q, e_k, e_v},
               "gemm_q8_qkv");
@@ -1296,7 +1296,7 @@ int enqueue_forward(dtl_session* s, int T, size_t pos0, const int* pos_dev,
     } else if (fits_f32({&L.gate, &L.up}, true)) {
       a = rms(L.ffn_norm, {});
       f32_mats({&L.gate, &L.up}, true, a.x, {s->ln->ffo}, {}, {}, "gemm_f32_gate_up");
-    } else if (T > kGemvMaxT && fits_q8({&L.gate, &L.up}, true)) {
+    } else if (T > q8_gemv_max_t(L.gate) && fits_q8({&L.gate, &L.up}, true)) {
       a = rms(L.ffn_norm, {&L.gate});
       q8_mats({&L.gate, &L.up}, true, a, {s->ln->ffo}, {}, {}, "gemm_q8_gate_up");
     } else {

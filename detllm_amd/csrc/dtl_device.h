@@ -205,7 +205,7 @@ bool q8_mats_fit(const DevMat* const* mats, int nm, bool pair);
 bool launch_q8_mats(const DevMat* const* mats, int nm, bool pair, const DevAct& A, int T, float* const* outs,
                     const float* const* biases, const int* epis, int* err, hipStream_t s);
 
-// Positions up to which the decode GEMVs (one weight pass per position)
+// Positions up to which the decode GEMVs (one weight pass per position) can
 // replace the chunked-encode GEMMs.
 constexpr int kGemvMaxT = 8;
 // Q4_K, where the chunk GEMMs have their f32 copy: the GEMV's chains of all
@@ -220,6 +220,15 @@ constexpr int kGemvMaxT = 8;
 constexpr int kQ4kGemvMaxT = 3;
 inline int q4k_gemv_max_t(const DevMat& W) {
   return !W.w32 ? kGemvMaxT : kQ4kGemvMaxT + (W.rows <= 1024);
+}
+// Q8_0, and Q4_0 with its int8 copy (us per forward of four layers, GEMVs
+// against chunk GEMMs: 896 wide at 4 / 5 / 6 / 8 positions 227 / 265 / 293 /
+// 332 against 254 / 261 / 262 / 264; 1024 wide 228 / 275 / 311 / 331 against
+// 251 / 281 / 285 / 284; 576 wide 169 / 197 / 224 / 242 against 215 / 227 /
+// 231 / 232).
+constexpr int kQ8GemvMaxT = 5;
+inline int q8_gemv_max_t(const DevMat& W) {
+  return W.type == 8 /* Q8_0 */ || W.i8 ? kQ8GemvMaxT : kGemvMaxT;
 }
 // Tall Q8_0 / Q4_0 matrices on their own (the output projection): from this
 // many outputs the chunk GEMM, which reads the weights once for all

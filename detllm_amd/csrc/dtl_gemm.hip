@@ -491,6 +491,7 @@ void launch_dequant_q4k(const DevMat& W, float* out, hipStream_t s) {
 // K quarter l / 16 (16 bytes); result register i of lane l is row
 // 4 (l / 16) + i, position l % 16.
 typedef int dtl_v4i __attribute__((ext_vector_type(4)));
+typedef float dtl_v4f __attribute__((ext_vector_type(4)));
 
 __global__ void k_q6k_planes(DevMat W, int rows_pad, int8_t* planes) {
   const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -713,6 +714,22 @@ __global__ void __launch_bounds__(256) k_q6k_mfma(const int8_t* __restrict__ pla
 namespace {
 // A weight scale (a finite f16) by the hardware's conversion, exact.
 __device__ __forceinline__ float half_to_f32(uint16_t h) { return (float)__builtin_bit_cast(_Float16, h); }
+// The matrix and row of row tr of row tile rt (clamped to the last row; false
+// past it).
+template <bool PAIR, int TR>
+__device__ __forceinline__ bool q8_locate(const Q8Mats& M, int rt, int tr, int* mat, int* row) {
+  if (PAIR) {
+    const int r = rt * (TR / 2) + (tr >> 1);
+    *mat = tr & 1;
+    *row = r < M.rows[0] ? r : M.rows[0] - 1;
+    return r < M.rows[0];
+  }
+  const int g = rt * TR + tr;
+  const int gc = g < M.total_rows ? g : M.total_rows - 1;
+  *mat = (gc >= M.row_end[0] ? 1 : 0) + (gc >= M.row_end[1] ? 1 : 0);
+  *row = gc - (*mat == 0 ? 0 : (*mat == 1 ? M.row_end[0] : M.row_end[1]));
+  return g < M.total_rows;
+}
 }  // namespace
 
 template <int RW, int PW, int WR, int WP, bool V4, bool PAIR>
@@ -732,20 +749,7 @@ __global__ void __launch_bounds__(64 * WR * WP) k_q8_tile(Q8Mats M, const int8_t
   const int wr = wave / WP, wp = wave % WP;
   const int q = lane >> 4, li = lane & 15;
   const int nb = M.nb, cols = nb * 32;
-  // The matrix and row of tile row tr (clamped to the last row).
-  auto locate = [&](int tr, int* mat, int* row) -> bool {
-    if (PAIR) {
-      const int r = rt * (TR / 2) + (tr >> 1);
-      *mat = tr & 1;
-      *row = r < M.rows[0] ? r : M.rows[0] - 1;
-      return r < M.rows[0];
-    }
-    const int g = rt * TR + tr;
-    const int gc = g < M.total_rows ? g : M.total_rows - 1;
-    *mat = (gc >= M.row_end[0] ? 1 : 0) + (gc >= M.row_end[1] ? 1 : 0);
-    *row = gc - (*mat == 0 ? 0 : (*mat == 1 ? M.row_end[0] : M.row_end[1]));
-    return g < M.total_rows;
-  };
+  auto locate = [&](int tr, int* mat, int* row) -> bool { return q8_locate<PAIR, TR>(M, rt, tr, mat, row); };
   // Staging: chunk f = tid + k NT is byte column 16 (f % 8) of row f / 8.
   const int cc = 16 * (tid & 7);
   const int8_t* asrc[NA];
@@ -971,6 +975,135 @@ __global__ void __launch_bounds__(64 * WR * WP) k_q8_tile(Q8Mats M, const int8_t
   if (!ok) flag(err, ERRBIT_NON_FINITE);
 }
 
+// The same blocks for launches of few tiles, where k_q8_tile's waves walk K
+// alone on their SIMDs: a workgroup of W waves owns one tile of 16 rows x 16
+// positions and splits K.  Per round each wave forms the terms (dw * da) *
+// isum of its four blocks, its operands straight from memory, and leaves them
+// in LDS; then each of 256 threads adds the round's 4 W terms of its output in
+// block order.  Two rounds of loads are in flight; the terms are double
+// buffered, so a round has one barrier.
+template <int W, bool V4, bool PAIR>
+__global__ void __launch_bounds__(64 * W) k_q8_split(Q8Mats M, const int8_t* __restrict__ qa,
+                                                     const float* __restrict__ da, int T, int* err) {
+  constexpr int BR = 4 * W;  // blocks of a round
+  __shared__ __align__(16) float terms[2][BR][256];  // [block][position * 16 + row]
+  const int rt = blockIdx.x, pt = blockIdx.y;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int q = lane >> 4, li = lane & 15;
+  const int nb = M.nb, cols = nb * 32;
+  auto locate = [&](int tr, int* mat, int* row) -> bool { return q8_locate<PAIR, 16>(M, rt, tr, mat, row); };
+  int mat, row;
+  (void)locate(li, &mat, &row);
+  const int8_t* asrc = pick3(M.w, mat) + (size_t)row * cols;
+  const uint16_t* wsc[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    (void)locate(4 * q + i, &mat, &row);
+    wsc[i] = pick3(M.d16, mat) + (size_t)row * nb;
+  }
+  int p = pt * 16 + li;
+  p = p < T ? p : T - 1;
+  const int8_t* bsrc = qa + (size_t)p * cols;
+  const float* dsc = da + (size_t)p * nb;
+  struct Regs {
+    dtl_v4i a[2], b[2];
+    uint2 w[4];  // four f16 scales of each row
+    dtl_v4f d;
+  };
+  auto issue = [&](Regs& r, int s) {
+    const int b0 = (s * W + wave) * 4;
+#pragma unroll
+    for (int pp = 0; pp < 2; pp++) {
+      int col = b0 * 32 + 64 * pp + 16 * q;
+      col = col < cols ? col : 0;
+      r.a[pp] = *(const dtl_v4i*)(asrc + col);
+      r.b[pp] = *(const dtl_v4i*)(bsrc + col);
+    }
+    if constexpr (V4) {
+      const int b = b0 < nb ? b0 : 0;
+#pragma unroll
+      for (int i = 0; i < 4; i++) r.w[i] = *(const uint2*)(wsc[i] + b);
+      r.d = *(const dtl_v4f*)(dsc + b);
+    } else {
+      int b[4];
+#pragma unroll
+      for (int k = 0; k < 4; k++) b[k] = b0 + k < nb ? b0 + k : 0;
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        r.w[i].x = (uint32_t)wsc[i][b[0]] | ((uint32_t)wsc[i][b[1]] << 16);
+        r.w[i].y = (uint32_t)wsc[i][b[2]] | ((uint32_t)wsc[i][b[3]] << 16);
+      }
+#pragma unroll
+      for (int k = 0; k < 4; k++) r.d[k] = dsc[b[k]];
+    }
+  };
+  const dtl_v4i zero = {0, 0, 0, 0};
+  auto form = [&](const Regs& r, int buf, int s) {
+    const int b0 = (s * W + wave) * 4;
+    dtl_v4i acc[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const dtl_v4i bm = (q >> 1) == (k & 1) ? r.b[k >> 1] : zero;
+      acc[k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(r.a[k >> 1], bm, zero, 0, 0, 0);
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const float dv = b0 + k < nb ? r.d[k] : 0.0f;  // past the row: terms of +-0
+      dtl_v4f t;
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const uint32_t u = k < 2 ? r.w[i].x : r.w[i].y;
+        const float dw = half_to_f32((uint16_t)((k & 1) ? u >> 16 : u & 0xffffu));
+        t[i] = (dw * dv) * (float)acc[k][i];
+      }
+      *(dtl_v4f*)&terms[buf][4 * wave + k][li * 16 + 4 * q] = t;
+    }
+  };
+  const int ns = (nb + BR - 1) / BR;
+  Regs r[2];
+  issue(r[0], 0);
+  __builtin_amdgcn_sched_barrier(0);
+  issue(r[1], 1);
+  __builtin_amdgcn_sched_barrier(0);
+  // the thread's output: row tid % 16, position tid / 16
+  const int o = tid & 255;
+  const int pos = pt * 16 + (o >> 4);
+  const bool live = locate(o & 15, &mat, &row) && pos < T;
+  const int R = pick3(M.rows, mat), epi = pick3(M.epi, mat);
+  const size_t at = (size_t)(pos < T ? pos : T - 1) * R + row;
+  const float pre = PAIR ? 0.0f : epilogue_operand(pick3(M.out, mat), at, pick3(M.bias, mat), row, epi);
+  float sum = 0.0f;
+  for (int s0 = 0; s0 < ns; s0 += 2) {
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      if (s0 + u < ns) {
+        form(r[u], u, s0 + u);
+        issue(r[u], s0 + u + 2);
+        __syncthreads();
+        float t[BR];
+#pragma unroll
+        for (int k = 0; k < BR; k++) t[k] = terms[u][k][o];
+#pragma unroll
+        for (int k = 0; k < BR; k++) sum += t[k];
+      }
+    }
+  }
+  if (tid >= 256) return;
+  bool ok = true;
+  if constexpr (PAIR) {
+    const float other = __shfl_xor(sum, 1);
+    if (live && !(o & 1)) {
+      const float v = silu_det(sum) * other;
+      ok = finite(sum) && finite(other) && finite(v);
+      M.out[0][at] = v;
+    }
+  } else if (live) {
+    ok = store_epilogue_pre(sum, pre, pick3(M.out, mat), at, epi);
+  }
+  if (!ok) flag(err, ERRBIT_NON_FINITE);
+}
+
 // int8 copy of a Q4_0 matrix in element order (nibble - 8; det-quant
 // lib.rs:259-279: element i < 16 is the low nibble of byte i, element
 // i + 16 its high nibble), the A operand of k_q8_tile.
@@ -1060,13 +1193,22 @@ void launch_q8_tile(const Q8Mats& M, const DevAct& A, int T, int* err, hipStream
   launch_kernel((k_q8_tile<RW, PW, WR, WP, V4, PAIR>), dim3(rt, pt), dim3(64 * WR * WP), 0, s, M, A.qa, A.da, T, err);
 }
 
-// The largest tile that still gives every CU two workgroups (one for 32 x
+// Up to 300 tiles of 16 x 16 (512 where a row has 64 blocks or more) the
+// kernel that splits K.  us per launch, k_q8_split against k_q8_tile, 896 x
+// 896 and 896 x 4864 on average: 8.3 / 8.8 / 8.4 / 11.8 / 21.3 at 16 / 32 /
+// 64 / 128 / 256 positions (56 tiles each 16) against 13.7 / 15.1 / 15.0 /
+// 15.0 / 14.9; 1152 x 896 5.0 / 6.8 / 9.2 at 16 / 64 / 128 (72) against 6.7 /
+// 7.2 / 7.1; 960 x 576 5.8 / 7.7 at 64 / 128 (240, 480) against 7.5 / 7.8;
+// gate + up with SwiGLU 3072 x 576 5.5 at 16 (192) against 6.2, 9728 x 896
+// 9.8 (608) against 8.5.  Eight waves instead of four were never faster.
+//
+// Else the largest tile that still gives every CU two workgroups (one for 32 x
 // 64): a larger tile reads LDS less often per product, a smaller one spreads
 // a short launch.  Up to 16 positions one position tile, 64 rows where that
 // fills the chip, else 16.  us per launch, Qwen2.5-0.5B shape, against the
 // kernel without LDS staging that these replace (one to four position tiles
 // a wave, every operand straight from memory): output projection (151936 x
-// 896) 31 / 73 / 129 / 234 / 442 at 9 / 64 / 128 / 256 / 512 positions
+// 896) 30 / 70 / 126 / 233 / 444 at 9 / 64 / 128 / 256 / 512 positions
 // against 595 (one lane per row) / 157 / 291 / 566 / 1111; gate + up with
 // SwiGLU 49 at 512 against 2 x 49 + 8; wo and down on average 14 at 9, 19 at
 // 512.  Large launches run at about 0.36 of the 424 T multiply-adds/s that
@@ -1075,7 +1217,10 @@ template <bool V4, bool PAIR>
 void launch_q8_tiles(const Q8Mats& M, const DevAct& A, int T, int* err, hipStream_t s) {
   const int rows = PAIR ? 2 * M.rows[0] : M.total_rows;
   auto wgs = [&](int tr, int tp) { return (long)((rows + tr - 1) / tr) * ((T + tp - 1) / tp); };
-  if (T <= 16 && wgs(64, 16) >= 256) launch_q8_tile<1, 1, 4, 1, V4, PAIR>(M, A, T, err, s);
+  if (wgs(16, 16) <= (M.nb >= 64 ? 512 : 300))
+    launch_kernel((k_q8_split<4, V4, PAIR>), dim3((rows + 15) / 16, (T + 15) / 16), dim3(256), 0, s, M, A.qa, A.da, T,
+                  err);
+  else if (T <= 16 && wgs(64, 16) >= 256) launch_q8_tile<1, 1, 4, 1, V4, PAIR>(M, A, T, err, s);
   else if (T <= 16) launch_q8_tile<1, 1, 1, 1, V4, PAIR>(M, A, T, err, s);
   else if (wgs(128, 64) >= 512) launch_q8_tile<4, 2, 2, 2, V4, PAIR>(M, A, T, err, s);
   else if (wgs(64, 64) >= 512) launch_q8_tile<2, 2, 2, 2, V4, PAIR>(M, A, T, err, s);

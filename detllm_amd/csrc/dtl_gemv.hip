@@ -1880,9 +1880,9 @@ void launch_q8f(const FusedMats& M, const FusedIn& in, int T, int R, bool norm, 
 }  // namespace
 
 bool gemv_fused_fits(const DevMat* const* mats, int nm, bool pair_swiglu, bool norm, int T) {
-  if (nm < 1 || nm > 3 || (pair_swiglu && nm != 2) || T < 1 || T > kGemvMaxT) return false;
+  if (nm < 1 || nm > 3 || (pair_swiglu && nm != 2) || T < 1) return false;
   const DevMat& m0 = *mats[0];
-  if (m0.type != kGgmlQ8_0 && m0.type != kGgmlQ4_0) return false;
+  if ((m0.type != kGgmlQ8_0 && m0.type != kGgmlQ4_0) || T > q8_gemv_max_t(m0)) return false;
   for (int i = 0; i < nm; i++) {
     const DevMat& m = *mats[i];
     if (m.type != m0.type || m.cols != m0.cols || m.nb != m0.nb) return false;

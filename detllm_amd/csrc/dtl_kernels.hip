@@ -428,11 +428,11 @@ void launch_gemm(const DevMat& W, const DevAct& A, int T, float* out, const floa
   }
   // Up to kGemvMaxT positions a decode GEMV per position; beyond, the
   // kernels that decode the weights once for a tile of positions (Q6_K from
-  // two positions on, Q4_K and tall Q8_0 / Q4_0 matrices as their constants
-  // say).
+  // two positions on, Q4_K, Q8_0 and Q4_0 as their constants say).
   const bool q8 = W.type == kGgmlQ8_0 || W.type == kGgmlQ4_0;
   const bool chunk = (W.type == kGgmlQ6K && T >= 2) || (W.type == kGgmlQ4K && T > q4k_gemv_max_t(W)) ||
-                     (q8 && T >= 2 && (long)T * W.rows >= kQ8TileOutputs && gemm_tok_supported(W));
+                     (q8 && T >= 2 && (T > q8_gemv_max_t(W) || (long)T * W.rows >= kQ8TileOutputs) &&
+                      gemm_tok_supported(W));
   if (T <= kGemvMaxT && !chunk && launch_gemv(W, A, T, out, bias, epi, err, s)) return;
   if (gemm_tok_supported(W)) {
     launch_gemm_tok(W, A, T, out, bias, epi, err, s);

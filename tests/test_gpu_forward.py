@@ -103,6 +103,19 @@ def test_chunks_past_the_decode_gemvs_match_oracle(name, layers, n_tok, chunk):
     _compare_with_oracle(synth.build_model(w, layers=layers), synth.tokens(w, n_tok), chunk)
 
 
+@pytest.mark.parametrize("d,chunk", [(576, 5), (576, 6), (512, 7), (1024, 5), (1024, 6), (1024, 8)])
+def test_int8_few_positions_match_oracle(d, chunk):
+    # Q8_0 chunks at the edge between the GEMVs and the chunk GEMMs,
+    # block counts of a row that are and are not multiples of four, a gate and
+    # up pair of few rows (K split over the waves).
+    import dataclasses
+
+    from detllm_amd import synth
+
+    w = dataclasses.replace(synth.WORKLOADS["smollm2"], d=d, heads=d // 64, kv_heads=1, ff=736, vocab=300)
+    _compare_with_oracle(synth.build_model(w, layers=2), synth.tokens(w, 2 * chunk), chunk)
+
+
 @pytest.mark.parametrize("mirror", [True, False])
 @pytest.mark.parametrize("chunk", [3, 4, 8])
 def test_q4k_few_positions_match_oracle(monkeypatch, mirror, chunk):

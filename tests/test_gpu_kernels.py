@@ -113,10 +113,13 @@ def test_f32_rows_bitexact(rows, cols, T):
 # (rows, cols, T): every tile of the int8 chunk GEMM (64 x 16, 32 x 32, 32 x
 # 64, 64 x 64 and 128 x 64 rows x positions), partial tiles of each, one block
 # per row, block counts that are and are not multiples of four, an odd and an
-# even number of four-block stages.
+# even number of four-block stages; the kernel that splits K, with partial
+# tiles, one and several rounds, and both sides of its limits.
 @pytest.mark.parametrize("rows,cols,T", [
     (1, 32, 9), (70, 896, 13), (64, 128, 16), (129, 576, 16), (33, 160, 17), (65, 64, 32), (37, 256, 33),
     (40, 896, 70), (2050, 96, 129), (4099, 32, 511), (8200, 64, 512), (8195, 160, 449),
+    (5003, 160, 13), (2500, 96, 31), (4800, 192, 16), (4801, 192, 16),
+    (8192, 2048, 9), (8193, 2048, 9), (8192, 2016, 9), (130, 4864, 61), (17, 544, 10), (16, 1056, 7),
     (45003, 64, 2), (11250, 160, 8), (11249, 96, 8),  # tall matrices of a few positions, and just too short
 ])
 @pytest.mark.parametrize("ggml_type", [8, 2])
