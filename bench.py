@@ -27,7 +27,7 @@ import time
 from pathlib import Path
 
 # Eight hardware queues for this process (HIP's default is four), so that
-# each of the four streams of the pipelined encode gets its own; set before
+# each stream of the pipelined encode (up to four) gets its own; set before
 # anything initialises HIP.
 os.environ["GPU_MAX_HW_QUEUES"] = "8"
 
@@ -579,7 +579,7 @@ def main() -> int:
         roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                     "frac": round(achieved / HBM_PEAK_GBS, 4)}
     roofline["timed_over"] = ("one chunk-at-a-time step timing the dominant class alone (launches not "
-                              "overlapped); the timed steps run four chunks in flight")
+                              "overlapped); the timed steps run two chunks of 256 positions in flight")
     roofline.update({"kernel": dom_name, "avg_launch_us": round(avg_ms * 1e3, 2), "launches": dom["launches"],
                      "algorithmic_bytes_per_launch": per_launch_bytes,
                      "algorithmic_flops_per_launch": per_launch_flops})

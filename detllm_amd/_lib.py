@@ -33,8 +33,9 @@ def _load() -> C.CDLL:
     return C.CDLL(str(LIB_PATH))
 
 
-# With at least five hardware queues per process the pipelined encode keeps
-# four chunks in flight on four streams, else three (HIP's default is four
+# The pipelined encode keeps two chunks of 256 positions in flight; sessions
+# with a larger max_chunk keep up to four of those on four streams when the
+# process has at least five hardware queues, else three (HIP's default is four
 # queues).  Eight queues unless the caller chose otherwise; HIP reads the
 # setting when it initialises, i.e. at the library's first HIP call.
 os.environ.setdefault("GPU_MAX_HW_QUEUES", "8")
