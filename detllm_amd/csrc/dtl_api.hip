@@ -759,12 +759,15 @@ struct dtl_session {
                          // with the session, the others by the first call that
                          // needs them (ensure_lanes)
   Arena lane_arena[kMaxLanes];
-  // Lanes of kEncodeRows positions for the pipelined encode of sessions with
-  // a smaller max_chunk, set up by its first call with more tokens than that.
-  Arena wide_arena;
+  // Lanes of wide_rows positions (kEncodeRows, or the window if that is less)
+  // for the pipelined encode of sessions with a smaller max_chunk, set up by
+  // the first call that needs them; where there is no memory for one the
+  // session's own lanes serve.
+  Arena wide_arena[kWideLanes];
   Lane wide[kWideLanes];
-  size_t wide_rows = 0;  // positions per chunk there (0: not set up)
-  bool wide_failed = false;  // no memory for them: the session's own lanes serve
+  size_t wide_rows = 0;  // 0: none (DETLLM_NO_WIDE_LANES)
+  // Device bytes that lanes past the first may still take (DETLLM_LANE_MEMORY).
+  size_t lane_budget = SIZE_MAX;
   // Pinned slices and their events for large results (copy_out), set up by
   // the first such copy.
   uint8_t* out_pin = nullptr;
@@ -794,8 +797,10 @@ struct dtl_session {
 };
 
 // Sets up a lane for chunks of up to C positions: its stream, its events, its
-// device buffers (owned by A) and its pinned staging.
-static int lane_init(dtl_session* s, Arena& A, Lane& L, size_t C) {
+// device buffers (owned by A, of at most `budget` bytes) and its pinned staging.
+// For C positions the buffers take about C * (8 vocab + 4 heads n_ctx + 12 ff)
+// bytes: logits and the CDF's exps, attention scores, FFN rows.
+static int lane_init(dtl_session* s, Arena& A, Lane& L, size_t C, size_t budget) {
   const dtl_model* m = s->m;
   const HostConfig& c = m->c;
   const size_t hd = m->head_dim;
@@ -840,7 +845,9 @@ static int lane_init(dtl_session* s, Arena& A, Lane& L, size_t C) {
     ALLOC(c_scratch, cdf_scratch_bytes((int)C, (int)m->vocab));
     ALLOC(c_rows, C);
 #undef ALLOC
-    if (!base && (st = A.alloc(&base, at))) return st;
+    if (base) break;
+    if (at > budget) return DTL_ERR_OUT_OF_MEMORY;
+    if ((st = A.alloc(&base, at))) return st;
   }
   L.kv_ready.assign(c.block_count, nullptr);
   for (hipEvent_t& e : L.kv_ready) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
@@ -861,34 +868,21 @@ size_t max_input_width(const dtl_model* m) {
   return w;
 }
 
-// Sets up lanes 1 .. n - 1; how many of lanes 0 .. n - 1 there are (fewer
-// when memory is short).
-int ensure_lanes(dtl_session* s, int n) {
-  for (int li = 1; li < n; li++)
-    if (!s->lanes[li].stream && lane_init(s, s->lane_arena[li], s->lanes[li], s->max_chunk) != DTL_OK) {
+// Sets up those of lanes 0 .. n - 1 that a call needs and that are not there,
+// each with buffers of its own for `rows` positions; how many of them there are
+// (fewer when memory is short, or when the next would pass DETLLM_LANE_MEMORY).
+int ensure_lanes(dtl_session* s, Lane* lanes, Arena* arenas, int n, size_t rows) {
+  for (int li = 0; li < n; li++) {
+    if (lanes[li].stream) continue;
+    if (lane_init(s, arenas[li], lanes[li], rows, s->lane_budget) != DTL_OK) {
       (void)hipGetLastError();
-      s->lanes[li].release();
-      s->lane_arena[li].release();
+      lanes[li].release();
+      arenas[li].release();
       return li;
     }
+    if (s->lane_budget != SIZE_MAX) s->lane_budget -= arenas[li].bytes();
+  }
   return n;
-}
-
-// Sets up the wide lanes; false when there is no memory for them.
-bool ensure_wide(dtl_session* s) {
-  if (s->wide_rows) return true;
-  if (s->wide_failed) return false;
-  const size_t rows = kEncodeRows < s->n_ctx ? kEncodeRows : s->n_ctx;
-  for (Lane& L : s->wide)
-    if (lane_init(s, s->wide_arena, L, rows) != DTL_OK) {
-      (void)hipGetLastError();
-      for (Lane& W : s->wide) W.release();
-      s->wide_arena.release();
-      s->wide_failed = true;
-      return false;
-    }
-  s->wide_rows = rows;
-  return true;
 }
 
 bool ensure_copy_out(dtl_session* s) {
@@ -1620,7 +1614,9 @@ int dtl_session_new(const dtl_model* m, size_t n_ctx, size_t max_chunk, dtl_sess
   ALLOC(pos_dev, 1);
 #undef ALLOC
   s->nlanes = lane_count();
-  if ((st = lane_init(s.get(), s->lane_arena[0], s->lanes[0], C))) return st;  // the others: ensure_lanes
+  s->wide_rows = getenv("DETLLM_NO_WIDE_LANES") ? 0 : std::min(kEncodeRows, n_ctx);
+  if (const char* e = getenv("DETLLM_LANE_MEMORY")) s->lane_budget = (size_t)strtoull(e, nullptr, 10);
+  if ((st = lane_init(s.get(), s->lane_arena[0], s->lanes[0], C, SIZE_MAX))) return st;  // the others: ensure_lanes
   HIP_TRY(hipHostMalloc((void**)&s->pos_host, sizeof(int), hipHostMallocDefault));
   HIP_TRY(hipMemsetAsync(s->kc, 0, kv * 4, s->ln->stream));
   HIP_TRY(hipMemsetAsync(s->vc, 0, kv * 4, s->ln->stream));
@@ -1784,12 +1780,23 @@ int dtl_forward_ranges(dtl_session* s, const uint32_t* tokens, size_t n, size_t 
     if (symbols[i] >= V + tail) return DTL_ERR_CDF_SYMBOL_OUT_OF_RANGE;
   }
   HIP_TRY(hipSetDevice(m->device));
-  const bool wide = n > s->max_chunk && s->max_chunk < kEncodeRows && ensure_wide(s);
-  Lane* const lanes = wide ? s->wide : s->lanes;
-  const size_t C = wide ? s->wide_rows : s->max_chunk;  // positions (and symbols per CDF launch) of a lane
-  const size_t nchunks = (n + C - 1) / C;
-  int nl = (int)std::min((size_t)(wide ? std::min(kWideLanes, s->nlanes) : s->nlanes), nchunks);
-  if (!wide) nl = ensure_lanes(s, nl);
+  // Lanes: as many as the call has chunks, at most the session's count (two of
+  // the wide ones).
+  Lane* lanes = s->lanes;
+  size_t C = s->max_chunk, nchunks = 0;  // positions (and symbols per CDF launch) of a lane
+  int nl = 0;
+  if (s->wide_rows && n > s->max_chunk && s->max_chunk < kEncodeRows) {
+    lanes = s->wide;
+    C = s->wide_rows;
+    nchunks = (n + C - 1) / C;
+    nl = ensure_lanes(s, lanes, s->wide_arena, (int)std::min((size_t)std::min(kWideLanes, s->nlanes), nchunks), C);
+  }
+  if (nl == 0) {
+    lanes = s->lanes;
+    C = s->max_chunk;
+    nchunks = (n + C - 1) / C;
+    nl = ensure_lanes(s, lanes, s->lane_arena, (int)std::min((size_t)s->nlanes, nchunks), C);
+  }
   // Back on lane 0 with every lane drained however this returns.
   struct Restore {
     dtl_session* s;

@@ -131,7 +131,12 @@ int dtl_model_get_config(const dtl_model *model, dtl_model_config *out);
 /* F32Llama::forward_workspace + KvCache::new + RopeTables::llama
  * (det-model lib.rs:1244, 850, 813).  n_ctx <= context_length positions of
  * RoPE table and KV cache; max_chunk = most positions one dtl_forward_chunk
- * call may carry (1 for pure decode). */
+ * call may carry (1 for pure decode).
+ *
+ * Device memory: the KV cache (8 bytes per layer, KV head, position and head
+ * dimension) and one set of work buffers ("lane") for max_chunk positions, of
+ * about 8 vocab + 4 heads n_ctx + 18 max(embedding, FFN) + 32 embedding bytes
+ * per position.  dtl_forward_ranges adds lanes, which the session keeps. */
 int dtl_session_new(const dtl_model *model, size_t n_ctx, size_t max_chunk, dtl_session **out);
 void dtl_session_free(dtl_session *session);
 /* A fresh KvCache for window replay (det-cli main.rs:691-701). */
@@ -206,11 +211,19 @@ int dtl_symbol_ranges_rows(dtl_session *session, size_t n, const uint32_t *rows,
  * state.sync / symbol_range / advance), batched.  Forwards tokens[0..n) at
  * positions pos0.. in chunks (of 256 positions, or the session's max_chunk if
  * that is more) and codes symbols[i] against the logits of token rows[i]
- * (rows relative to pos0, non-decreasing, < n).  The same results as dtl_forward_chunk followed by
- * dtl_symbol_ranges_rows per chunk; two chunks (up to four of a larger
- * max_chunk) are in flight on streams of their own, whose buffers are set up
- * by the first call that needs them.  Afterwards no logits rows are valid
- * (dtl_session_logits and dtl_cdf need a new forward). */
+ * (rows relative to pos0, non-decreasing, < n).  The same results as
+ * dtl_forward_chunk followed by dtl_symbol_ranges_rows per chunk.  Afterwards
+ * no logits rows are valid (dtl_session_logits and dtl_cdf need a new forward).
+ *
+ * Two chunks (up to four of a larger max_chunk) are in flight on lanes of their
+ * own, which the first call that needs them sets up and the session keeps: for
+ * a max_chunk below 256, one of 256 positions by a call of more than max_chunk
+ * tokens and a second by one of more than 256 (a vocabulary of 151936: 360 MB
+ * each, against 90 MB for a lane of 64); otherwise one of max_chunk positions
+ * for each chunk past the first, up to three.  Where one does not fit, the call
+ * runs on those there are.  Environment, read by dtl_session_new: DETLLM_LANES
+ * (1-4) bounds the chunks in flight, DETLLM_LANE_MEMORY the bytes that the
+ * added lanes may take, DETLLM_NO_WIDE_LANES keeps chunks at max_chunk. */
 int dtl_forward_ranges(dtl_session *session, const uint32_t *tokens, size_t n, size_t pos0,
                        size_t n_sym, const uint32_t *rows, const uint32_t *symbols,
                        size_t tail_symbols, uint64_t *cum, uint32_t *freq, uint64_t *total);

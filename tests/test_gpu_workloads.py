@@ -99,7 +99,7 @@ def test_qwen05_decode_ranges_and_pipeline_match_golden():
             cum.append(c[0]), freq.append(f[0]), total.append(tt[0])
     assert h.hexdigest() == gold["logits_sha256"]
     assert _ranges_hash(cum, freq, total) == gold["next_token_ranges_sha256"]
-    print("qwen05: pipelined encode, chunks of 64", flush=True)
+    print("qwen05: pipelined encode, chunks of 256", flush=True)
     with Session(m, 2048, 64) as s:
         c, f, tt = s.forward_ranges(toks, 0, list(range(n)), nxt, 256)
     assert _ranges_hash(c, f, tt) == gold["next_token_ranges_sha256"]
@@ -109,8 +109,8 @@ def test_qwen05_decode_ranges_and_pipeline_match_golden():
 
 def test_tinyllama_encode_and_decode_match_golden(monkeypatch):
     """The benchmark's own workload end to end: the timed encode
-    (dtl_forward_ranges, chunks of 64 in flight on 4 lanes as the bench
-    runs it, and on 3) must code every one of the 2048 next tokens with the
+    (dtl_forward_ranges, chunks of 256 in flight on two lanes as the bench
+    runs it, and chunks of 64 on four) must code every one of the 2048 next tokens with the
     reference's (cum, freq, total), as det-cli's encode loop does
     (main.rs:521-551; cdf.rs:130-199).  Expected ranges: the golden's
     (the oracle's logits and symbol_range in the build container), and the
@@ -138,14 +138,17 @@ def test_tinyllama_encode_and_decode_match_golden(monkeypatch):
         assert [tuple(t) for t in gold["next_token_ranges"]] == want
     if "next_token_ranges_sha256" in gold:
         assert _ranges_hash(*zip(*want)) == gold["next_token_ranges_sha256"]
-    for lanes in ("4", "3"):
-        monkeypatch.setenv("DETLLM_LANES", lanes)  # read when the session is created
+    for lanes in ("two wide", "four 64-position"):
+        if lanes != "two wide":  # read when the session is created
+            monkeypatch.setenv("DETLLM_NO_WIDE_LANES", "1")
+            monkeypatch.setenv("DETLLM_LANES", "4")
         print(f"tinyllama: pipelined encode on {lanes} lanes", flush=True)
         with Session(m, 2048, 64) as s:
             c, f, tt = s.forward_ranges(toks, 0, list(range(n)), nxt, 256)
         got = [(int(a), int(b), int(d)) for a, b, d in zip(c, f, tt)]
         bad = [i for i in range(n) if got[i] != want[i]]
         assert not bad, f"{lanes} lanes: {len(bad)} rows differ, first {bad[0]}"
+    monkeypatch.delenv("DETLLM_NO_WIDE_LANES")
     monkeypatch.delenv("DETLLM_LANES")
     print("tinyllama: single-token decode", flush=True)
     _check_rows(_decode_rows(m, toks, 2048), gold, "decode")
