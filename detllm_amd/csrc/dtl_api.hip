@@ -717,13 +717,10 @@ struct Lane {
   // that their copies are plain DMA rather than staged pageable copies.
   uint64_t* h_io = nullptr;
 
-  // Drains the stream and frees everything but the device buffers (the
-  // arena's), leaving an empty lane.
+  // Drains the stream (the session's) and frees everything but the device
+  // buffers (the arena's), leaving an empty lane.
   void release() {
-    if (stream) {
-      (void)hipStreamSynchronize(stream);
-      (void)hipStreamDestroy(stream);
-    }
+    if (stream) (void)hipStreamSynchronize(stream);
     for (hipEvent_t e : kv_ready)
       if (e) (void)hipEventDestroy(e);
     for (void* p : {(void*)h_cum, (void*)h_io})
@@ -754,6 +751,14 @@ struct dtl_session {
   size_t n_ctx = 0, max_chunk = 0, max_in = 0;
   Arena arena;
   float *rope_cos = nullptr, *rope_sin = nullptr, *kc = nullptr, *vc = nullptr;
+  // Streams of the lanes (lane i's, and wide lane i's: the two kinds never run
+  // at once), created together with the session.  A stream takes the hardware
+  // queue that is least used when it is created.  Created by the first call that
+  // needed them, both streams of the second of three sessions were on one queue
+  // (kernel trace, four queues) and its chunks ran one after the other: encode of
+  // 1000 tokens with the Qwen2.5-0.5B shape by three sessions in turn 8.9 to 10.6
+  // ms a call, against 8.1 with one session or with streams created together.
+  hipStream_t streams[kMaxLanes] = {};
   Lane lanes[kMaxLanes];
   int nlanes = 1;        // lanes the pipelined encode may use; lane 0 is set up
                          // with the session, the others by the first call that
@@ -787,6 +792,8 @@ struct dtl_session {
   ~dtl_session() {
     for (Lane& L : lanes) L.release();
     for (Lane& L : wide) L.release();
+    for (hipStream_t q : streams)
+      if (q) (void)hipStreamDestroy(q);
     for (hipGraphExec_t g : graph)
       if (g) (void)hipGraphExecDestroy(g);
     if (pos_host) (void)hipHostFree(pos_host);
@@ -796,16 +803,16 @@ struct dtl_session {
   }
 };
 
-// Sets up a lane for chunks of up to C positions: its stream, its events, its
+// Sets up a lane on `stream` for chunks of up to C positions: its events, its
 // device buffers (owned by A, of at most `budget` bytes) and its pinned staging.
 // For C positions the buffers take about C * (8 vocab + 4 heads n_ctx + 12 ff)
 // bytes: logits and the CDF's exps, attention scores, FFN rows.
-static int lane_init(dtl_session* s, Arena& A, Lane& L, size_t C, size_t budget) {
+static int lane_init(dtl_session* s, Arena& A, Lane& L, hipStream_t stream, size_t C, size_t budget) {
   const dtl_model* m = s->m;
   const HostConfig& c = m->c;
   const size_t hd = m->head_dim;
   int st;
-  HIP_TRY(hipStreamCreateWithFlags(&L.stream, hipStreamNonBlocking));
+  L.stream = stream;
   // One device allocation, each buffer at a 256-byte boundary: first the
   // sizes, then the places.
   uint8_t* base = nullptr;
@@ -874,7 +881,7 @@ size_t max_input_width(const dtl_model* m) {
 int ensure_lanes(dtl_session* s, Lane* lanes, Arena* arenas, int n, size_t rows) {
   for (int li = 0; li < n; li++) {
     if (lanes[li].stream) continue;
-    if (lane_init(s, arenas[li], lanes[li], rows, s->lane_budget) != DTL_OK) {
+    if (lane_init(s, arenas[li], lanes[li], s->streams[li], rows, s->lane_budget) != DTL_OK) {
       (void)hipGetLastError();
       lanes[li].release();
       arenas[li].release();
@@ -1613,10 +1620,14 @@ int dtl_session_new(const dtl_model* m, size_t n_ctx, size_t max_chunk, dtl_sess
   ALLOC(vc, kv);
   ALLOC(pos_dev, 1);
 #undef ALLOC
-  s->nlanes = lane_count();
   s->wide_rows = getenv("DETLLM_NO_WIDE_LANES") ? 0 : std::min(kEncodeRows, n_ctx);
+  // as many lanes as a call can have chunks
+  const size_t chunk = std::max(C, s->wide_rows);
+  s->nlanes = (int)std::min((size_t)lane_count(), (n_ctx + chunk - 1) / chunk);
+  if (s->wide_rows > C) s->nlanes = std::min(s->nlanes, kWideLanes);
+  for (int li = 0; li < s->nlanes; li++) HIP_TRY(hipStreamCreateWithFlags(&s->streams[li], hipStreamNonBlocking));
   if (const char* e = getenv("DETLLM_LANE_MEMORY")) s->lane_budget = (size_t)strtoull(e, nullptr, 10);
-  if ((st = lane_init(s.get(), s->lane_arena[0], s->lanes[0], C, SIZE_MAX))) return st;  // the others: ensure_lanes
+  if ((st = lane_init(s.get(), s->lane_arena[0], s->lanes[0], s->streams[0], C, SIZE_MAX))) return st;  // the others: ensure_lanes
   HIP_TRY(hipHostMalloc((void**)&s->pos_host, sizeof(int), hipHostMallocDefault));
   HIP_TRY(hipMemsetAsync(s->kc, 0, kv * 4, s->ln->stream));
   HIP_TRY(hipMemsetAsync(s->vc, 0, kv * 4, s->ln->stream));
@@ -1780,16 +1791,15 @@ int dtl_forward_ranges(dtl_session* s, const uint32_t* tokens, size_t n, size_t 
     if (symbols[i] >= V + tail) return DTL_ERR_CDF_SYMBOL_OUT_OF_RANGE;
   }
   HIP_TRY(hipSetDevice(m->device));
-  // Lanes: as many as the call has chunks, at most the session's count (two of
-  // the wide ones).
+  // Lanes: as many as the call has chunks, at most the session's count.
   Lane* lanes = s->lanes;
   size_t C = s->max_chunk, nchunks = 0;  // positions (and symbols per CDF launch) of a lane
   int nl = 0;
-  if (s->wide_rows && n > s->max_chunk && s->max_chunk < kEncodeRows) {
+  if (n > s->max_chunk && s->wide_rows > s->max_chunk) {
     lanes = s->wide;
     C = s->wide_rows;
     nchunks = (n + C - 1) / C;
-    nl = ensure_lanes(s, lanes, s->wide_arena, (int)std::min((size_t)std::min(kWideLanes, s->nlanes), nchunks), C);
+    nl = ensure_lanes(s, lanes, s->wide_arena, (int)std::min((size_t)s->nlanes, nchunks), C);
   }
   if (nl == 0) {
     lanes = s->lanes;

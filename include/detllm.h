@@ -221,7 +221,8 @@ int dtl_symbol_ranges_rows(dtl_session *session, size_t n, const uint32_t *rows,
  * tokens and a second by one of more than 256 (a vocabulary of 151936: 360 MB
  * each, against 90 MB for a lane of 64); otherwise one of max_chunk positions
  * for each chunk past the first, up to three.  Where one does not fit, the call
- * runs on those there are.  Environment, read by dtl_session_new: DETLLM_LANES
+ * runs on those there are (at most two of max_chunk positions in place of the
+ * 256-position ones).  Environment, read by dtl_session_new: DETLLM_LANES
  * (1-4) bounds the chunks in flight, DETLLM_LANE_MEMORY the bytes that the
  * added lanes may take, DETLLM_NO_WIDE_LANES keeps chunks at max_chunk. */
 int dtl_forward_ranges(dtl_session *session, const uint32_t *tokens, size_t n, size_t pos0,
