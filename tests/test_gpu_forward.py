@@ -278,6 +278,29 @@ def test_single_position_graph_replay_matches_oracle(monkeypatch, name):
             assert np.array_equal(s.forward_one(tok, p).view(np.uint32), ref[p].view(np.uint32))
 
 
+@pytest.mark.parametrize("cores", [1, 2, 99])
+def test_large_logits_reach_the_host_whatever_the_cores(cores):
+    # Results of 2 MB and more by as many threads as the caller has cores; one
+    # core takes the single copy.  Rows on both sides of a slice's end.
+    import os
+
+    from detllm_amd import synth
+
+    w = synth.WORKLOADS["smollm2"]
+    m = _model(synth.build_model(w, layers=1))
+    toks = synth.tokens(w, 45)
+    mine = os.sched_getaffinity(0)
+    with m.forward_workspace(45, 45) as s:
+        s.forward_chunk(toks, 0)
+        want = np.concatenate([s.logits(i, 1) for i in range(45)])  # 197 KB each: one copy
+        try:
+            os.sched_setaffinity(0, set(sorted(mine)[:cores]))
+            for n in (11, 16, 17, 45):  # two slices and a part, three, three and a part, eight and a part
+                assert np.array_equal(s.logits(0, n).view(np.uint32), want[:n].view(np.uint32))
+        finally:
+            os.sched_setaffinity(0, mine)
+
+
 def test_repeat_runs_are_bitwise_identical():
     from detllm_amd import synth
 
