@@ -457,22 +457,24 @@ namespace {
 // Copies the chunked-encode GEMMs read instead of the GGUF blocks: the
 // exact f32 value of every Q4_K weight, the int8 matrix-core planes of
 // every Q6_K matrix and the int8 values of every Q4_0 matrix; and the
-// decode GEMV's layout of tall Q6_K matrices (the output projection).  DETLLM_NO_F32_MIRROR=1 keeps Q4_K packed only and
-// DETLLM_NO_Q6K_PLANES=1 keeps Q6_K packed only (the GEMMs then decode the
-// superblocks themselves; results are identical either way).
+// decode GEMV's layout of tall Q6_K matrices (the output projection).
+// DETLLM_NO_F32_MIRROR=1 keeps Q4_K packed only, DETLLM_NO_Q6K_PLANES=1 Q6_K
+// and DETLLM_NO_Q4_0_INT8=1 Q4_0, as a device without room does (the GEMMs then
+// decode the blocks themselves; results are identical either way).
 bool env_flag(const char* name) {
   const char* v = getenv(name);
   return v && *v && *v != '0';
 }
 bool f32_mirror_enabled() { return !env_flag("DETLLM_NO_F32_MIRROR"); }
 bool q6k_planes_enabled() { return !env_flag("DETLLM_NO_Q6K_PLANES"); }
+bool q4_0_int8_enabled() { return !env_flag("DETLLM_NO_Q4_0_INT8"); }
 
 int build_encode_copies(dtl_model* m) {
   std::vector<DevMat*> q4k, q6k, q40, q6d;
   auto add = [&](DevMat* M) {
     if (M->type == GGML_Q4_K && f32_mirror_enabled()) q4k.push_back(M);
     if (M->type == GGML_Q6_K && q6k_planes_enabled()) q6k.push_back(M);
-    if (M->type == GGML_Q4_0) q40.push_back(M);
+    if (M->type == GGML_Q4_0 && q4_0_int8_enabled()) q40.push_back(M);
     if (M->type == GGML_Q6_K && q6k_decode_layout_applies(*M)) q6d.push_back(M);
   };
   for (Layer& L : m->layers)
@@ -1633,7 +1635,7 @@ int dtl_session_new(const dtl_model* m, size_t n_ctx, size_t max_chunk, dtl_sess
   ALLOC(vc, kv);
   ALLOC(pos_dev, 1);
 #undef ALLOC
-  s->wide_rows = getenv("DETLLM_NO_WIDE_LANES") ? 0 : std::min(kEncodeRows, n_ctx);
+  s->wide_rows = env_flag("DETLLM_NO_WIDE_LANES") ? 0 : std::min(kEncodeRows, n_ctx);
   // as many lanes as a call can have chunks
   const size_t chunk = std::max(C, s->wide_rows);
   s->nlanes = (int)std::min((size_t)lane_count(), (n_ctx + chunk - 1) / chunk);
@@ -2457,7 +2459,7 @@ int upload_raw_matrix(Scratch& sc, int ggml_type, const uint8_t* weights, size_t
     launch_q6k_planes(W, planes, sc.stream);
     W.planes = planes;
   }
-  if (W.type == GGML_Q4_0) {
+  if (W.type == GGML_Q4_0 && q4_0_int8_enabled()) {
     int8_t* i8;
     if ((st = sc.arena.alloc(&i8, rows * cols))) return st;
     launch_q4_0_i8(W, i8, sc.stream);

@@ -86,24 +86,8 @@ __device__ float row_dot_f32(const float* w, const float* x, int n) {
   return finish_8lane(acc);
 }
 
-// dot_q8_0_q8a (det-quant lib.rs:237-257): exact i32 per block, then
+// dot_q4_0_q8a (det-quant lib.rs:259-279, 492-504): exact i32 per block, then
 // (dw*da)*isum added in block order.
-__device__ float row_dot_q8_0(const int8_t* wq, const uint16_t* wd, const int8_t* aq,
-                              const float* ad, int nb) {
-  float sum = 0.0f;
-  const int* w4 = (const int*)wq;
-  const int* a4 = (const int*)aq;
-  for (int b = 0; b < nb; b++) {
-    int isum = 0;
-#pragma unroll
-    for (int k = 0; k < 8; k++) isum = __builtin_amdgcn_sdot4(w4[b * 8 + k], a4[b * 8 + k], isum, false);
-    float scale = f16_to_f32(wd[b]) * ad[b];
-    sum += scale * (float)isum;
-  }
-  return sum;
-}
-
-// dot_q4_0_q8a (lib.rs:259-279, 492-504)
 __device__ float row_dot_q4_0(const uint8_t* wq, const uint16_t* wd, const int8_t* aq,
                               const float* ad, int nb) {
   float sum = 0.0f;
@@ -119,51 +103,6 @@ __device__ float row_dot_q4_0(const uint8_t* wq, const uint16_t* wd, const int8_
     float scale = f16_to_f32(wd[b]) * ad[b];
     sum += scale * (float)isum;
   }
-  return sum;
-}
-
-// dot_q4_k_q8a (lib.rs:281-315): one sequential chain over the whole row,
-// weight = (d*sc)*q - dmin*m, activation = da*qa, sum += weight*activation.
-__device__ float row_dot_q4k(const uint8_t* qs, const uint8_t* hdr, const float* af, int nsb) {
-  float sum = 0.0f;
-  for (int sb = 0; sb < nsb; sb++) {
-    const uint8_t* h = hdr + sb * 16;
-    float d = f16_to_f32(ld_u16(h)), dmin = f16_to_f32(ld_u16(h + 2));
-    for (int sub = 0; sub < 8; sub++) {
-      int sc, mn;
-      q4k_scale_min(h + 4, sub, &sc, &mn);
-      float dsc = d * (float)sc, dm = dmin * (float)mn;
-      const uint8_t* q = qs + sb * 128 + (sub / 2) * 32;
-      const float* a = af + sb * 256 + sub * 32;
-      int shift = (sub & 1) * 4;
-      for (int w = 0; w < 32; w++) {
-        float weight = dsc * (float)((q[w] >> shift) & 0x0f) - dm;
-        sum += weight * a[w];
-      }
-    }
-  }
-  return sum;
-}
-
-// dot_q6_k_q8k (lib.rs:353-397): exact i32 lane sums (lane = index mod 8)
-// per superblock, f32 lane accumulators, sequential lane combine from 0.0.
-__device__ float row_dot_q6k(const uint8_t* body, const uint16_t* wd, const int8_t* qk,
-                             const float* dk, int nsb) {
-  float sums[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  for (int sb = 0; sb < nsb; sb++) {
-    const uint8_t* b = body + (size_t)sb * 208;
-    const int8_t* a = qk + sb * 256;
-    int aux[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    // Q8_K quants are stored class-major: element e sits at (e % 8) * 32 + e / 8.
-    for (int e = 0; e < 256; e++)
-      aux[e & 7] += q6k_scale(b, e) * (int)a[(e & 7) * 32 + (e >> 3)] * q6k_quant(b, e);
-    float d = f16_to_f32(wd[sb]) * dk[sb];
-#pragma unroll
-    for (int l = 0; l < 8; l++) sums[l] += d * (float)aux[l];
-  }
-  float sum = 0.0f;
-#pragma unroll
-  for (int l = 0; l < 8; l++) sum += sums[l];
   return sum;
 }
 
@@ -381,34 +320,20 @@ void launch_rmsnorm(const float* x, const float* w, float eps, int T, int n, flo
 // ---------------------------------------------------------------------------
 // GEMM: out[t][r] = row r . activation t, one lane per (r, t), with the
 // bias add (add_optional_bias, lib.rs:1982-1998) or residual add
-// (residual_add, lib.rs:1967-1980) applied to the finished dot.
+// (residual_add, lib.rs:1967-1980) applied to the finished dot.  For what no
+// other kernel takes: F32 rows whose width is not a multiple of four, and more
+// than kGemvMaxT positions of Q4_0 without its int8 copy.
 __global__ void __launch_bounds__(256) k_gemm_rowlane(DevMat W, DevAct A, int T, float* out,
                                                       const float* bias, int epi, int* err) {
   int r = blockIdx.x * blockDim.x + threadIdx.x;
   int t = blockIdx.y;
   if (r >= W.rows || t >= T) return;
   float v;
-  switch (W.type) {
-    case kGgmlF32:
-      v = row_dot_f32((const float*)W.w + (size_t)r * W.cols, A.x + (size_t)t * W.cols, W.cols);
-      break;
-    case kGgmlQ8_0:
-      v = row_dot_q8_0((const int8_t*)W.w + (size_t)r * W.cols, W.d16 + (size_t)r * W.nb,
-                       A.qa + (size_t)t * W.cols, A.da + (size_t)t * (W.cols / 32), W.nb);
-      break;
-    case kGgmlQ4_0:
-      v = row_dot_q4_0((const uint8_t*)W.w + (size_t)r * W.nb * 16, W.d16 + (size_t)r * W.nb,
-                       A.qa + (size_t)t * W.cols, A.da + (size_t)t * (W.cols / 32), W.nb);
-      break;
-    case kGgmlQ4K:
-      v = row_dot_q4k((const uint8_t*)W.w + (size_t)r * W.nb * 128, W.hdr + (size_t)r * W.nb * 16,
-                      A.af + (size_t)t * W.cols, W.nb);
-      break;
-    default:
-      v = row_dot_q6k((const uint8_t*)W.w + (size_t)r * W.nb * 208, W.d16 + (size_t)r * W.nb,
-                      A.qk + (size_t)t * W.cols, A.dk + (size_t)t * (W.cols / 256), W.nb);
-      break;
-  }
+  if (W.type == kGgmlF32)
+    v = row_dot_f32((const float*)W.w + (size_t)r * W.cols, A.x + (size_t)t * W.cols, W.cols);
+  else
+    v = row_dot_q4_0((const uint8_t*)W.w + (size_t)r * W.nb * 16, W.d16 + (size_t)r * W.nb,
+                     A.qa + (size_t)t * W.cols, A.da + (size_t)t * (W.cols / 32), W.nb);
   bool bad = !finite(v);
   size_t o = (size_t)t * W.rows + r;
   if (epi == EPI_BIAS) {

@@ -84,11 +84,13 @@ def test_exp_clamped_device_matches_oracle():
     assert L.lib.dtl_kernel_exp_clamped_f32(_p(y, C.c_float), _p(out, C.c_float), 2) == 42
 
 
-@pytest.mark.parametrize("rows,cols", [(1, 4), (8, 64), (33, 100), (40, 576), (65, 68), (192, 1028), (16389, 32)])
-@pytest.mark.parametrize("T", [1, 2, 3, 5, 8, 9, 15, 31, 33, 70])
+@pytest.mark.parametrize("rows,cols", [(1, 4), (8, 64), (33, 100), (40, 576), (65, 68), (192, 1028), (16389, 32),
+                                       (1, 1), (33, 30), (300, 33)])
+@pytest.mark.parametrize("T", [1, 2, 3, 4, 5, 8, 9, 15, 31, 33, 70])
 def test_f32_rows_bitexact(rows, cols, T):
-    # The F32 GEMV (up to eight positions) and the matrix-core products (more):
-    # partial row groups, position tiles and column slices, bit for bit.
+    # The F32 GEMV (up to four positions) and the matrix-core products (more):
+    # partial row groups, position tiles and column slices, bit for bit; and
+    # one lane per row for widths that are not a multiple of four.
     L = _lib()
     rng = np.random.default_rng(rows * 131 + cols + T)
     w = rng.normal(0, 0.1, (rows, cols)).astype(np.float32)
@@ -253,10 +255,11 @@ def test_rmsnorm_bitexact():
             assert np.array_equal(out[r].view(np.uint32), detref.rmsnorm(x[r], w, eps).view(np.uint32))
 
 
-# (type, rows, cols, positions): T <= 8 runs the decode GEMVs (rows per wave
-# grows with the row count: Q8_0/Q4_0 1/2/4/8, Q6_K 64/nsb, Q4_K 8/32),
-# T >= 16 the token-parallel GEMMs (Q8_0 / Q4_0 / Q6_K on the matrix
-# cores), T in between the row-lane kernel.
+# (type, rows, cols, positions): the decode GEMVs up to five positions of Q8_0
+# and Q4_0, three (or four, up to 1024 rows) of Q4_K and one of Q6_K (rows per
+# wave grows with the row count: Q8_0/Q4_0 1/2/4/8, Q6_K 64/nsb, Q4_K 8/32),
+# the chunk GEMMs beyond (Q8_0 / Q4_0 / Q6_K on the int8 matrix cores, Q4_K
+# from its f32 copy) and for two and more positions of tall Q8_0 and Q4_0.
 GEMV_CASES = [
     (0, 37, 64, 3), (0, 20, 128, 1),
     (8, 61, 576, 1), (8, 33, 896, 5), (8, 9, 4864, 2), (8, 5000, 64, 1), (8, 17000, 64, 2),
@@ -271,11 +274,10 @@ GEMV_CASES = [
     # Q4_K chunk GEMMs: partial row and position tiles, one and several
     # slices per superblock, the ffn_down width
     (12, 17, 2048, 16), (12, 130, 1024, 33), (12, 48, 5632, 64), (12, 1, 256, 17),
-    # 8 positions x 5632 columns: the split decode kernel's LDS does not hold
-    # the activations, so the one-lane-per-row Q4_K kernel serves it
+    # 8 positions x 5632 columns: more than the decode kernel's LDS holds
     (12, 20, 5632, 8),
     (14, 50, 2048, 1), (14, 9, 5632, 2), (14, 20, 512, 64), (14, 300, 256, 1), (14, 33, 4096, 1),
-    # Q6_K decode at full TinyLlama ffn_down size (T = 8), odd row counts, and
+    # Q6_K at full TinyLlama ffn_down size (T = 8), odd row counts, and
     # a 16384-row matrix (the split-superblock kernel's largest)
     (14, 2048, 5632, 8), (14, 1000, 5632, 3), (14, 2049, 5632, 1), (14, 16384, 2048, 1),
     # tall Q6_K on the decode layout (k_gemv_q6k_cm): the TinyLlama output
@@ -283,8 +285,8 @@ GEMV_CASES = [
     # partial last groups and several positions
     (14, 32000, 2048, 1), (14, 16385, 256, 3), (14, 17000, 512, 1), (14, 20001, 1024, 2),
     (14, 16400, 4096, 1), (14, 16390, 8192, 2), (14, 16401, 256, 1), (14, 8, 16384, 1),
-    # Q8_0 / Q4_0 on the int8 matrix cores (T >= 16): odd block counts (a
-    # half block pair), row tiles of 16 / 32 / 64, partial position tiles
+    # Q8_0 / Q4_0 on the int8 matrix cores, 16 positions and more: odd block
+    # counts, partial row and position tiles
     (8, 40, 32, 16), (8, 37, 96, 33), (8, 2100, 160, 17), (8, 8200, 64, 16), (8, 100, 896, 64),
     (8, 64, 576, 100), (2, 40, 64, 16), (2, 33, 96, 70), (2, 2050, 64, 16),
 ]
@@ -305,6 +307,18 @@ def test_gemv_bitexact_against_oracle(ggml_type, rows, cols, T):
         want = np.array([detref.dot_row(ggml_type, w[r * rb:(r + 1) * rb], cols, x[t]) for r in range(rows)],
                         np.float32)
         assert np.array_equal(out[t].view(np.uint32), want.view(np.uint32)), (t,)
+
+
+@pytest.mark.parametrize("ggml_type,rows,cols,T,env", [
+    # without the copies that the chunk GEMMs read, as on a device without room
+    (2, 70, 96, 8, "DETLLM_NO_Q4_0_INT8"), (2, 70, 96, 9, "DETLLM_NO_Q4_0_INT8"),
+    (2, 300, 512, 40, "DETLLM_NO_Q4_0_INT8"),
+    (12, 20, 5632, 8, "DETLLM_NO_F32_MIRROR"), (12, 45, 512, 8, "DETLLM_NO_F32_MIRROR"),
+    (12, 45, 512, 9, "DETLLM_NO_F32_MIRROR"), (14, 45, 512, 9, "DETLLM_NO_Q6K_PLANES"),
+])
+def test_gemm_without_copies_bitexact_against_oracle(monkeypatch, ggml_type, rows, cols, T, env):
+    monkeypatch.setenv(env, "1")
+    test_gemv_bitexact_against_oracle(ggml_type, rows, cols, T)
 
 
 # (mode, overlapped, rows0, rows1, cols, T): the Q4_K chunk GEMMs of the
