@@ -80,10 +80,10 @@ def test_baseline_shapes_match_oracle(name, layers, n_tok, chunk):
     ("qwen05", 14, 2),   # biases on the concatenated q/k/v launch
     ("smollm2", 18, 6),  # 32-wide heads
 ])
-@pytest.mark.parametrize("chunk", [1, 3, 8, 13, 34])
+@pytest.mark.parametrize("chunk", [1, 3, 4, 8, 13, 34])
 def test_f32_model_matches_oracle(name, heads, kv_heads, chunk):
     # F32 weights: q/k/v and gate/up/SwiGLU in one launch each, by GEMV up to
-    # eight positions and on the matrix cores beyond.
+    # four positions and on the matrix cores beyond.
     import dataclasses
 
     from detllm_amd import synth
@@ -198,6 +198,93 @@ def test_chunk_attention_head_widths_match_oracle(name, d, heads, kv_heads, chun
             p += n
 
 
+@pytest.mark.parametrize("name,d,heads,kv_heads,ctx", [
+    ("smollm2", 64, 8, 4, 200),     # widths that only the general kernels take: 8
+    ("qwen05", 192, 8, 2, 200),     # 24, split-half RoPE, biases
+    ("smollm2", 384, 8, 2, 200),    # 48, one workgroup per group of heads
+    ("smollm2", 384, 8, 2, 9000),   # 48, a score row per wave in memory (no room in LDS)
+    ("smollm2", 864, 18, 1, 200),   # 48, more than sixteen heads per group
+    ("smollm2", 448, 4, 2, 200),    # 112
+    ("qwen05", 512, 2, 1, 200),     # 256
+    ("smollm2", 576, 2, 1, 200),    # 288, past the one-workgroup kernel's width
+    ("smollm2", 832, 13, 1, 200),   # 64, nine to sixteen heads per group
+    ("smollm2", 1152, 18, 1, 200),  # 64, more: the matrix-core launches
+])
+def test_attention_of_other_head_shapes_matches_oracle(name, d, heads, kv_heads, ctx):
+    import dataclasses
+
+    from detllm_amd import synth
+
+    w = dataclasses.replace(synth.WORKLOADS[name], d=d, heads=heads, kv_heads=kv_heads, ff=64, vocab=300, ctx=ctx)
+    data = synth.build_model(w, layers=2)
+    steps = (1, 5, 1, 33, 4, 70, 1, 3)
+    toks = [int(t) for t in synth.tokens(w, sum(steps))]
+    ref = detref.Model(data).logits(toks)
+    with _model(data).forward_workspace(ctx, 70) as s:
+        p = 0
+        for n in steps:
+            got = s.forward_chunk(toks[p:p + n], p, want_logits=True)
+            bad = np.nonzero(got.view(np.uint32) != ref[p:p + n].view(np.uint32))
+            assert bad[0].size == 0, (p, n, bad[0][:1], bad[1][:1])
+            p += n
+
+
+@pytest.mark.parametrize("d,heads,layers,prefix,chunks", [
+    (256, 2, 2, 1485, (33, 70)),    # 128-wide heads
+    (192, 2, 2, 700, (5, 130)),     # 96
+    (160, 2, 2, 700, (64, 17)),     # 80
+    (32, 2, 2, 2045, (6, 100)),     # 16
+    (1024, 16, 1, 1760, (20, 13, 30)),  # 64, sixteen heads per group: to and past the one-launch kernel's LDS
+])
+def test_chunk_attention_long_rows_match_oracle(d, heads, layers, prefix, chunks):
+    # Chunk attention far into a window: every position of the chunks is
+    # compared, and with two layers the prefix's own attention reaches them.
+    import dataclasses
+
+    from detllm_amd import synth
+
+    n = prefix + sum(chunks)
+    w = dataclasses.replace(synth.WORKLOADS["smollm2"], d=d, heads=heads, kv_heads=1, ff=64, vocab=300, ctx=n)
+    data = synth.build_model(w, layers=layers)
+    toks = [int(t) for t in synth.tokens(w, n)]
+    ref = detref.Model(data).logits(toks)
+    with _model(data).forward_workspace(n, 256) as s:
+        for p in range(0, prefix, 256):
+            s.forward_chunk(toks[p:min(prefix, p + 256)], p)
+        p = prefix
+        for c in chunks:
+            got = s.forward_chunk(toks[p:p + c], p, want_logits=True)
+            bad = np.nonzero(got.view(np.uint32) != ref[p:p + c].view(np.uint32))
+            assert bad[0].size == 0, (p, c, bad[0][:1], bad[1][:1])
+            p += c
+
+
+@pytest.mark.parametrize("d,heads,prefix,chunks", [
+    (512, 8, 4205, (8, 13, 30)),   # 64-wide heads, eight per group: to and past the one-launch kernel's LDS
+    (32, 2, 19100, (55, 25, 40)),  # 16-wide: past the softmax launch's LDS (about 19170 keys)
+])
+def test_chunk_attention_of_very_long_rows_equals_decode(d, heads, prefix, chunks):
+    # Rows too long for the oracle: the chunks' logits against those of single
+    # positions, whose attention the tests above compare with the oracle.
+    import dataclasses
+
+    from detllm_amd import synth
+
+    n = prefix + sum(chunks)
+    w = dataclasses.replace(synth.WORKLOADS["smollm2"], d=d, heads=heads, kv_heads=1, ff=64, vocab=300, ctx=n)
+    toks = [int(t) for t in synth.tokens(w, n)]
+    with _model(synth.build_model(w, layers=2)).forward_workspace(n, 512) as s:
+        for p in range(0, prefix, 512):
+            s.forward_chunk(toks[p:min(prefix, p + 512)], p)
+        p = prefix
+        for c in chunks:
+            got = s.forward_chunk(toks[p:p + c], p, want_logits=True)
+            for i in range(c):
+                one = s.forward_one(toks[p + i], p + i)
+                assert np.array_equal(got[i].view(np.uint32), one.view(np.uint32)), p + i
+            p += c
+
+
 def test_decode_attention_long_row_matches_oracle():
     # The Z chains run in segments of 8192 exps: rows just below, at and past one.
     import dataclasses
@@ -218,10 +305,10 @@ def test_decode_attention_long_row_matches_oracle():
             assert np.array_equal(got.view(np.uint32), ref[p:p + n].view(np.uint32)), (p, n)
 
 
-@pytest.mark.parametrize("name,chunk", [("qwen05", 1), ("qwen05", 8), ("smollm2", 5)])
+@pytest.mark.parametrize("name,chunk", [("qwen05", 1), ("qwen05", 4), ("smollm2", 5)])
 @pytest.mark.parametrize("fused", [True, False])
 def test_decode_gemv_fusion_matches_oracle(monkeypatch, name, chunk, fused):
-    # Up to eight positions the Q8_0 layers run the fused decode GEMVs
+    # Up to five positions the Q8_0 layers run the fused decode GEMVs
     # (rmsnorm / quantisation in the GEMV prologue, q/k/v in one launch,
     # gate/up finishing as swiglu); both that and the separate launches must
     # give the reference bits.

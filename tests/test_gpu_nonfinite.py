@@ -101,6 +101,9 @@ def test_load_rejects_non_finite_weights(case):
 FORWARD_CASES = {
     # the output projection's dot overflows (F32 GEMV result check)
     "f32 logits overflow": (W["tiny"], None, _edit("output.weight", _f32_fill(3e38))),
+    # the same inside a layer (one position by GEMV, chunks on the matrix cores)
+    "f32 q overflow": (W["tiny"], None, _edit("blk.0.attn_q.weight", _f32_fill(3e38))),
+    "f32 gate overflow": (W["tiny"], None, _edit("blk.1.ffn_gate.weight", _f32_fill(3e38))),
     # normed activations of 1e37 overflow the q/k/v block terms (Q8_0)
     "q8_0 gemv overflow": (W["smollm2"], 1, _edit("blk.0.attn_norm.weight", _f32_scale(1e37))),
     # rmsnorm's own output overflows (Q4_K layers: attention and FFN norms)
@@ -142,6 +145,55 @@ def test_forward_overflow_returns_non_finite(case):
     with Session(m, n, n) as s:
         syms = [int(t) for t in toks[1:n + 1]]
         assert _status(lambda: s.forward_ranges(toks[:n], 0, list(range(n)), syms, 256)) == NON_FINITE
+
+
+@pytest.mark.parametrize("hd,heads,graph", [
+    (16, 2, True), (16, 2, False), (48, 2, False),  # 48: the general kernels
+    (64, 2, True), (64, 2, False), (64, 9, False), (64, 18, False),  # groups of up to 8, 16 and more heads
+    (80, 2, True), (128, 2, True), (128, 2, False),
+])
+def test_overflowing_score_is_reported(monkeypatch, hd, heads, graph):
+    """q and k are large biases along one rotated pair, q = -k, so the score of
+    a key `n` positions back is -a^2 cos(0.3 n): for a^2 above the largest f32
+    a position's own score is -inf and the others are finite.  Softmax and P.V
+    then give finite values (the exp of -inf is that of the clamp), so only the
+    score's own check can report it.  At position 0 no score is formed."""
+    import dataclasses
+
+    from detllm_amd.model import F32Llama, Session
+
+    if not graph:
+        monkeypatch.setenv("DETLLM_NO_GRAPH", "1")
+    d = heads * hd
+    w = dataclasses.replace(W["qwen05"], d=d, heads=heads, kv_heads=1, ff=64, vocab=300, ctx=9,
+                            rope_base=float(np.float32(0.3 ** (-hd / 2))))
+
+    def model(a):
+        def e(t):
+            if t.name.endswith(("attn_q.bias", "attn_k.bias")):
+                b = np.zeros(len(t.data) // 4, np.float32)
+                b[1::hd] = -a if "attn_q" in t.name else a
+                t.data = b.tobytes()
+        return synth.build_model(w, 1, e)
+
+    toks = [int(t) for t in synth.tokens(w, 9)]
+    big, ok = model(np.sqrt(3.44e38)), model(np.sqrt(3.3e38))
+    assert _oracle_status(lambda: detref.Model(big).logits(toks[:1])) == 0
+    assert _oracle_status(lambda: detref.Model(big).logits(toks[:2])) == NON_FINITE
+    ref = detref.Model(ok).logits(toks)
+    assert np.isfinite(ref).all()
+    with Session(F32Llama.from_gguf(big), 9, 9) as s:
+        assert _status(lambda: s.forward_chunk(toks, 0)) == NON_FINITE
+        assert _status(lambda: s.forward_one(toks[0], 0)) == 0
+        assert _status(lambda: s.forward_one(toks[1], 1)) == NON_FINITE
+        assert _status(lambda: s.forward_chunk(toks[:3], 0)) == NON_FINITE
+    with Session(F32Llama.from_gguf(ok), 9, 9) as s:
+        for steps in ((9,), (1, 1, 1, 3, 1), (4, 5)):
+            p = 0
+            for n in steps:
+                got = s.forward_chunk(toks[p:p + n], p, want_logits=True)
+                assert np.array_equal(got.view(np.uint32), ref[p:p + n].view(np.uint32)), (steps, p)
+                p += n
 
 
 def test_healthy_model_after_failures_is_unaffected():
