@@ -5,6 +5,7 @@
 #include <sched.h>
 
 #include <atomic>
+#include <chrono>
 #include <cmath>
 #include <cstdlib>
 #include <cstdio>
@@ -755,12 +756,7 @@ struct dtl_session {
   Arena arena;
   float *rope_cos = nullptr, *rope_sin = nullptr, *kc = nullptr, *vc = nullptr;
   // Streams of the lanes (lane i's, and wide lane i's: the two kinds never run
-  // at once), created together with the session.  A stream takes the hardware
-  // queue that is least used when it is created.  Created by the first call that
-  // needed them, both streams of the second of three sessions were on one queue
-  // (kernel trace, four queues) and its chunks ran one after the other: encode of
-  // 1000 tokens with the Qwen2.5-0.5B shape by three sessions in turn 8.9 to 10.6
-  // ms a call, against 8.1 with one session or with streams created together.
+  // at once), the first with the session, the others by queue_stream.
   hipStream_t streams[kMaxLanes] = {};
   Lane lanes[kMaxLanes];
   int nlanes = 1;        // lanes the pipelined encode may use; lane 0 is set up
@@ -878,13 +874,77 @@ size_t max_input_width(const dtl_model* m) {
   return w;
 }
 
+// About 10 us on one wave (three sleeps of 127 x 64 cycles).
+__global__ void k_queue_probe() {
+  for (int i = 0; i < 3; i++) __builtin_amdgcn_s_sleep(127);
+}
+
+// us of six kernels on stream `a`; with `b`, of six more there that each wait for
+// one of them, as a lane waits for the one before it.  The session is idle; the
+// events are lane 0's.
+float probe_us(dtl_session* s, hipStream_t a, hipStream_t b) {
+  const std::vector<hipEvent_t>& ev = s->lanes[0].kv_ready;
+  const auto t = std::chrono::steady_clock::now();
+  for (size_t i = 0; i < 6; i++) {
+    launch_kernel(k_queue_probe, dim3(1), dim3(64), 0, a);
+    if (!b) continue;
+    (void)hipEventRecord(ev[i % ev.size()], a);
+    (void)hipStreamWaitEvent(b, ev[i % ev.size()], 0);
+    launch_kernel(k_queue_probe, dim3(1), dim3(64), 0, b);
+  }
+  (void)hipStreamSynchronize(a);
+  if (b) (void)hipStreamSynchronize(b);
+  return std::chrono::duration<float, std::micro>(std::chrono::steady_clock::now() - t).count();
+}
+
+// Stream li, tried against those of the lanes before it.  A new stream joins the
+// hardware queue that has the fewest, so which one it gets depends on every
+// stream that the process has created and destroyed.  It can be the queue of the
+// session's other lane (the two streams that follow the last free queue always
+// share one): the lanes then run one after the other.  Or, of more than four
+// queues, one on the same pipe (the fourth after it): a queue that waits for an
+// event then holds up the other's kernels, and two lanes take longer than one.
+// 1000 tokens, 24 layers of the Qwen2.5-0.5B shape: 9.0 ms side by side, 12.7 on
+// one lane, 12.3 on one queue, 18 on one pipe.  So up to eight streams are tried
+// and the one that runs best beside the others is kept, once in a session's life:
+// 0.35 ms for the first try, 0.1 for each further one.
+int queue_stream(dtl_session* s, int li) {
+  constexpr int kTries = 8;
+  // of the time alone: 1.5 to 1.9 side by side, 2.6 to 2.8 on one queue, 3.5 to
+  // 3.9 on one pipe (40 streams each at four and at eight queues)
+  constexpr float kBeside = 2.2f;
+  hipStream_t tried[kTries] = {};
+  int n = 0, best = -1;
+  float alone = 0.0f, best_us = 0.0f;
+  while (n < kTries && hipStreamCreateWithFlags(&tried[n], hipStreamNonBlocking) == hipSuccess) {
+    if (n == 0) {
+      (void)probe_us(s, s->streams[0], tried[0]);  // the first launches
+      alone = std::min(probe_us(s, s->streams[0], nullptr), probe_us(s, s->streams[0], nullptr));
+    }
+    float us = 0.0f;
+    for (int j = 0; j < li; j++) us = std::max(us, probe_us(s, s->streams[j], tried[n]));
+    if (best < 0 || us < best_us) {
+      best = n;
+      best_us = us;
+    }
+    n++;
+    if (us < kBeside * alone) break;
+  }
+  for (int i = 0; i < n; i++)
+    if (i != best) (void)hipStreamDestroy(tried[i]);
+  if (best < 0) return DTL_ERR_DEVICE;
+  s->streams[li] = tried[best];
+  return DTL_OK;
+}
+
 // Sets up those of lanes 0 .. n - 1 that a call needs and that are not there,
 // each with buffers of its own for `rows` positions; how many of them there are
 // (fewer when memory is short, or when the next would pass DETLLM_LANE_MEMORY).
 int ensure_lanes(dtl_session* s, Lane* lanes, Arena* arenas, int n, size_t rows) {
   for (int li = 0; li < n; li++) {
     if (lanes[li].stream) continue;
-    if (lane_init(s, arenas[li], lanes[li], s->streams[li], rows, s->lane_budget) != DTL_OK) {
+    if ((!s->streams[li] && queue_stream(s, li) != DTL_OK) ||
+        lane_init(s, arenas[li], lanes[li], s->streams[li], rows, s->lane_budget) != DTL_OK) {
       (void)hipGetLastError();
       lanes[li].release();
       arenas[li].release();
@@ -1640,7 +1700,7 @@ int dtl_session_new(const dtl_model* m, size_t n_ctx, size_t max_chunk, dtl_sess
   const size_t chunk = std::max(C, s->wide_rows);
   s->nlanes = (int)std::min((size_t)lane_count(), (n_ctx + chunk - 1) / chunk);
   if (s->wide_rows > C) s->nlanes = std::min(s->nlanes, kWideLanes);
-  for (int li = 0; li < s->nlanes; li++) HIP_TRY(hipStreamCreateWithFlags(&s->streams[li], hipStreamNonBlocking));
+  HIP_TRY(hipStreamCreateWithFlags(&s->streams[0], hipStreamNonBlocking));
   if (const char* e = getenv("DETLLM_LANE_MEMORY")) s->lane_budget = (size_t)strtoull(e, nullptr, 10);
   if ((st = lane_init(s.get(), s->lane_arena[0], s->lanes[0], s->streams[0], C, SIZE_MAX))) return st;  // the others: ensure_lanes
   HIP_TRY(hipHostMalloc((void**)&s->pos_host, sizeof(int), hipHostMallocDefault));
