@@ -48,12 +48,16 @@ FP32_VECTOR_PEAK_TFLOPS = 157.3        # FMA counted as two flops
 # registers, eight waves per SIMD).
 FP32_UNFUSED_PEAK_TFLOPS = 78.6
 
+# Positions of the chunks that dtl_forward_ranges forms for a session of a
+# smaller max_chunk.
+ENCODE_ROWS = 256
+
 # Kernel classes that form their products on the matrix cores (k_q4k_mfp) in
 # the chunk-at-a-time step the roofline is timed on: f32 16x16x1 MFMA outer
 # products, then one VALU add per multiply-add.  A SIMD runs the two one
 # after the other, so their bound is the pattern's own rate, which
 # dtl_mfp_probe measures live.
-MFMA_PRODUCT_CLASSES = {"gemm_q4_k_gate_up"}
+MFMA_PRODUCT_CLASSES = {"gemm_q4_k_gate_up", "gemm_q4_k", "gemm_q4_k_qk"}
 
 
 # HBM bytes per launch of the encode's Q4_K kernel classes (any of them can
@@ -63,12 +67,12 @@ MFMA_PRODUCT_CLASSES = {"gemm_q4_k_gate_up"}
 # counter onto the known bytes of a plain copy (--copy-probe-mib).  The
 # summary with the commands is the `source` file.
 MEASURED_TRAFFIC = {
-    "gemm_q4_k_gate_up": {"bytes": (63899.2 * 2.000 + 1408.1 * 1.000) * 1024.0,
-                          "source": "profiles/k_q4k_mfp_tinyllama_encode_chunk64.md"},
-    "gemm_q4_k": {"bytes": (16778.5 * 2.000 + 512.0 * 1.000) * 1024.0,
-                  "source": "profiles/k_q4k_f32m_tinyllama_encode_chunk64.md"},
-    "gemm_q4_k_qk": {"bytes": (11291.5 * 2.000 + 576.0 * 1.000) * 1024.0,
-                     "source": "profiles/k_q4k_f32m_tinyllama_encode_chunk64.md"},
+    "gemm_q4_k_gate_up": {"bytes": (339903.6 * 2.000 + 5632.8 * 1.000) * 1024.0,
+                          "source": "profiles/k_q4k_mfp_tinyllama_encode_chunk256.md"},
+    "gemm_q4_k": {"bytes": (27003.3 * 2.000 + 2048.0 * 1.000) * 1024.0,
+                  "source": "profiles/k_q4k_mfp_tinyllama_encode_chunk256.md"},
+    "gemm_q4_k_qk": {"bytes": (17451.4 * 2.000 + 2304.0 * 1.000) * 1024.0,
+                     "source": "profiles/k_q4k_mfp_tinyllama_encode_chunk256.md"},
 }
 
 
@@ -375,10 +379,11 @@ def golden(name: str):
 
 
 def encode_leg(name: str, chunk: int, steps: int) -> dict:
-    """Chunked encode of a workload's whole token stream (dtl_forward_ranges,
-    chunks of `chunk` in flight) with the next token's symbol range (256
-    byte escapes): tokens/s, the ranges against the committed golden, and the
-    per-class kernel times of one chunk-at-a-time pass."""
+    """Chunked encode of a workload's whole token stream (dtl_forward_ranges
+    of a session of `chunk`-position chunks: two of ENCODE_ROWS in flight) with
+    the next token's symbol range (256 byte escapes): tokens/s, the ranges
+    against the committed golden, and the per-class kernel times of one pass of
+    such chunks, one at a time."""
     import hashlib
     import struct
 
@@ -400,9 +405,11 @@ def encode_leg(name: str, chunk: int, steps: int) -> dict:
             got = s.forward_ranges(toks, 0, rows, nxt, 256)
         dt = (time.perf_counter() - t) / steps
         same = all(np.array_equal(a, b) for a, b in zip(first, got))
+    rows_at_once = max(chunk, ENCODE_ROWS)
+    with m.forward_workspace(w.ctx, rows_at_once) as s:
         s.set_profiling(True)
-        for p in range(0, n, chunk):
-            s.forward_chunk(toks[p:p + chunk], p)
+        for p in range(0, n, rows_at_once):
+            s.forward_chunk(toks[p:p + rows_at_once], p)
         prof = s.profile()
         s.set_profiling(False)
     h = hashlib.sha256()
@@ -484,6 +491,8 @@ def main() -> int:
     log(f"[bench] loaded to device ({model.device_bytes / 1e6:.1f} MB) in {time.time() - t:.1f}s")
     n, chunk = toks.size, w.chunk
     sess = model.forward_workspace(n, chunk)
+    # the chunks that the encode forms, for kernel timing
+    psess = None if args.no_kernel_timing else model.forward_workspace(n, max(chunk, ENCODE_ROWS))
     tail = 256
 
     rows = np.arange(n - 1, dtype=np.uint32)
@@ -491,19 +500,21 @@ def main() -> int:
 
     def step():
         """One teacher-forced encode: every position's forward and the range of
-        the next token, three chunks in flight (dtl_forward_ranges)."""
+        the next token, two chunks of ENCODE_ROWS in flight
+        (dtl_forward_ranges)."""
         return sess.forward_ranges(toks, 0, rows, syms, tail)
 
     def step_chunked():
-        """The same work one chunk at a time (dtl_forward_chunk +
+        """The same chunks one at a time (dtl_forward_chunk +
         dtl_symbol_ranges): launches never overlap, so per-launch events time
         each kernel alone."""
         out = [[], [], []]
-        for p in range(0, n, chunk):
-            sess.forward_chunk(toks[p:p + chunk], p)
-            m = min(chunk, n - 1 - p)
+        for p in range(0, n, psess.max_chunk):
+            T = min(psess.max_chunk, n - p)
+            psess.forward_chunk(toks[p:p + T], p)
+            m = min(T, n - 1 - p)
             if m > 0:
-                for dst, src in zip(out, sess.symbol_ranges(toks[p + 1:p + 1 + m], 0, tail)):
+                for dst, src in zip(out, psess.symbol_ranges(toks[p + 1:p + 1 + m], 0, tail)):
                     dst.append(src)
         return tuple(np.concatenate(x) for x in out)
 
@@ -520,15 +531,15 @@ def main() -> int:
     prof = {}
     chunked = None
     if not args.no_kernel_timing:
-        sess.set_profiling(True)
+        psess.set_profiling(True)
         chunked = step_chunked()
-        breakdown = sess.profile()
+        breakdown = psess.profile()
         dom_name = max(breakdown.items(), key=lambda kv: kv[1]["total_ms"])[0]
-        sess.set_profiling(True)
-        sess.profile_only(dom_name)
+        psess.set_profiling(True)
+        psess.profile_only(dom_name)
         step_chunked()
-        prof = sess.profile()
-        sess.set_profiling(False)
+        prof = psess.profile()
+        psess.set_profiling(False)
         log(f"[bench] profiled chunk-at-a-time steps: dominant kernel class {dom_name}")
     results = []
     t0 = time.perf_counter()
@@ -578,8 +589,8 @@ def main() -> int:
         achieved = per_launch_bytes / (avg_ms * 1e-3) / 1e9
         roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                     "frac": round(achieved / HBM_PEAK_GBS, 4)}
-    roofline["timed_over"] = ("one chunk-at-a-time step timing the dominant class alone (launches not "
-                              "overlapped); the timed steps run two chunks of 256 positions in flight")
+    roofline["timed_over"] = (f"one step of {psess.max_chunk}-position chunks, one at a time, timing the dominant "
+                              "class alone (launches not overlapped); the timed steps run two such chunks in flight")
     roofline.update({"kernel": dom_name, "avg_launch_us": round(avg_ms * 1e3, 2), "launches": dom["launches"],
                      "algorithmic_bytes_per_launch": per_launch_bytes,
                      "algorithmic_flops_per_launch": per_launch_flops})
