@@ -656,22 +656,24 @@ const char* lm_head_class(int type) {
 }  // namespace
 
 // The buffers of one chunk in flight: activations, logits, the CDF staging,
-// the error flag and the stream its launches go to.  A session has 3 or 4 of
-// them, so the pipelined encode (dtl_forward_ranges) runs the next chunks
-// beside chunk c; every other entry point works on lane 0.
-// Measured on MI355X for the 64-position encode: with HIP's default of four
-// hardware queues per process three lanes (14.6k tokens/s; four lanes make
-// two streams share a queue: 13.0k); with GPU_MAX_HW_QUEUES=8 four lanes
-// (15.2k; five: 14.1k).  A session takes four lanes when the process has at
-// least five queues, else three; DETLLM_LANES (1-4) overrides.
+// the error flag and the stream its launches go to.  The pipelined encode
+// (dtl_forward_ranges) runs the next chunks beside chunk c on further lanes;
+// every other entry point works on lane 0.  A session takes up to four lanes
+// when the process has at least five hardware queues, else three (the null
+// stream has one of HIP's four): with their streams on whichever queue they got,
+// four lanes of 64 positions took 122 ms per 2048-token window of the
+// TinyLlama-1.1B shape at four queues, three 103, and at eight queues 94 and 102.
+// Since queue_stream they take 94.7 and 103.5 at either.  DETLLM_LANES (1-4)
+// overrides.
 constexpr int kMaxLanes = 4;
 
 // The pipelined encode takes at least this many positions per chunk, whatever
 // the session's max_chunk, on two lanes of its own: fewer, larger launches
 // fill the chip better than more, smaller ones side by side.  ms per window,
-// four lanes of 64 positions / two of 256 / four of 256 / two of 512: 2048
-// tokens of the TinyLlama-1.1B shape 127 / 88 / 90 / 86, 1000 tokens of the
-// Qwen2.5-0.5B shape (before the int8 GEMM's LDS tiles) 42 / 16 / 16 / 14.
+// three and four lanes of 64 positions / one, two and four of 256 / two of 512:
+// 2048 tokens of the TinyLlama-1.1B shape 103.5, 94.7 / 95.9, 87.0, 82.7 / 83.9;
+// 1000 tokens of the Qwen2.5-0.5B shape 17.6, 17.6 / 12.8, 9.1, 8.4 / 8.2.  Two
+// of 256 rather than four or two of 512, for their memory.
 constexpr size_t kEncodeRows = 256;
 constexpr int kWideLanes = 2;
 
@@ -1701,7 +1703,8 @@ int dtl_session_new(const dtl_model* m, size_t n_ctx, size_t max_chunk, dtl_sess
   s->nlanes = (int)std::min((size_t)lane_count(), (n_ctx + chunk - 1) / chunk);
   if (s->wide_rows > C) s->nlanes = std::min(s->nlanes, kWideLanes);
   HIP_TRY(hipStreamCreateWithFlags(&s->streams[0], hipStreamNonBlocking));
-  if (const char* e = getenv("DETLLM_LANE_MEMORY")) s->lane_budget = (size_t)strtoull(e, nullptr, 10);
+  const char* room = getenv("DETLLM_LANE_MEMORY");
+  if (room && *room) s->lane_budget = (size_t)strtoull(room, nullptr, 10);
   if ((st = lane_init(s.get(), s->lane_arena[0], s->lanes[0], s->streams[0], C, SIZE_MAX))) return st;  // the others: ensure_lanes
   HIP_TRY(hipHostMalloc((void**)&s->pos_host, sizeof(int), hipHostMallocDefault));
   HIP_TRY(hipMemsetAsync(s->kc, 0, kv * 4, s->ln->stream));

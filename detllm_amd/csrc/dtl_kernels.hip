@@ -1400,8 +1400,8 @@ __global__ void __launch_bounds__(kPvThreads) k_attn_split_pv(const float* score
 
 // softmax_in_place (lib.rs:2361-2388) of the score row, then
 // out[d] = 0; out[d] += p_j * v_j[d] (j ascending, lib.rs:2390-2420) for
-// dimensions [16 blockIdx.x, +16), rows of any length and heads of any
-// width.  The score row stays in LDS (as probabilities); V passes through it
+// dimensions [16 blockIdx.x, +16), rows as long as LDS holds (about 32100
+// keys) and the head widths of tiles_width.  The score row stays in LDS (as probabilities); V passes through it
 // dimension-major in tiles of 256 keys, double-buffered, with four tiles of
 // loads in flight per thread (one tile's sums take about 1400 cycles, less
 // than a memory round trip).  The chain-major exps of the Z chains share LDS
@@ -1411,9 +1411,11 @@ __global__ void __launch_bounds__(kPvThreads) k_attn_split_pv(const float* score
 // / chain_group_dot_lds: one chain per 16-lane row, each product formed just
 // before its add).
 //
-// Bound by the serial P.V sums (about 5.5 cycles per key).  Scores and P.V
-// together, 128-wide heads, 8 query / 2 key heads: 10.5 us at 500 keys, 12.4
-// at 1000, 20.3 at 2903, 24.0 at 4000, against 165, 347, 1003 and 1377 us of
+// Scores and P.V together, 128-wide heads, 8 query / 2 key heads: 10.5 us at 500
+// keys, 12.4 at 1000, 20.3 at 2903, 24.0 at 4000: about 8.6 us and 9 cycles per
+// key, of which the ordered P.V adds are 5 to 5.5; what takes the rest (the
+// row's exps and divisions in one workgroup, a barrier and the chains' restart
+// every 256 keys) is not measured.  Against 165, 347, 1003 and 1377 us of
 // the one-workgroup-per-group kernel that served this width before.  64-wide
 // heads up to 2048 keys keep k_attn_split_pv, whose whole row of V is loaded
 // ahead of the softmax (token of the Qwen2.5-0.5B shape at 1501 keys 1145 us
