@@ -760,6 +760,7 @@ struct dtl_session {
   // Streams of the lanes (lane i's, and wide lane i's: the two kinds never run
   // at once), the first with the session, the others by queue_stream.
   hipStream_t streams[kMaxLanes] = {};
+  float probe_alone_us = 0.0f;  // queue_stream's measure
   Lane lanes[kMaxLanes];
   int nlanes = 1;        // lanes the pipelined encode may use; lane 0 is set up
                          // with the session, the others by the first call that
@@ -876,18 +877,19 @@ size_t max_input_width(const dtl_model* m) {
   return w;
 }
 
-// About 10 us on one wave (three sleeps of 127 x 64 cycles).
+// About 20 us on one wave (six sleeps of 127 x 64 cycles): long enough that the
+// host enqueues faster.
 __global__ void k_queue_probe() {
-  for (int i = 0; i < 3; i++) __builtin_amdgcn_s_sleep(127);
+  for (int i = 0; i < 6; i++) __builtin_amdgcn_s_sleep(127);
 }
 
-// us of six kernels on stream `a`; with `b`, of six more there that each wait for
+// us of four kernels on stream `a`; with `b`, of four more there that each wait for
 // one of them, as a lane waits for the one before it.  The session is idle; the
 // events are lane 0's.
 float probe_us(dtl_session* s, hipStream_t a, hipStream_t b) {
   const std::vector<hipEvent_t>& ev = s->lanes[0].kv_ready;
   const auto t = std::chrono::steady_clock::now();
-  for (size_t i = 0; i < 6; i++) {
+  for (size_t i = 0; i < 4; i++) {
     launch_kernel(k_queue_probe, dim3(1), dim3(64), 0, a);
     if (!b) continue;
     (void)hipEventRecord(ev[i % ev.size()], a);
@@ -908,29 +910,35 @@ float probe_us(dtl_session* s, hipStream_t a, hipStream_t b) {
 // event then holds up the other's kernels, and two lanes take longer than one.
 // 1000 tokens, 24 layers of the Qwen2.5-0.5B shape: 9.0 ms side by side, 12.7 on
 // one lane, 12.3 on one queue, 18 on one pipe.  So up to eight streams are tried
-// and the one that runs best beside the others is kept, once in a session's life:
-// 0.35 ms for the first try, 0.1 for each further one.
+// and the one that runs best beside the others is kept, once in a session's life
+// and mostly the first: 0.3 ms for the time alone and 0.14 for each earlier lane
+// (a session's first call with two lanes is 0.5 ms longer for it, with four 1.4).
 int queue_stream(dtl_session* s, int li) {
   constexpr int kTries = 8;
-  // of the time alone: 1.5 to 1.9 side by side, 2.6 to 2.8 on one queue, 3.5 to
-  // 3.9 on one pipe (40 streams each at four and at eight queues)
-  constexpr float kBeside = 2.2f;
+  // of the time alone: 1.4 to 1.6 side by side, 2.3 to 2.4 on one queue, 2.7 to 3
+  // on one pipe (160 streams, mostly at eight queues)
+  constexpr float kBeside = 1.9f;
   hipStream_t tried[kTries] = {};
   int n = 0, best = -1;
-  float alone = 0.0f, best_us = 0.0f;
+  float best_us = 0.0f;
+  if (s->probe_alone_us == 0.0f) {
+    (void)probe_us(s, s->streams[0], nullptr);  // the first launches
+    s->probe_alone_us = std::min(probe_us(s, s->streams[0], nullptr), probe_us(s, s->streams[0], nullptr));
+  }
+  const float limit = kBeside * s->probe_alone_us;
   while (n < kTries && hipStreamCreateWithFlags(&tried[n], hipStreamNonBlocking) == hipSuccess) {
-    if (n == 0) {
-      (void)probe_us(s, s->streams[0], tried[0]);  // the first launches
-      alone = std::min(probe_us(s, s->streams[0], nullptr), probe_us(s, s->streams[0], nullptr));
-    }
     float us = 0.0f;
-    for (int j = 0; j < li; j++) us = std::max(us, probe_us(s, s->streams[j], tried[n]));
+    for (int j = li - 1; j >= 0 && us < limit; j--) {
+      float t = probe_us(s, s->streams[j], tried[n]);
+      if (t >= limit) t = std::min(t, probe_us(s, s->streams[j], tried[n]));  // a queue's first use takes longer
+      us = std::max(us, t);
+    }
     if (best < 0 || us < best_us) {
       best = n;
       best_us = us;
     }
     n++;
-    if (us < kBeside * alone) break;
+    if (us < limit) break;
   }
   for (int i = 0; i < n; i++)
     if (i != best) (void)hipStreamDestroy(tried[i]);
